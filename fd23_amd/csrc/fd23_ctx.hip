@@ -212,6 +212,10 @@ struct fd23_ctx {
     };
     std::map<std::tuple<int, int, int>, Chunk> graphs;
 
+    // packed device rows on their way to or from the host (pitched copies)
+    void *stage = nullptr;
+    size_t stage_cap = 0;
+
     // box coupling state (see fd23_box.hip)
     void *box = nullptr;
 };
@@ -308,7 +312,7 @@ static void free_ctx(fd23_ctx *c) {
                       c->d_taps, c->d_src, c->d_stf, c->d_roff, c->d_nrec, c->seis, c->d_tap_start,
                       c->d_rec_start, c->d_tapsT, c->d_recs, c->d_ftap_start, c->d_frec_start, c->d_ftaps,
                       c->d_frecs, c->d_pfirst, c->d_plast, c->d_pwin, c->d_btap_start, c->d_brec_start,
-                      c->d_btaps, c->d_brecs};
+                      c->d_btaps, c->d_brecs, c->stage};
     for (auto p : others) if (p) hipFree(p);
     if (c->own_stream && c->stream) hipStreamDestroy(c->stream);
     for (int i = 0; i < 3; i++) {
@@ -443,16 +447,83 @@ extern "C" int fd23_ctx_destroy(fd23_ctx *c) {
 }
 
 // ---------------------------------------------------------------------------
+// pitched transfers
+// ---------------------------------------------------------------------------
+// Rows between a pitched device array and host memory.  The runtime copies a
+// pitched region row by row (about 8 us each: 58 ms for the seismograms of 64
+// shots x 64 frames, 8.8 ms for a 301 x 223 checkpoint), so the rows are
+// packed on the device (k_pack_rows / k_unpack_rows, which also convert
+// scaled storage to the compute type) into a buffer of the context and cross
+// the host link as one contiguous copy per kStageBytes: 8.1 ms and 0.4 ms.
+// kStageBytes is where a copy's fixed cost (a launch and a wait, 30-40 us) is
+// a tenth of its 250 us on the link.
+static const size_t kStageBytes = (size_t)4 << 20;
+
+template <class S> static int rows_xfer_t(fd23_ctx *c, void *dev, long pitch, long w, long h, void *host, float scale,
+                                          bool to_host) {
+    using C = typename Store<S>::C;
+    const size_t row = (size_t)w * sizeof(C);
+    const long per = std::max<long>(1, (long)std::min<size_t>(kStageBytes / row, (size_t)h)); // rows of one copy
+    if ((size_t)per * row > c->stage_cap) {
+        if (c->stage) HIPCHK(hipFree(c->stage));
+        c->stage = nullptr;
+        c->stage_cap = 0;
+        HIPCHK(hipMalloc(&c->stage, (size_t)per * row));
+        c->stage_cap = (size_t)per * row;
+    }
+    const dim3 block(256);
+    for (long r = 0; r < h; r += per) {
+        const long n = std::min(per, h - r);
+        const dim3 grid((unsigned)std::min<long>((w + 255) / 256, 1024), (unsigned)std::min<long>(n, 4096));
+        S *d = (S *)dev + r * pitch;
+        char *p = (char *)host + (size_t)r * row;
+        if (to_host) {
+            hipLaunchKernelGGL((k_pack_rows<S>), grid, block, 0, c->stream, (C *)c->stage, d, pitch, w, n, scale);
+            HIPCHK(hipGetLastError());
+            HIPCHK(hipMemcpyAsync(p, c->stage, (size_t)n * row, hipMemcpyDeviceToHost, c->stream));
+        } else {
+            HIPCHK(hipMemcpyAsync(c->stage, p, (size_t)n * row, hipMemcpyHostToDevice, c->stream));
+            hipLaunchKernelGGL((k_unpack_rows<S>), grid, block, 0, c->stream, d, (const C *)c->stage, pitch, w, n,
+                               scale);
+            HIPCHK(hipGetLastError());
+        }
+    }
+    HIPCHK(hipStreamSynchronize(c->stream));
+    return FD23_OK;
+}
+
+// w x h values between host memory (compute type, packed) and a device array
+// of the given pitch in elements: fields and psi (storage type, one scale),
+// or material and seismograms (compute type)
+static int rows_xfer(fd23_ctx *c, void *dev, long pitch, long w, long h, void *host, float scale, bool to_host,
+                     bool stored) {
+    if (w <= 0 || h <= 0) return FD23_OK;
+    if (stored && c->d.storage == FD23_STORE_F16)
+        return rows_xfer_t<__half>(c, dev, pitch, w, h, host, scale, to_host);
+    if (stored && c->d.storage == FD23_STORE_BF16)
+        return rows_xfer_t<__hip_bfloat16>(c, dev, pitch, w, h, host, scale, to_host);
+    // plain values that are contiguous, or a single row, need no packing
+    if (pitch == w || h == 1) {
+        const size_t n = (size_t)w * h * c->csize;
+        HIPCHK(to_host ? hipMemcpyAsync(host, dev, n, hipMemcpyDeviceToHost, c->stream)
+                       : hipMemcpyAsync(dev, host, n, hipMemcpyHostToDevice, c->stream));
+        HIPCHK(hipStreamSynchronize(c->stream));
+        return FD23_OK;
+    }
+    return c->csize == 8 ? rows_xfer_t<double>(c, dev, pitch, w, h, host, scale, to_host)
+                         : rows_xfer_t<float>(c, dev, pitch, w, h, host, scale, to_host);
+}
+
+// ---------------------------------------------------------------------------
 // material, C-PML, scales
 // ---------------------------------------------------------------------------
 extern "C" int fd23_set_material(fd23_ctx *c, const void *const *arrays) {
     if (!c || !arrays) return fail(FD23_EINVAL, "null argument");
     for (int m = 0; m < c->nmat; m++) {
         if (!arrays[m]) return fail(FD23_EINVAL, "material array %d is null", m);
-        HIPCHK(hipMemcpy2DAsync(c->mat[m], (size_t)c->px * c->csize, arrays[m], (size_t)c->d.nx * c->csize,
-                                (size_t)c->d.nx * c->csize, c->d.nz, hipMemcpyHostToDevice, c->stream));
+        int r = rows_xfer(c, c->mat[m], c->px, c->d.nx, c->d.nz, (void *)arrays[m], 1.0f, false, false);
+        if (r) return r;
     }
-    HIPCHK(hipStreamSynchronize(c->stream));
     // largest BU/BW (P-SV) or BV (SH): a velocity is about bmax times a stress
     const int nb = is_psv(c) ? 2 : 1;
     double bm = 0;
@@ -467,10 +538,7 @@ extern "C" int fd23_set_material(fd23_ctx *c, const void *const *arrays) {
 
 extern "C" int fd23_get_material(fd23_ctx *c, int index, void *out) {
     if (!c || !out || index < 0 || index >= c->nmat) return fail(FD23_EINVAL, "bad arguments");
-    HIPCHK(hipMemcpy2DAsync(out, (size_t)c->d.nx * c->csize, c->mat[index], (size_t)c->px * c->csize,
-                            (size_t)c->d.nx * c->csize, c->d.nz, hipMemcpyDeviceToHost, c->stream));
-    HIPCHK(hipStreamSynchronize(c->stream));
-    return FD23_OK;
+    return rows_xfer(c, c->mat[index], c->px, c->d.nx, c->d.nz, out, 1.0f, true, false);
 }
 
 extern "C" int fd23_set_cpml(fd23_ctx *c, const double *packed) {
@@ -1808,13 +1876,10 @@ extern "C" int fd23_get_seismograms(fd23_ctx *c, int shot, int comp, float *out,
     if (nframes < 0 || nframes > c->d.max_frames) return fail(FD23_EINVAL, "nframes %d > capacity", nframes);
     const int n = c->h_nrec[(size_t)shot * c->ncomp + comp];
     if (nframes == 0 || n == 0) return FD23_OK;
-    HIPCHK(hipStreamSynchronize(c->stream));
     const long frame_stride = (long)c->d.nshots * c->ncomp * c->d.max_rec;
     const long off = ((long)shot * c->ncomp + comp) * c->d.max_rec;
-    // copies rows of n values out of the frame-major buffer
-    HIPCHK(hipMemcpy2D(out, (size_t)n * c->csize, (char *)c->seis + (size_t)off * c->csize,
-                       (size_t)frame_stride * c->csize, (size_t)n * c->csize, nframes, hipMemcpyDeviceToHost));
-    return FD23_OK;
+    // rows of n values out of the frame-major buffer
+    return rows_xfer(c, (char *)c->seis + (size_t)off * c->csize, frame_stride, n, nframes, out, 1.0f, true, false);
 }
 
 static int internal_field(const fd23_ctx *c, int field) {
@@ -1825,61 +1890,6 @@ static int internal_field(const fd23_ctx *c, int field) {
     return field >= 0 && field < 3 ? field : -1;
 }
 
-static float host_half_to_float(uint16_t h, int storage) {
-    if (storage == FD23_STORE_BF16) {
-        uint32_t u = (uint32_t)h << 16;
-        float f;
-        memcpy(&f, &u, 4);
-        return f;
-    }
-    __half hv;
-    memcpy(&hv, &h, 2);
-    return __half2float(hv);
-}
-static uint16_t host_float_to_half(float v, int storage) {
-    if (storage == FD23_STORE_BF16) {
-        __hip_bfloat16 b = __float2bfloat16(v);
-        uint16_t u;
-        memcpy(&u, &b, 2);
-        return u;
-    }
-    __half hv = __float2half(v);
-    uint16_t u;
-    memcpy(&u, &hv, 2);
-    return u;
-}
-
-// copy one pitched array (n rows of w elements) between device and host,
-// converting scaled storage to the compute type
-static int xfer(fd23_ctx *c, void *dev, long pitch, int w, int h, void *host, float scale, bool to_host) {
-    const int es = c->esize, cs = c->csize;
-    std::vector<char> tmp((size_t)w * h * es);
-    if (to_host) {
-        HIPCHK(hipMemcpy2DAsync(tmp.data(), (size_t)w * es, dev, (size_t)pitch * es, (size_t)w * es, h,
-                                hipMemcpyDeviceToHost, c->stream));
-        HIPCHK(hipStreamSynchronize(c->stream));
-        if (es == cs) {
-            memcpy(host, tmp.data(), tmp.size());
-        } else {
-            const uint16_t *src = (const uint16_t *)tmp.data();
-            float *dst = (float *)host;
-            for (size_t i = 0; i < (size_t)w * h; i++) dst[i] = host_half_to_float(src[i], c->d.storage) * scale;
-        }
-    } else {
-        if (es == cs) {
-            memcpy(tmp.data(), host, tmp.size());
-        } else {
-            const float *src = (const float *)host;
-            uint16_t *dst = (uint16_t *)tmp.data();
-            for (size_t i = 0; i < (size_t)w * h; i++) dst[i] = host_float_to_half(src[i] / scale, c->d.storage);
-        }
-        HIPCHK(hipMemcpy2DAsync(dev, (size_t)pitch * es, tmp.data(), (size_t)w * es, (size_t)w * es, h,
-                                hipMemcpyHostToDevice, c->stream));
-        HIPCHK(hipStreamSynchronize(c->stream));
-    }
-    return FD23_OK;
-}
-
 static int field_xfer(fd23_ctx *c, int shot, int field, void *host, bool to_host) {
     const int fi = internal_field(c, field);
     if (fi < 0 || shot < 0 || shot >= c->d.nshots || !host) return fail(FD23_EINVAL, "bad field/shot");
@@ -1887,7 +1897,7 @@ static int field_xfer(fd23_ctx *c, int shot, int field, void *host, bool to_host
     HIPCHK(hipStreamSynchronize(c->stream));
     HIPCHK(hipMemcpy(sc, c->scl, sizeof sc, hipMemcpyDeviceToHost));
     void *dev = (char *)c->fields[fi] + (size_t)shot * c->sstride * c->esize;
-    return xfer(c, dev, c->px, c->d.nx, c->d.nz, host, sc[fi], to_host);
+    return rows_xfer(c, dev, c->px, c->d.nx, c->d.nz, host, sc[fi], to_host, true);
 }
 
 extern "C" int fd23_get_field(fd23_ctx *c, int shot, int field, void *out) {
@@ -1917,7 +1927,7 @@ static int state_xfer(fd23_ctx *c, int shot, void *buf, size_t bytes, bool to_ho
     for (int f = 0; f < c->nfield; f++) {
         const int fi = internal_field(c, f);
         void *dev = (char *)c->fields[fi] + (size_t)shot * c->sstride * c->esize;
-        int r = xfer(c, dev, c->px, c->d.nx, c->d.nz, p, sc[fi], to_host);
+        int r = rows_xfer(c, dev, c->px, c->d.nx, c->d.nz, p, sc[fi], to_host, true);
         if (r) return r;
         p += N * c->csize;
     }
@@ -1926,7 +1936,7 @@ static int state_xfer(fd23_ctx *c, int shot, void *buf, size_t bytes, bool to_ho
         const long n = q < half ? c->xpsi : c->zpsi;
         if (n == 0) continue;
         void *dev = (char *)c->psi[q] + (size_t)shot * n * c->esize;
-        int r = xfer(c, dev, n, (int)n, 1, p, sc[c->nfield + q], to_host);
+        int r = rows_xfer(c, dev, n, n, 1, p, sc[c->nfield + q], to_host, true);
         if (r) return r;
         p += (size_t)n * c->csize;
     }

@@ -1340,6 +1340,25 @@ __global__ void k_commit_scales(float *scl, unsigned mask) {
     if (f < kNextScale && ((mask >> f) & 1u)) scl[f] = scl[kNextScale + f];
 }
 
+// Rows of w values between a pitched array in its storage type and a packed
+// buffer in the compute type, for the host link: bound by that link (16 GB/s
+// into pageable memory), so one value per lane, rows strided over grid.y.
+template <class S>
+__global__ __launch_bounds__(256) void k_pack_rows(typename Store<S>::C *__restrict__ dst, const S *__restrict__ src,
+                                                   long pitch, long w, long h, float scale) {
+    for (long r = blockIdx.y; r < h; r += gridDim.y)
+        for (long i = blockIdx.x * 256L + threadIdx.x; i < w; i += gridDim.x * 256L)
+            dst[r * w + i] = Store<S>::ld(src, r * pitch + i, scale);
+}
+template <class S>
+__global__ __launch_bounds__(256) void k_unpack_rows(S *__restrict__ dst, const typename Store<S>::C *__restrict__ src,
+                                                     long pitch, long w, long h, float scale) {
+    const float inv = Store<S>::scaled ? inv_pow2(scale) : 1.f;
+    for (long r = blockIdx.y; r < h; r += gridDim.y)
+        for (long i = blockIdx.x * 256L + threadIdx.x; i < w; i += gridDim.x * 256L)
+            Store<S>::st(dst, r * pitch + i, src[r * w + i], inv);
+}
+
 // advance the step clock after a captured chunk of steps
 __global__ void k_tick(int *clock, int steps) {
     if (threadIdx.x == 0) clock[0] += steps;

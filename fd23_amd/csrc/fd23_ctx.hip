@@ -770,17 +770,29 @@ extern "C" int fd23_set_shot_slot(fd23_ctx *c, int shot, int active, int t0) {
 extern "C" int fd23_reset_shot(fd23_ctx *c, int shot) {
     if (!c || shot < 0 || shot >= c->d.nshots) return fail(FD23_EINVAL, "bad shot %d", shot);
     const size_t es = c->esize;
+    ZeroRegions z{};
+    int n = 0;
+    unsigned most = 1;
+    auto region = [&](char *p, long pitch, size_t bytes, size_t rows) {
+        if (!bytes || !rows) return;
+        z.r[n++] = ZeroRegions::R{p, pitch, (unsigned)(bytes / 4), (unsigned)rows};
+        most = std::max(most, (unsigned)rows);
+    };
     for (int set = 0; set < 2; set++) {
         void *const *f = set ? c->alt_fields : c->fields;
         void *const *q = set ? c->alt_psi : c->psi;
         if (set && !c->alt_alloc[0]) break; // no second buffer set yet
+        // whole pitches: the columns past nx are padding, always zero
+        const long row = (long)c->px * es;
         for (int i = 0; i < c->nfield; i++)
-            HIPCHK(hipMemset2DAsync((char *)f[i] + (size_t)shot * c->sstride * es, (size_t)c->px * es, 0,
-                                    (size_t)c->d.nx * es, c->d.nz, c->stream));
+            region((char *)f[i] + (size_t)shot * c->sstride * es, row, row, c->d.nz);
+        // a psi array is contiguous: nz rows of 2*npml values (x), npml rows
+        // of 2*nx values (z), an even count of 2 to 8 bytes each
         const int half = c->npsi / 2;
         for (int p = 0; p < c->npsi; p++) {
-            const size_t n = p < half ? c->xpsi : c->zpsi;
-            if (n) HIPCHK(hipMemsetAsync((char *)q[p] + (size_t)shot * n * es, 0, n * es, c->stream));
+            const size_t len = p < half ? c->xpsi : c->zpsi;
+            const size_t rows = p < half ? c->d.nz : c->d.npml;
+            if (len) region((char *)q[p] + (size_t)shot * len * es, (long)(len / rows * es), len / rows * es, rows);
         }
     }
     // the shot's seismogram entries of every frame (receivers off the grid
@@ -788,8 +800,11 @@ extern "C" int fd23_reset_shot(fd23_ctx *c, int shot) {
     if (c->seis && c->d.max_rec > 0) {
         const size_t frame = (size_t)c->d.nshots * c->ncomp * c->d.max_rec * c->csize;
         const size_t mine = (size_t)c->ncomp * c->d.max_rec * c->csize;
-        HIPCHK(hipMemset2DAsync((char *)c->seis + shot * mine, frame, 0, mine, c->d.max_frames, c->stream));
+        region((char *)c->seis + shot * mine, (long)frame, mine, c->d.max_frames);
     }
+    if (n == 0) return FD23_OK;
+    hipLaunchKernelGGL(k_zero_regions, dim3(std::min(most, 256u), n), dim3(256), 0, c->stream, z);
+    HIPCHK(hipGetLastError());
     return FD23_OK;
 }
 

@@ -82,3 +82,28 @@ def test_seismograms_are_the_recorded_velocities(nrec, max_rec, frames):
             for f in (0, frames // 2, frames - 1):
                 assert np.array_equal(got[f], want[s, f]), (s, f)
             assert np.count_nonzero(np.abs(got).sum(axis=1)) == len({0, frames // 2, frames - 1})
+
+
+@pytest.mark.parametrize("nx,nz,npml", [(16, 16, 0), (63, 17, 5), (300, 130, 12)])
+@pytest.mark.parametrize("storage", [_lib.STORE_F32, _lib.STORE_F64, _lib.STORE_F16])
+def test_reset_zeroes_one_shot_alone(nx, nz, npml, storage):
+    rng = np.random.default_rng(nx)
+    with Context(_lib.WAVE_PSV, nx, nz, npml, nshots=3, storage=storage, max_frames=4, max_rec=3) as ctx:
+        if storage == _lib.STORE_F16:
+            ctx.set_scales(np.ones(13, np.float32))
+        n = ctx.state_bytes() // np.dtype(ctx.cdtype).itemsize
+        data = [rng.integers(-9, 9, n).astype(ctx.cdtype).tobytes() for _ in range(3)]
+        for s in range(3):
+            ctx.set_state(data[s], s)
+            for c in range(2):
+                ctx.set_receivers(s, c, np.array([1, 2, 3], np.int32), np.array([4, 5, 6], np.int32))
+        for f in range(4):
+            ctx.record(f, 1)
+        seis = [[ctx.seismograms(s, c, 4) for c in range(2)] for s in range(3)]
+        ctx.reset_shot(1)
+        assert not np.frombuffer(ctx.get_state(1), np.uint8).any()
+        assert not any(ctx.seismograms(1, c, 4).any() for c in range(2))
+        for s in (0, 2):
+            assert ctx.get_state(s) == data[s]
+            for c in range(2):
+                assert np.array_equal(ctx.seismograms(s, c, 4), seis[s][c])

@@ -124,11 +124,13 @@ def run_gpu(wl, steps, warmup, autotune=True, tile=None, passes=True, chains=Non
     fused = kind == _lib.TILE_FUSED and wl.wave == _lib.WAVE_PSV and wl.punch_after is None
     # steps per launch of the SH block step, 0 when another path runs
     block = ctx.tile_shape()[2] if kind == _lib.TILE_BLOCK and wl.punch_after is None else 0
+    # steps per launch of the marching P-SV step (it is one of the fused shapes)
+    march = ctx.tile_shape()[2] if fused and ctx.tile_shape()[3] == -1 else 0
     names = kernel_names(ctx, wl)
     s_ms, v_ms = ctx.time_passes(20) if passes else (None, None)
     ctx.close()
     return dict(elapsed=el, stress_ms=s_ms, vel_ms=v_ms, tile=tile, tune_ms=tune_ms, finite=finite, fused=fused,
-                block=block, kernels=names, chains=chains)
+                block=block, march=march, kernels=names, chains=chains)
 
 
 STORE_TYPE = {0: "float", 1: "__half", 2: "__hip_bfloat16", 3: "double"}
@@ -155,6 +157,10 @@ def kernel_names(ctx, wl):
     # shape in place of a fused one)
     window = wl.punch_after is not None
     if kind == _lib.TILE_FUSED and not window:
+        if blk == -1:  # the marching step: its interior kernel and its frame's two passes
+            n = tuple("fd23::k_psv_march<%s, %d>" % (t, w) for w in (256, 512)) + \
+                tuple("fd23::k_psv_%s<%s, 4, 1, 2, true>" % (p, t) for p in ("stress", "velocity"))
+            return (n, n)
         # block rows 0: the tile-parallel fused step, segments of 4*CZ rows
         n = ("fd23::k_psv_fused_tile<%s, %d>" % (t, seg // 4),) if blk == 0 else \
             ("fd23::k_psv_fused<%s, %d, %d>" % (t, seg, blk),)
@@ -556,7 +562,12 @@ def measure_line(wl, steps, warmup, autotune=True, tile=None, chains=None):
     gcell = cells / r["elapsed"] / 1e9
     ms = r["elapsed"] / steps * 1e3
     sb, vb = pass_bytes(wl)
-    if r["fused"]:
+    if r["march"]:
+        # time_passes reports the time per step; a launch (the interior kernel
+        # and its frame) reads and writes the state once for `march` steps
+        name, nbytes, kms, kname = "march", fused_bytes(wl), r["stress_ms"] * r["march"], r["kernels"][0]
+        step_bytes = nbytes / r["march"]
+    elif r["fused"]:
         name, nbytes, kms, kname = "fused", fused_bytes(wl), r["stress_ms"], r["kernels"][0]
         step_bytes = nbytes
     elif r["block"]:

@@ -4,6 +4,7 @@
 #include "fd_kernels.hpp"
 #include "fd_fused.hpp"
 #include "fd_block.hpp"
+#include "fd_march.hpp"
 
 #include <hip/hip_runtime.h>
 
@@ -58,6 +59,7 @@ extern "C" void fd23_set_error_(const char *msg) { g_err = msg; }
 struct TileCfg {
     int rz, spb, fh, fr, split; // fused: segment height fh, rows per block fr
     int bk, bcz, bw;            // block: steps per launch, rows per thread, wavefronts
+    int mk;                     // march: steps per launch (its frame runs the rz, spb passes)
 };
 // tile 0, the shape untuned contexts run (the serving engine, the driver),
 // is the one the autotuner picks on most workloads measured
@@ -69,7 +71,8 @@ static constexpr TileCfg kTiles[] = {
     {0, 1, 0, 0, 0, 1, 3, 8},  {0, 1, 0, 0, 0, 1, 3, 16}, {0, 1, 0, 0, 0, 2, 3, 16},
     {0, 1, 0, 0, 0, 2, 4, 16}, {0, 1, 0, 0, 0, 2, 6, 8},
     {0, 1, 16, 0, 0}, {0, 1, 32, 0, 0}, {1, 1, 0, 0, 0},
-    {0, 1, 0, 0, 0, 2, 4, 10}, {0, 1, 0, 0, 0, 2, 3, 12}};
+    {0, 1, 0, 0, 0, 2, 4, 10}, {0, 1, 0, 0, 0, 2, 3, 12},
+    {4, 1, 0, 0, 1, 0, 0, 0, 2}};
 static const int kNumTiles = sizeof(kTiles) / sizeof(kTiles[0]);
 
 extern "C" int fd23_num_tiles(void) { return kNumTiles; }
@@ -78,8 +81,8 @@ extern "C" int fd23_tile_shape(int tile, int *rz, int *spb, int *seg_rows, int *
     const TileCfg &t = kTiles[tile];
     if (rz) *rz = t.bk > 0 ? t.bcz : t.rz;
     if (spb) *spb = t.spb;
-    if (seg_rows) *seg_rows = t.bk > 0 ? t.bk : t.fh;
-    if (block_rows) *block_rows = t.bk > 0 ? t.bw * t.bcz : t.fr;
+    if (seg_rows) *seg_rows = t.bk > 0 ? t.bk : t.mk > 0 ? t.mk : t.fh;
+    if (block_rows) *block_rows = t.bk > 0 ? t.bw * t.bcz : t.mk > 0 ? -1 : t.fr;
     return FD23_OK;
 }
 extern "C" int fd23_tile_split(int tile) {
@@ -88,7 +91,9 @@ extern "C" int fd23_tile_split(int tile) {
 }
 extern "C" int fd23_tile_kind(int tile) {
     if (tile < 0 || tile >= kNumTiles) return fail(FD23_EINVAL, "bad tile %d", tile);
-    return kTiles[tile].bk > 0 ? FD23_TILE_BLOCK : kTiles[tile].fh > 0 ? FD23_TILE_FUSED : FD23_TILE_TILED;
+    return kTiles[tile].bk > 0                           ? FD23_TILE_BLOCK
+           : kTiles[tile].fh > 0 || kTiles[tile].mk > 0 ? FD23_TILE_FUSED
+                                                        : FD23_TILE_TILED;
 }
 
 constexpr int kMaxTZ = 32;     // largest tile height (BY * max RZ)
@@ -196,6 +201,7 @@ struct fd23_ctx {
     int *d_nrec = nullptr;
     std::vector<long> h_roff;
     std::vector<int> h_nrec;
+    std::vector<int> h_recz; // deepest receiver row per shot and component
     void *seis = nullptr;
 
     int tile = 0;
@@ -352,6 +358,7 @@ extern "C" int fd23_ctx_create(const fd23_desc *desc, fd23_ctx **out) {
     c->nscale = psv ? SC_PSV_N : SC_SH_N;
     c->src.resize(d.nshots);
     c->h_nrec.assign((size_t)d.nshots * c->ncomp, 0);
+    c->h_recz.assign((size_t)d.nshots * c->ncomp, -1);
     c->h_roff.assign((size_t)d.nshots * c->ncomp * std::max(d.max_rec, 1), -1);
 
 #define ALLOC(ptr, n)                                                           \
@@ -411,7 +418,7 @@ extern "C" int fd23_ctx_create(const fd23_desc *desc, fd23_ctx **out) {
     ALLOC(c->d_fieldtab, sizeof(void *) * 5);
     ALLOC(c->d_comptab, sizeof(void *) * 2);
     ALLOC(c->d_compfield, sizeof(int) * 2);
-    ALLOC(c->scl, sizeof(float) * 2 * kNextScale);
+    ALLOC(c->scl, sizeof(float) * kScaleBanks);
     ALLOC(c->amax, sizeof(unsigned) * 16 * kAmaxSpread);
     ALLOC(c->clock, sizeof(int) * 2);
     ALLOC(c->d_src, sizeof(SrcInfo) * S);
@@ -426,7 +433,7 @@ extern "C" int fd23_ctx_create(const fd23_desc *desc, fd23_ctx **out) {
     hipMemcpy(c->d_comptab, comps, sizeof(void *) * 2, hipMemcpyHostToDevice);
     int cf[2] = {0, 1};
     hipMemcpy(c->d_compfield, cf, sizeof cf, hipMemcpyHostToDevice);
-    std::vector<float> ones(2 * kNextScale, 1.0f);
+    std::vector<float> ones(kScaleBanks, 1.0f);
     hipMemcpy(c->scl, ones.data(), sizeof(float) * ones.size(), hipMemcpyHostToDevice);
     hipMemcpy(c->d_roff, c->h_roff.data(), sizeof(long) * c->h_roff.size(), hipMemcpyHostToDevice);
     c->tile = (d.nshots >= 4) ? 4 : 0;
@@ -569,9 +576,10 @@ extern "C" int fd23_set_scales(fd23_ctx *c, const float *scales, int n) {
             return fail(FD23_EINVAL, "scale %d (%g) is not a power of two in [2^-%d, 2^%d]", i, scales[i],
                         kScaleExpMax, kScaleExpMax);
     }
-    // current and next scales alike
+    // current, next and previous scales alike
     HIPCHK(hipMemcpyAsync(c->scl, scales, sizeof(float) * n, hipMemcpyHostToDevice, c->stream));
     HIPCHK(hipMemcpyAsync(c->scl + kNextScale, scales, sizeof(float) * n, hipMemcpyHostToDevice, c->stream));
+    HIPCHK(hipMemcpyAsync(c->scl + kPrevScale, scales, sizeof(float) * n, hipMemcpyHostToDevice, c->stream));
     HIPCHK(hipStreamSynchronize(c->stream));
     c->scales_init = true;
     return FD23_OK;
@@ -717,17 +725,19 @@ extern "C" int fd23_set_receivers(fd23_ctx *c, int shot, int comp, const int *rx
     if (n > 0 && (!rx || !rz)) return fail(FD23_EINVAL, "null receiver arrays");
     const long nx = c->d.nx, N = nx * (long)c->d.nz;
     const long base = ((long)shot * c->ncomp + comp) * c->d.max_rec;
+    int deep = -1;
     for (int i = 0; i < c->d.max_rec; i++) {
         long off = -1;
         if (i < n) {
             // flat index rx + rz*nx (cu_record.cu:144): a receiver at x=-1
             // lands on the previous row's last cell
             long q = (long)rx[i] + (long)rz[i] * nx;
-            if (q >= 0 && q < N) off = (q / nx) * c->px + (q % nx);
+            if (q >= 0 && q < N) off = (q / nx) * c->px + (q % nx), deep = std::max(deep, (int)(q / nx));
         }
         c->h_roff[base + i] = off;
     }
     c->h_nrec[(size_t)shot * c->ncomp + comp] = n;
+    c->h_recz[(size_t)shot * c->ncomp + comp] = deep;
     HIPCHK(hipMemcpyAsync(c->d_roff + base, c->h_roff.data() + base, sizeof(long) * c->d.max_rec,
                           hipMemcpyHostToDevice, c->stream));
     HIPCHK(hipMemcpyAsync(c->d_nrec, c->h_nrec.data(), sizeof(int) * c->h_nrec.size(), hipMemcpyHostToDevice,
@@ -813,6 +823,7 @@ extern "C" int fd23_reset_shot(fd23_ctx *c, int shot) {
 // ---------------------------------------------------------------------------
 static bool tile_fused(int t) { return kTiles[t].fh > 0; }
 static bool tile_block(int t) { return kTiles[t].bk > 0; }
+static bool tile_march(int t) { return kTiles[t].mk > 0; }
 static bool scaled_storage(const fd23_ctx *c) {
     return c->d.storage == FD23_STORE_F16 || c->d.storage == FD23_STORE_BF16;
 }
@@ -823,6 +834,39 @@ static bool scaled_storage(const fd23_ctx *c) {
 static bool use_fused(const fd23_ctx *c) { return tile_fused(c->tile) && is_psv(c) && !c->box && !c->punch; }
 static bool use_block(const fd23_ctx *c) {
     return tile_block(c->tile) && !is_psv(c) && !scaled_storage(c) && !c->punch;
+}
+// The rectangle whose cells, and the 12 around them that a marching step
+// recomputes, run plain arithmetic (full order, no C-PML, no free surface);
+// its sides at multiples of 16 cells (64 bytes of FP32); false when there is
+// none.
+static bool march_rect(const fd23_ctx *c, MarchWork &w) {
+    const int lo = std::max(c->d.npml, 4) + kMarchReach, ztop = (c->d.topabsorb ? lo : 4 + kMarchReach);
+    w.x0 = round_up(lo, 16);
+    w.x1 = std::max(c->d.nx - lo, 0) / 16 * 16;
+    w.z0 = round_up(ztop, 16);
+    w.z1 = std::max(c->d.nz - lo, 0) / 16 * 16;
+    if (w.x1 <= w.x0 || w.z1 <= w.z0) return false;
+    // Sources and receivers near the surface are left to the frame when that
+    // costs the rectangle at most an eighth of its rows: items with events run
+    // checked rows, and a launch lasts as long as its slowest item (8 shots of
+    // 4096 x 2048 with the source at row 8: 972 against 712 us).
+    int deep = w.z0 - 1;
+    for (const HostSrc &h : c->src)
+        if (h.kind >= 0 && !h.stf.empty()) deep = std::max(deep, h.zs + 1 + kMarchReach);
+    for (int z : c->h_recz) deep = std::max(deep, z);
+    const int z0 = round_up(deep + 1, 16);
+    if (z0 - w.z0 <= (w.z1 - w.z0) / 8) w.z0 = z0;
+    return true;
+}
+// The marching step runs in fd23_run for P-SV contexts with FP32, FP16 or
+// BF16 storage that have such a rectangle, without a box, a first-arrival
+// window or idle slots (a slot that is left alone must keep its fields in
+// place), each shot's array within a buffer resource's 2 GiB.  Everything
+// else, and the last step of an odd run, takes the two passes.
+static bool use_march(const fd23_ctx *c) {
+    MarchWork w;
+    return tile_march(c->tile) && is_psv(c) && c->d.storage != FD23_STORE_F64 && !c->box && !c->punch && !c->idle &&
+           (size_t)c->sstride * c->csize < 0x7fffffffu && march_rect(c, w);
 }
 static int pass_tile(const fd23_ctx *c) { return tile_fused(c->tile) || tile_block(c->tile) ? 0 : c->tile; }
 static int tile_rows(const fd23_ctx *c) { return BY * kTiles[pass_tile(c)].rz; }
@@ -922,13 +966,49 @@ static int build_events(fd23_ctx *c) {
     return FD23_OK;
 }
 
+// Work of a marching launch.  Two wavefronts run on each SIMD (256 VGPRs),
+// 1024 workgroups of 256 columns or 512 of 512 columns on the chip at once; a
+// segment of H rows takes H + 24 iterations, whose time does not depend on the
+// width.  Width and segments are those with the least (rounds) x (H + 24), H
+// a multiple of the 8 rows of the unrolled loop: 8 shots of 4096 x 2048 take
+// 1008 items of 256 x 288 (701 us; 832 at H = 96, 925 at 392), 64 shots of
+// 1024 x 512 512 items of 512 x 112 (336 us; 384 with 256 columns).
+static MarchWork march_work(const fd23_ctx *c) {
+    MarchWork w;
+    march_rect(c, w);
+    const int rows = w.z1 - w.z0;
+    long best = LONG_MAX;
+    for (int W : {256, 512}) {
+        const int own = W - 2 * MH, nstrip = (w.x1 - w.x0 + own - 1) / own;
+        const long columns = (long)nstrip * c->d.nshots, slots = 262144 / W;
+        for (int H = round_up(rows, 8); H >= 16; H -= 8) {
+            const long seg = (rows + H - 1) / H, cost = (columns * seg + slots - 1) / slots * (H + kMarchTail);
+            if (cost < best) {
+                best = cost;
+                w.W = W;
+                w.nstrip = nstrip;
+                w.H = H;
+                w.nseg = (int)seg;
+            }
+        }
+    }
+    w.nwork = w.nstrip * w.nseg * c->d.nshots;
+    return w;
+}
+
 // Lists of the fused step: source taps per (strip, shot) -- every strip
 // whose 64 stress columns (its 56 own columns and 4 on each side) hold
 // the tap -- and receivers per (segment, strip, shot) sorted by row.
 static int build_fused_events(fd23_ctx *c) {
     if (!c->fevents_dirty && c->fevents_tile == c->tile) return FD23_OK;
-    const int H = kTiles[c->tile].fh;
-    const int nstrip = (c->d.nx + FO - 1) / FO, nseg = (c->d.nz + H - 1) / H;
+    // strips of `own` columns from x0 on, `halo` more on each side, segments
+    // of H rows from z0 on; the marching step's lists hold its rectangle
+    int H = kTiles[c->tile].fh, own = FO, halo = HALO, x0 = 0, z0 = 0, x1 = c->d.nx, z1 = c->d.nz, reach = c->d.nz;
+    if (use_march(c)) {
+        const MarchWork w = march_work(c);
+        H = w.H, own = w.W - 2 * MH, halo = MH, x0 = w.x0, z0 = w.z0, x1 = w.x1, z1 = w.z1, reach = kMarchReach;
+    }
+    const int nstrip = (x1 - x0 + own - 1) / own, nseg = (z1 - z0 + H - 1) / H;
     const int S = c->d.nshots;
     std::vector<std::vector<TapF>> tb((size_t)nstrip * S);
     std::vector<std::vector<RecF>> rb((size_t)nseg * nstrip * S);
@@ -937,9 +1017,10 @@ static int build_fused_events(fd23_ctx *c) {
         for (int i = 0; i < si.ntap; i++) {
             const Tap &tp = c->h_taps[si.tap0 + i];
             const int z = (int)(tp.off / c->px), x = (int)(tp.off % c->px);
+            if (z < z0 - reach || z >= z1 + reach) continue;
             for (int st = 0; st < nstrip; st++) {
-                const int lane = x - (st * FO - HALO);
-                if (lane >= 0 && lane < FW) tb[(size_t)st * S + s].push_back(TapF{z, lane, tp.field, tp.mode, tp.m, tp.q});
+                const int lane = x - (x0 + st * own - halo);
+                if (lane >= 0 && lane < own + 2 * halo) tb[(size_t)st * S + s].push_back(TapF{z, lane, tp.field, tp.mode, tp.m, tp.q});
             }
         }
         for (int comp = 0; comp < c->ncomp; comp++) {
@@ -949,8 +1030,10 @@ static int build_fused_events(fd23_ctx *c) {
                 const long off = c->h_roff[base + r];
                 if (off < 0) continue; // outside the grid: the frame keeps 0
                 const int z = (int)(off / c->px), x = (int)(off % c->px);
-                const int st = x / FO, sg = z / H;
-                rb[((size_t)sg * nstrip + st) * S + s].push_back(RecF{z, x - st * FO + HALO, comp, (int)(base + r)});
+                if (x < x0 || x >= x1 || z < z0 || z >= z1) continue;
+                const int st = (x - x0) / own, sg = (z - z0) / H;
+                rb[((size_t)sg * nstrip + st) * S + s].push_back(
+                    RecF{z, x - x0 - st * own + halo, comp, (int)(base + r)});
             }
         }
     }
@@ -1133,6 +1216,7 @@ static Work make_work(const fd23_ctx *c, int RZ, int SPB, dim3 &grid, int region
     w.ntz = (c->d.nz + TZ - 1) / TZ;
     w.ngroups = (c->d.nshots + SPB - 1) / SPB;
     w.g0 = 0;
+    w.kx0 = w.kx1 = w.kz0 = w.kz1 = 0;
     if (c->chain >= 0) { // part c->chain of c->chains of the shot groups
         const int h = (w.ngroups + c->chains - 1) / c->chains;
         w.g0 = std::min(c->chain * h, w.ngroups);
@@ -1196,16 +1280,16 @@ static void launch_stress_t(fd23_ctx *c, const Events &ev, unsigned *amax) {
                 const Work we = make_work(c, RZ, SPB, ge, REGION_EDGE);
                 if (wi.nwork > 0)
                     hipLaunchKernelGGL((k_psv_stress<S, RZ, SPB, REGION_INTERIOR>), gi, block, 0, c->stream, f, m, ps,
-                                       pr, g, wi, ev, c->scl, amax);
+                                       pr, g, wi, ev, c->scl, amax, f, ps);
                 if (we.nwork > 0)
                     hipLaunchKernelGGL((k_psv_stress<S, RZ, SPB, REGION_EDGE>), ge, block, 0, c->stream, f, m, ps,
-                                       pr, g, we, ev, c->scl, amax);
+                                       pr, g, we, ev, c->scl, amax, f, ps);
                 split_done = true;
             }
         }
         if (!split_done) {
             hipLaunchKernelGGL((k_psv_stress<S, RZ, SPB, REGION_ALL>), grid, block, 0, c->stream, f, m, ps, pr, g, w,
-                               ev, c->scl, amax);
+                               ev, c->scl, amax, f, ps);
         }
     } else {
         ShFields<S> f{(S *)c->fields[0], (S *)c->fields[1], (S *)c->fields[2]};
@@ -1240,16 +1324,16 @@ static void launch_velocity_t(fd23_ctx *c, const Events &ev, unsigned *amax) {
                 const Work we = make_work(c, RZ, SPB, ge, REGION_EDGE);
                 if (wi.nwork > 0)
                     hipLaunchKernelGGL((k_psv_velocity<S, RZ, SPB, REGION_INTERIOR>), gi, block, 0, c->stream, f, m,
-                                       ps, pr, g, wi, ev, c->scl, amax);
+                                       ps, pr, g, wi, ev, c->scl, amax, f, ps);
                 if (we.nwork > 0)
                     hipLaunchKernelGGL((k_psv_velocity<S, RZ, SPB, REGION_EDGE>), ge, block, 0, c->stream, f, m, ps,
-                                       pr, g, we, ev, c->scl, amax);
+                                       pr, g, we, ev, c->scl, amax, f, ps);
                 split_done = true;
             }
         }
         if (!split_done) {
             hipLaunchKernelGGL((k_psv_velocity<S, RZ, SPB, REGION_ALL>), grid, block, 0, c->stream, f, m, ps, pr, g,
-                               w, ev, c->scl, amax);
+                               w, ev, c->scl, amax, f, ps);
         }
     } else {
         ShFields<S> f{(S *)c->fields[0], (S *)c->fields[1], (S *)c->fields[2]};
@@ -1340,6 +1424,7 @@ template <class S, int CZ> static void launch_fused_tile_t(fd23_ctx *c, int k, i
     w.ntz = (c->d.nz + OZ - 1) / OZ;
     w.ngroups = c->d.nshots;
     w.g0 = 0;
+    w.kx0 = w.kx1 = w.kz0 = w.kz1 = 0;
     const int lo = std::max(c->d.npml, 4), ztop = c->d.topabsorb ? lo : 4;
     w.ix0 = (lo + HALO + FO - 1) / FO; // x0 - 4 >= lo
     w.ix1 = c->d.nx - lo - HALO - FO >= 0 ? (c->d.nx - lo - HALO - FO) / FO + 1 : 0; // x0 + 60 <= nx - lo
@@ -1410,6 +1495,97 @@ static void dispatch_fused(fd23_ctx *c, int k, int itrecord, bool record = true,
     case FD23_STORE_BF16: launch_fused_h<__hip_bfloat16>(c, k, itrecord, record, amax); break;
     case FD23_STORE_F64: launch_fused_h<double>(c, k, itrecord, record, nullptr); break;
     default: launch_fused_h<float>(c, k, itrecord, record, nullptr); break;
+    }
+    swap_sets(c);
+}
+
+// Marching step (k_psv_march): steps k and k+1, from the current set to the
+// other.  The frame around the rectangle runs the two passes of both steps in
+// the other set (the first ones read the current set), over the tiles that
+// hold a cell of the frame or of the 12 cells inside it that the frame's
+// stencils need; the marching kernel then writes every cell of the rectangle
+// from the current set.  scaled storage: between the first
+// step's passes their scales are committed as in the two-pass loop (commit),
+// the marching kernel still reads the current set in the previous ones.
+static void enqueue_commit(fd23_ctx *c, bool stress, bool save = true);
+template <class S>
+static void launch_march_t(fd23_ctx *c, int k, int itrecord, bool events, bool commit, unsigned *amax) {
+    using C = float;
+    const Grid g = make_grid(c);
+    const MarchWork mw = march_work(c);
+    const int TZ = BY * 4;
+    Work w{};
+    w.ntx = (c->d.nx + TX - 1) / TX;
+    w.ntz = (c->d.nz + TZ - 1) / TZ;
+    w.ngroups = c->d.nshots;
+    w.kx0 = mw.x0, w.kx1 = mw.x1, w.kz0 = mw.z0, w.kz1 = mw.z1;
+    // the tiles that hold a cell outside the rectangle or up to `reach` cells
+    // inside it
+    auto frame = [&](int reach) {
+        Work f = w;
+        f.ix0 = (mw.x0 + reach + TX - 1) / TX, f.ix1 = (mw.x1 - reach) / TX;
+        f.iz0 = (mw.z0 + reach + TZ - 1) / TZ, f.iz1 = (mw.z1 - reach) / TZ;
+        if (f.ix1 <= f.ix0 || f.iz1 <= f.iz0) f.ix0 = f.ix1 = f.iz0 = f.iz1 = 0;
+        f.ntiles = w.ntx * w.ntz - (f.ix1 - f.ix0) * (f.iz1 - f.iz0);
+        f.nwork = f.ntiles * f.ngroups;
+        return f;
+    };
+    const Work wide = frame(kMarchReach), narrow = frame(0);
+    const dim3 gw(round_up(wide.nwork, 8)), gn(round_up(std::max(narrow.nwork, 1), 8)), block(TX, BY);
+    auto fields = [](void *const *f) {
+        return PsvFields<S>{(S *)f[0], (S *)f[1], (S *)f[2], (S *)f[3], (S *)f[4]};
+    };
+    const PsvFields<S> fa = fields(c->fields), fb = fields(c->alt_fields);
+    auto spsi = [](void *const *p) { return PsvStressPsi<S>{(S *)p[2], (S *)p[3], (S *)p[6], (S *)p[7]}; };
+    auto vpsi = [](void *const *p) { return PsvVelPsi<S>{(S *)p[0], (S *)p[1], (S *)p[5], (S *)p[4]}; };
+    const PsvStressMat<C> sm{(const C *)c->mat[4], (const C *)c->mat[2], (const C *)c->mat[3]};
+    const PsvVelMat<C> vm{(const C *)c->mat[0], (const C *)c->mat[1]};
+    const PsvStressProf<C> spr{prof_of<C>(c, 2), prof_of<C>(c, 3), prof_of<C>(c, 6), prof_of<C>(c, 7)};
+    const PsvVelProf<C> vpr{prof_of<C>(c, 0), prof_of<C>(c, 1), prof_of<C>(c, 5), prof_of<C>(c, 4)};
+    for (int half = 0; half < 2; half++) {
+        const Events ev = events ? make_events(c, k + half, itrecord) : Events{};
+        unsigned *am = half ? amax : nullptr;
+        const PsvFields<S> f = half ? fb : fa;
+        hipLaunchKernelGGL((k_psv_stress<S, 4, 1, REGION_EDGE, true>), gw, block, 0, c->stream, f, sm,
+                           spsi(half ? c->alt_psi : c->psi), spr, g, wide, ev, c->scl, am, fb, spsi(c->alt_psi));
+        if (commit && !half) enqueue_commit(c, true, false);
+        hipLaunchKernelGGL((k_psv_velocity<S, 4, 1, REGION_EDGE, true>), half ? gn : gw, block, 0, c->stream, f, vm,
+                           vpsi(half ? c->alt_psi : c->psi), vpr, g, half ? narrow : wide, ev, c->scl, am, fb,
+                           vpsi(c->alt_psi));
+        if (commit && !half) enqueue_commit(c, false, false);
+    }
+    FusedEvents ev{};
+    if (events) {
+        ev.clock = c->clock;
+        ev.k = k;
+        ev.itrecord = itrecord;
+        ev.tap_start = c->d_ftap_start;
+        ev.taps = c->d_ftaps;
+        ev.src = c->d_src;
+        ev.stf = c->d_stf;
+        ev.rec_start = c->d_frec_start;
+        ev.recs = c->d_frecs;
+        ev.seis = c->seis;
+        ev.max_frames = c->seis ? c->d.max_frames : 0;
+        ev.frame_size = (long)c->d.nshots * c->ncomp * c->d.max_rec;
+    }
+    const PsvMat5<C> m{(const C *)c->mat[0], (const C *)c->mat[1], (const C *)c->mat[2], (const C *)c->mat[3],
+                       (const C *)c->mat[4]};
+    if (mw.W == 256)
+        hipLaunchKernelGGL((k_psv_march<S, 256>), dim3(round_up(mw.nwork, 8)), dim3(256 / NC), 0, c->stream, fa, fb, m,
+                           g, mw, ev, c->scl + kPrevScale, c->scl, amax);
+    else
+        hipLaunchKernelGGL((k_psv_march<S, 512>), dim3(round_up(mw.nwork, 8)), dim3(512 / NC), 0, c->stream, fa, fb, m,
+                           g, mw, ev, c->scl + kPrevScale, c->scl, amax);
+    if (commit) enqueue_commit(c, false, true);
+}
+static void dispatch_march(fd23_ctx *c, int k, int itrecord, bool events = true, bool commit = false,
+                           bool track = false) {
+    unsigned *amax = track ? c->amax : nullptr;
+    switch (c->d.storage) {
+    case FD23_STORE_F16: launch_march_t<__half>(c, k, itrecord, events, commit, amax); break;
+    case FD23_STORE_BF16: launch_march_t<__hip_bfloat16>(c, k, itrecord, events, commit, amax); break;
+    default: launch_march_t<float>(c, k, itrecord, events, commit, nullptr); break;
     }
     swap_sets(c);
 }
@@ -1574,6 +1750,7 @@ static int init_scales(fd23_ctx *c) {
     }
     HIPCHK(hipMemcpyAsync(c->scl, sc, sizeof sc, hipMemcpyHostToDevice, c->stream));
     HIPCHK(hipMemcpyAsync(c->scl + kNextScale, sc, sizeof sc, hipMemcpyHostToDevice, c->stream));
+    HIPCHK(hipMemcpyAsync(c->scl + kPrevScale, sc, sizeof sc, hipMemcpyHostToDevice, c->stream));
     HIPCHK(hipStreamSynchronize(c->stream));
     c->scales_init = true;
     return FD23_OK;
@@ -1601,8 +1778,10 @@ static unsigned pass_mask(const fd23_ctx *c, bool stress) {
                   : (1u << SC_V) | (1u << SC_PTX_X) | (1u << SC_PTZ_Z);
 }
 
-static void enqueue_commit(fd23_ctx *c, bool stress) {
-    hipLaunchKernelGGL(k_commit_scales, dim3(1), dim3(64), 0, c->stream, c->scl, pass_mask(c, stress));
+// after the velocity pass no array is left in the scales before the check
+static void enqueue_commit(fd23_ctx *c, bool stress, bool save) {
+    hipLaunchKernelGGL(k_commit_scales, dim3(1), dim3(64), 0, c->stream, c->scl, pass_mask(c, stress),
+                       save && !stress);
 }
 
 // a step bound truncated toward zero as the reference's int() does, held
@@ -1740,6 +1919,13 @@ static int enqueue_launch(fd23_ctx *c, int k, int left, int itrecord, int *taken
         *taken = n;
         return FD23_OK;
     }
+    if (use_march(c) && left >= 2) { // k is even: a scale check never falls between the two steps
+        const bool sc = scaled_storage(c), check = (k + 2) % kScaleEvery == 0;
+        dispatch_march(c, k, itrecord, !c->timing, sc && k % kScaleEvery == 0, sc && check);
+        if (sc && check) enqueue_scale_control(c);
+        *taken = 2;
+        return FD23_OK;
+    }
     *taken = 1;
     return enqueue_step(c, k, itrecord);
 }
@@ -1756,7 +1942,7 @@ static int enqueue_launch(fd23_ctx *c, int k, int left, int itrecord, int *taken
 // the autotuner decides).  The two-pass path with more than one shot group
 // and no state shared by the halves (scales, box, window).
 static bool chains_possible(const fd23_ctx *c, int n = 2) {
-    if (use_fused(c) || use_block(c) || scaled_storage(c) || c->box || c->punch) return false;
+    if (use_fused(c) || use_block(c) || use_march(c) || scaled_storage(c) || c->box || c->punch) return false;
     const int spb = kTiles[pass_tile(c)].spb;
     return (c->d.nshots + spb - 1) / spb >= n; // a shot group per chain at least
 }
@@ -1828,7 +2014,7 @@ static int run_prologue(fd23_ctx *c, int it0, int nt, int itrecord) {
         return fail(FD23_EINVAL, "the box and the first-arrival window run every shot from step 0");
     if (c->box && (r = fd23_box_check_run(c, it0, nt))) return r;
     if ((r = build_events(c))) return r;
-    if (use_fused(c) && ((r = ensure_alt(c)) || (r = build_fused_events(c)))) return r;
+    if ((use_fused(c) || use_march(c)) && ((r = ensure_alt(c)) || (r = build_fused_events(c)))) return r;
     if (use_block(c) && ((r = ensure_alt(c)) || (r = build_block_events(c)))) return r;
     return init_scales(c);
 }
@@ -1970,7 +2156,7 @@ extern "C" int fd23_set_state(fd23_ctx *c, int shot, const void *buf, size_t byt
 // ---------------------------------------------------------------------------
 extern "C" int fd23_set_tile(fd23_ctx *c, int tile) {
     if (!c || tile < 0 || tile >= kNumTiles) return fail(FD23_EINVAL, "bad tile %d", tile);
-    if (tile_fused(tile) && !is_psv(c)) return fail(FD23_EINVAL, "the fused step is P-SV only");
+    if ((tile_fused(tile) || tile_march(tile)) && !is_psv(c)) return fail(FD23_EINVAL, "the fused step is P-SV only");
     if (tile_block(tile) && (is_psv(c) || scaled_storage(c)))
         return fail(FD23_EINVAL, "the block step is SH with FP32 or FP64 storage only");
     if (tile_fused(tile) && kTiles[tile].fr == 0 && scaled_storage(c))
@@ -1991,6 +2177,7 @@ extern "C" double fd23_bytes_per_step(const fd23_ctx *c) {
     const double nzp = (c->d.topabsorb ? 2.0 : 1.0) * c->d.npml * c->d.nx;
     // the fused step reads the five fields once and writes them once
     if (is_psv(c) && use_fused(c)) return S * (10 * wf * N + 8 * wf * (nxp + nzp)) + 5 * wm * N;
+    if (use_march(c)) return (S * (10 * wf * N + 8 * wf * (nxp + nzp)) + 5 * wm * N) / kTiles[c->tile].mk;
     // the block step reads the state (V Tx Tz, four psi) and the material
     // once per launch of bk steps and writes the state once
     if (use_block(c)) return (S * (6 * wf * N + 4 * wf * (nxp + nzp)) + 3 * wm * N) / kTiles[c->tile].bk;
@@ -2007,7 +2194,8 @@ extern "C" int fd23_time_passes(fd23_ctx *c, int nsteps, double *stress_ms, doub
     HIPCHK(hipEventCreate(&e1));
     HIPCHK(hipEventCreate(&e2));
     const bool sc = scaled_storage(c);
-    const bool fused = use_fused(c), block = use_block(c);
+    const bool fused = use_fused(c), block = use_block(c), march = use_march(c);
+    if (march && (r = ensure_alt(c))) return r;
     if (fused && ((r = ensure_alt(c)) || (r = build_fused_events(c)))) return r;
     if (block && (r = ensure_alt(c))) return r;
     if (block) {
@@ -2017,6 +2205,14 @@ extern "C" int fd23_time_passes(fd23_ctx *c, int nsteps, double *stress_ms, doub
         dispatch_block(c, 0, K, 1, false);
         hipEventRecord(e0, c->stream);
         for (int i = 0; i < nsteps; i++) dispatch_block(c, 0, K, 1, false);
+        hipEventRecord(e1, c->stream);
+        hipEventRecord(e2, c->stream);
+    } else if (march) {
+        // nsteps marching launches of two steps back to back (no sources or
+        // receivers): the first value is the time per step, the second 0
+        dispatch_march(c, 0, 1, false, sc);
+        hipEventRecord(e0, c->stream);
+        for (int i = 0; i < nsteps; i++) dispatch_march(c, 0, 1, false);
         hipEventRecord(e1, c->stream);
         hipEventRecord(e2, c->stream);
     } else if (fused) {
@@ -2055,7 +2251,7 @@ extern "C" int fd23_time_passes(fd23_ctx *c, int nsteps, double *stress_ms, doub
     hipEventDestroy(e1);
     hipEventDestroy(e2);
     if (se != hipSuccess) return fail(FD23_EHIP, "%s", hipGetErrorString(se));
-    const int per = block ? kTiles[c->tile].bk : 1; // steps per launch
+    const int per = block ? kTiles[c->tile].bk : march ? kTiles[c->tile].mk : 1; // steps per launch
     if (stress_ms) *stress_ms = a / nsteps / per;
     if (velocity_ms) *velocity_ms = b / nsteps / per;
     return check_launch();
@@ -2132,7 +2328,7 @@ extern "C" int fd23_autotune(fd23_ctx *c, int steps, double *best_ms) {
         return r;
     }
     // scales and running maxima too (FP16/BF16 storage)
-    float scl_saved[2 * kNextScale];
+    float scl_saved[kScaleBanks];
     std::vector<unsigned> amax_saved((size_t)16 * kAmaxSpread);
     HIPCHK(hipMemcpy(scl_saved, c->scl, sizeof scl_saved, hipMemcpyDeviceToHost));
     HIPCHK(hipMemcpy(amax_saved.data(), c->amax, sizeof(unsigned) * amax_saved.size(), hipMemcpyDeviceToHost));
@@ -2150,6 +2346,7 @@ extern "C" int fd23_autotune(fd23_ctx *c, int steps, double *best_ms) {
         if (tile_block(t) && (is_psv(c) || scaled_storage(c) || c->punch)) continue;
         if (tile_fused(t) && kTiles[t].fr == 0 && scaled_storage(c)) continue;
         c->tile = t;
+        if (tile_march(t) && !use_march(c)) continue; // would run as the split two-pass shape
         double a, b;
         fd23_time_passes(c, 1, &a, &b); // warm-up
         // the faster of two timings, so that one slow interval does not
@@ -2175,7 +2372,7 @@ extern "C" int fd23_autotune(fd23_ctx *c, int steps, double *best_ms) {
     c->chains = 1;
     if (c->cur != orig_set) swap_sets(c);
     c->tile = best;
-    auto two_pass = [](int t) { return !tile_fused(t) && !tile_block(t); };
+    auto two_pass = [](int t) { return !tile_fused(t) && !tile_block(t) && !tile_march(t); };
     if (r == FD23_OK && two_pass(best) && chains_possible(c)) {
         std::vector<int> cands;
         for (const auto &ct : timed) {

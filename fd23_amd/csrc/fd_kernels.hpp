@@ -67,7 +67,14 @@ struct Work {
     int ntiles;            // tiles of this launch's region
     int nwork;             // ntiles*ngroups (logical workgroups)
     int g0;                // first shot group of the launch
+    // frame launches of the marching step: the cells of this rectangle that
+    // the frame's tiles hold are computed for their neighbours' sake; another
+    // kernel writes them last, records their receivers, tracks their maxima
+    int kx0, kx1, kz0, kz1;
 };
+__device__ __forceinline__ bool cell_kept(const Work &w, int x, int z) {
+    return x >= w.kx0 && x < w.kx1 && z >= w.kz0 && z < w.kz1;
+}
 struct TileId {
     int tile, group, x0, z0; // tile: index in the whole grid (ntx per row)
 };
@@ -317,8 +324,9 @@ template <class C> struct PsvStressProf {
 // Tzz_z Txz_z U_z W_z = 5..12
 enum { SC_U = 0, SC_W, SC_TXX, SC_TZZ, SC_TXZ, SC_PTXX_X, SC_PTXZ_X, SC_PU_X, SC_PW_X,
        SC_PTZZ_Z, SC_PTXZ_Z, SC_PU_Z, SC_PW_Z, SC_PSV_N };
-// scale buffer: current scales [0, kNextScale), next scales after them
-constexpr int kNextScale = 16;
+// scale buffer: current scales [0, kNextScale), next scales after them, then
+// those of the step before the last commit (the set a marching step reads)
+constexpr int kNextScale = 16, kPrevScale = 32, kScaleBanks = 48;
 constexpr int kScaleExpMax = 100;
 
 // ---------------------------------------------------------------------------
@@ -390,12 +398,19 @@ __device__ __forceinline__ void psv_stress_exact(const Grid &g, int ix, int iz, 
     }
 }
 
-template <class S, int RZ, int SPB, int REGION>
+// TO: the updated arrays are written to another buffer set (fo, po) instead
+// of in place, for the first of the two steps of a marching launch's frame
+template <class S, int RZ, int SPB, int REGION, bool TO = false>
 __global__ __launch_bounds__(TX *BY) void k_psv_stress(PsvFields<S> f, PsvStressMat<typename Store<S>::C> m,
                                                        PsvStressPsi<S> ps,
                                                        PsvStressProf<typename Store<S>::C> pr, Grid g, Work w,
                                                        Events ev, const float *__restrict__ scl,
-                                                       unsigned *__restrict__ amax) {
+                                                       unsigned *__restrict__ amax, PsvFields<S> fo,
+                                                       PsvStressPsi<S> po) {
+    if (!TO) {
+        fo = f;
+        po = ps;
+    }
     using C = typename Store<S>::C;
     using ST = Store<S>;
     constexpr int TZ = BY * RZ;
@@ -474,6 +489,8 @@ __global__ __launch_bounds__(TX *BY) void k_psv_stress(PsvFields<S> f, PsvStress
         const long org = (long)shot * g.sstride - (long)HALO * px - HALO;
         const BufRsrc bU = buf_rsrc(f.U + org), bW = buf_rsrc(f.W + org);
         const BufRsrc bXX = buf_rsrc(f.Txx + org), bZZ = buf_rsrc(f.Tzz + org), bXZ = buf_rsrc(f.Txz + org);
+        const BufRsrc oXX = TO ? buf_rsrc(fo.Txx + org) : bXX, oZZ = TO ? buf_rsrc(fo.Tzz + org) : bZZ,
+                      oXZ = TO ? buf_rsrc(fo.Txz + org) : bXZ;
         Stage<S, TZ, true, true> rU, rW;
         rU.loadb(bU, pxb, vcol, x0, z0, ty, sc_u);
         rW.loadb(bW, pxb, vcol, x0, z0, ty, sc_w);
@@ -541,11 +558,11 @@ __global__ __launch_bounds__(TX *BY) void k_psv_stress(PsvFields<S> f, PsvStress
                 const C wz = dp(pw, LW, c0, c1, c2, c3);
                 if constexpr (kPrePsi)
                     psv_stress_exact<S, C, true>(g, ix, iz, shot, ux, uz, wx, wz, lam[r], mu[r], mua[r], txx[r],
-                                                 tzz[r], txz[r], ps, ps, true, pr, psc, mp, pq[0][r], pq[1][r],
+                                                 tzz[r], txz[r], ps, po, true, pr, psc, mp, pq[0][r], pq[1][r],
                                                  pq[2][r], pq[3][r]);
                 else
                     psv_stress_exact<S, C>(g, ix, iz, shot, ux, uz, wx, wz, lam[r], mu[r], mua[r], txx[r], tzz[r],
-                                           txz[r], ps, ps, true, pr, psc, mp);
+                                           txz[r], ps, po, true, pr, psc, mp);
             }
         }
         // fused source injection: the owner of a tap cell adds it after the
@@ -574,10 +591,10 @@ __global__ __launch_bounds__(TX *BY) void k_psv_stress(PsvFields<S> f, PsvStress
             const int gz = z0 + lz0 + r;
             if (gx >= nx || gz >= nz) continue;
             const unsigned so = (unsigned)(gz + HALO) * pxb;
-            ST::stb(bXX, vcol, so, txx[r], wi_xx);
-            ST::stb(bZZ, vcol, so, tzz[r], wi_zz);
-            ST::stb(bXZ, vcol, so, txz[r], wi_xz);
-            if (ST::scaled && amax) { // the maxima are gathered on the step before a check
+            ST::stb(oXX, vcol, so, txx[r], wi_xx);
+            ST::stb(oZZ, vcol, so, tzz[r], wi_zz);
+            ST::stb(oXZ, vcol, so, txz[r], wi_xz);
+            if (ST::scaled && amax && !(TO && cell_kept(w, gx, gz))) { // the maxima are gathered on the step before a check
                 mx_xx = fmaxf(mx_xx, fabsf((float)txx[r]));
                 mx_zz = fmaxf(mx_zz, fabsf((float)tzz[r]));
                 mx_xz = fmaxf(mx_xz, fabsf((float)txz[r]));
@@ -597,10 +614,11 @@ __global__ __launch_bounds__(TX *BY) void k_psv_stress(PsvFields<S> f, PsvStress
 
 // gather fused into a velocity pass: the new values of the tile are parked
 // in LDS (the staging buffers are free once every wave has computed), then
-// the tile's receivers read them.  Uniform per workgroup.
-template <class C, int RZ, int NC>
+// the tile's receivers read them.  Uniform per workgroup.  KEPT: receivers
+// in the work's kept rectangle are recorded by another kernel.
+template <class C, int RZ, int NV, bool KEPT = false>
 __device__ __forceinline__ void fused_record(const Events &ev, int it, int key, C *park0, C *park1,
-                                             const C (&val)[NC][RZ], int lz0, int t0) {
+                                             const C (&val)[NV][RZ], int lz0, int t0, const Work &w, int x0, int z0) {
     const int e0 = ev.rec_start[key], e1 = ev.rec_start[key + 1];
     const int ts = it - t0; // step of the shot
     if (e1 <= e0 || ts < 0 || ts % ev.itrecord != 0) return;
@@ -610,12 +628,13 @@ __device__ __forceinline__ void fused_record(const Events &ev, int it, int key, 
 #pragma unroll
     for (int r = 0; r < RZ; r++) {
         park0[(lz0 + r) * TX + threadIdx.x] = val[0][r];
-        if (NC > 1) park1[(lz0 + r) * TX + threadIdx.x] = val[NC - 1][r];
+        if (NV > 1) park1[(lz0 + r) * TX + threadIdx.x] = val[NV - 1][r];
     }
     __syncthreads();
     C *seis = (C *)ev.seis + (long)frame * ev.frame_size;
     for (int e = e0 + threadIdx.y * TX + threadIdx.x; e < e1; e += TX * BY) {
         const RecT rc = ev.recs[e];
+        if (KEPT && cell_kept(w, x0 + rc.cell % TX, z0 + rc.cell / TX)) continue;
         seis[rc.out] = rc.comp == 0 ? park0[rc.cell] : park1[rc.cell];
     }
 }
@@ -689,12 +708,18 @@ __device__ __forceinline__ void psv_velocity_exact(const Grid &g, int ix, int iz
     }
 }
 
-template <class S, int RZ, int SPB, int REGION>
+// TO: as in k_psv_stress; the stresses are those of the other set
+template <class S, int RZ, int SPB, int REGION, bool TO = false>
 __global__ __launch_bounds__(TX *BY) void k_psv_velocity(PsvFields<S> f, PsvVelMat<typename Store<S>::C> m,
                                                          PsvVelPsi<S> ps,
                                                          PsvVelProf<typename Store<S>::C> pr, Grid g, Work w,
                                                          Events ev, const float *__restrict__ scl,
-                                                         unsigned *__restrict__ amax) {
+                                                         unsigned *__restrict__ amax, PsvFields<S> fo,
+                                                         PsvVelPsi<S> po) {
+    if (!TO) {
+        fo = f;
+        po = ps;
+    }
     using C = typename Store<S>::C;
     using ST = Store<S>;
     constexpr int TZ = BY * RZ;
@@ -768,7 +793,8 @@ __global__ __launch_bounds__(TX *BY) void k_psv_velocity(PsvFields<S> f, PsvVelM
         // buffer origin of this shot's arrays: element (row -HALO, column -HALO)
         const long org = (long)shot * g.sstride - (long)HALO * px - HALO;
         const BufRsrc bU = buf_rsrc(f.U + org), bW = buf_rsrc(f.W + org);
-        const BufRsrc bXX = buf_rsrc(f.Txx + org), bZZ = buf_rsrc(f.Tzz + org), bXZ = buf_rsrc(f.Txz + org);
+        const BufRsrc bXX = buf_rsrc(fo.Txx + org), bZZ = buf_rsrc(fo.Tzz + org), bXZ = buf_rsrc(fo.Txz + org);
+        const BufRsrc oU = TO ? buf_rsrc(fo.U + org) : bU, oW = TO ? buf_rsrc(fo.W + org) : bW;
         Stage<S, TZ, false, true> rXX;
         Stage<S, TZ, true, false> rZZ;
         Stage<S, TZ, true, true> rXZ;
@@ -837,11 +863,11 @@ __global__ __launch_bounds__(TX *BY) void k_psv_velocity(PsvFields<S> f, PsvVelM
                 const C dzTxz = dp(&sXZ[o], LW, c0, c1, c2, c3);
                 if constexpr (kPrePsi)
                     psv_velocity_exact<S, C, true>(g, ix, iz, shot, dxTxx, dzTzz, dxTxz, dzTxz, bu[r], bw[r],
-                                                   nv[0][r], nv[1][r], ps, ps, true, pr, psc, mp, pq[0][r],
+                                                   nv[0][r], nv[1][r], ps, po, true, pr, psc, mp, pq[0][r],
                                                    pq[1][r], pq[2][r], pq[3][r]);
                 else
                     psv_velocity_exact<S, C>(g, ix, iz, shot, dxTxx, dzTzz, dxTxz, dzTxz, bu[r], bw[r], nv[0][r],
-                                             nv[1][r], ps, ps, true, pr, psc, mp);
+                                             nv[1][r], ps, po, true, pr, psc, mp);
             }
         }
 #pragma unroll
@@ -849,14 +875,15 @@ __global__ __launch_bounds__(TX *BY) void k_psv_velocity(PsvFields<S> f, PsvVelM
             const int gz = z0 + lz0 + r;
             if (gx >= nx || gz >= nz) continue;
             const unsigned so = (unsigned)(gz + HALO) * pxb;
-            ST::stb(bU, vcol, so, nv[0][r], wi_u);
-            ST::stb(bW, vcol, so, nv[1][r], wi_w);
-            if (ST::scaled && amax) { // the maxima are gathered on the step before a check
+            ST::stb(oU, vcol, so, nv[0][r], wi_u);
+            ST::stb(oW, vcol, so, nv[1][r], wi_w);
+            if (ST::scaled && amax && !(TO && cell_kept(w, gx, gz))) { // the maxima are gathered on the step before a check
                 mx_u = fmaxf(mx_u, fabsf((float)nv[0][r]));
                 mx_w = fmaxf(mx_w, fabsf((float)nv[1][r]));
             }
         }
-        if (ev.clock) fused_record<C, RZ, 2>(ev, it, t.tile * g.nshots + shot, sXX, sZZ, nv, lz0, ev.src[shot].t0);
+        if (ev.clock)
+            fused_record<C, RZ, 2, TO>(ev, it, t.tile * g.nshots + shot, sXX, sZZ, nv, lz0, ev.src[shot].t0, w, x0, z0);
     }
     if (ST::scaled) {
         amax_update(amax, SC_U, mx_u);
@@ -1221,7 +1248,7 @@ __global__ __launch_bounds__(TX *BY) void k_sh_velocity(ShFields<S> f, const typ
             ST::stb(bV, vcol, (unsigned)(gz + HALO) * pxb, nv[0][r], wi_v);
             if (ST::scaled && amax) mx_v = fmaxf(mx_v, fabsf((float)nv[0][r]));
         }
-        if (ev.clock) fused_record<C, RZ, 1>(ev, it, t.tile * g.nshots + shot, sX, sX, nv, lz0, ev.src[shot].t0);
+        if (ev.clock) fused_record<C, RZ, 1>(ev, it, t.tile * g.nshots + shot, sX, sX, nv, lz0, ev.src[shot].t0, w, x0, z0);
     }
     if (ST::scaled) {
         amax_update(amax, SC_V, mx_v);
@@ -1334,10 +1361,14 @@ __global__ void k_scale_control(float *scl, unsigned *amax, int n, int lo, int h
     }
 }
 
-// the arrays a pass has rewritten now hold values in the next scales
-__global__ void k_commit_scales(float *scl, unsigned mask) {
+// the arrays a pass has rewritten now hold values in the next scales; save:
+// no array is left in an older scale
+__global__ void k_commit_scales(float *scl, unsigned mask, bool save) {
     const int f = threadIdx.x;
-    if (f < kNextScale && ((mask >> f) & 1u)) scl[f] = scl[kNextScale + f];
+    if (f >= kNextScale) return;
+    const float cur = (mask >> f) & 1u ? scl[kNextScale + f] : scl[f];
+    scl[f] = cur;
+    if (save) scl[kPrevScale + f] = cur;
 }
 
 // Rows of w values between a pitched array in its storage type and a packed

@@ -61,8 +61,6 @@ struct TileCfg {
     int bk, bcz, bw;            // block: steps per launch, rows per thread, wavefronts
     int mk;                     // march: steps per launch (its frame runs the rz, spb passes)
 };
-// tile 0, the shape untuned contexts run (the serving engine, the driver),
-// is the one the autotuner picks on most workloads measured
 static constexpr TileCfg kTiles[] = {
     {2, 1, 0, 0, 0},   {4, 1, 0, 0, 0},   {8, 1, 0, 0, 0},    {4, 2, 0, 0, 0},   {4, 4, 0, 0, 0},
     {4, 8, 0, 0, 0},   {8, 2, 0, 0, 0},   {8, 4, 0, 0, 0},    {2, 4, 0, 0, 0},   {2, 8, 0, 0, 0},
@@ -74,6 +72,44 @@ static constexpr TileCfg kTiles[] = {
     {0, 1, 0, 0, 0, 2, 4, 10}, {0, 1, 0, 0, 0, 2, 3, 12},
     {4, 1, 0, 0, 1, 0, 0, 0, 2}};
 static const int kNumTiles = sizeof(kTiles) / sizeof(kTiles[0]);
+
+enum { kTileTwo = 0, kTileFour = 1, kTileBlock2x16 = 20, kTileOne = 25, kTileBlock2x12 = 27, kTileMarch = 28 };
+
+// The shape of a context that is not tuned (the serving engine, the par-file
+// programs), from its cells N = nx*nz*nshots and storage.  Each line is where
+// the faster of two shapes changes, us per step of 64 replayed steps:
+//  - SH, FP32/FP64: the two-step block shapes while their workgroups (one per
+//    36 x 8 or 36 x 20 cells) fit one per CU: 256 x 128 5.3 against 7.1 (tile
+//    25) and 8.5 (tile 0), 400 x 200 6.0 / 7.2 / 8.7; past that 256 x 128 x 8
+//    10.8 / 9.0 / 9.0;
+//  - one row per thread up to 300 K cells (P-SV FP32 256 x 128 7.8 against
+//    10.2, 512 x 256 x 2 10.2 / 11.3, 1024 x 512 14.9 / 14.2), 200 K with
+//    16-bit P-SV storage, 600 K in FP64 (1024 x 512 21.5 / 23.2);
+//  - the marching step where the five fields outgrow the 256 MB MALL, 200 MB
+//    of them (2000 x 1000 x 8 168 against 227, x 4 102 / 90; FP16 1400 x 900
+//    x 16 184 / 191), on grids mostly interior;
+//  - four rows per thread for large SH and 16-bit P-SV batches (SH 1024 x 512
+//    x 16 69 / 75, x 2 15.9 / 15.5; P-SV FP16 2000 x 1000 x 4 87 / 99); two
+//    rows otherwise.
+static int default_tile(const fd23_desc &d) {
+    const double N = (double)d.nx * d.nz * d.nshots;
+    const bool psv = d.wave == FD23_WAVE_PSV, f64 = d.storage == FD23_STORE_F64;
+    const bool half = d.storage == FD23_STORE_F16 || d.storage == FD23_STORE_BF16;
+    if (!psv && !half) {
+        auto groups = [&](int ox, int oz) {
+            return (double)((d.nx + ox - 1) / ox) * ((d.nz + oz - 1) / oz) * d.nshots;
+        };
+        if (groups(36, 8) <= 256) return kTileBlock2x12;
+        if (groups(36, 20) <= 256) return kTileBlock2x16;
+    }
+    if (N <= (psv && half ? 2e5 : psv && f64 ? 6e5 : 3e5)) return kTileOne;
+    if (psv) {
+        const double inner = std::max(0.0, d.nx - 2.0 * (d.npml + 16)) * std::max(0.0, d.nz - 1.5 * (d.npml + 16));
+        if (!f64 && 5.0 * (half ? 2 : 4) * N >= 2e8 && inner >= 0.6 * d.nx * d.nz) return kTileMarch;
+        return half && N >= 5e6 ? kTileFour : kTileTwo;
+    }
+    return N >= (half ? 1e6 : 2e6) ? kTileFour : kTileTwo;
+}
 
 extern "C" int fd23_num_tiles(void) { return kNumTiles; }
 extern "C" int fd23_tile_shape(int tile, int *rz, int *spb, int *seg_rows, int *block_rows) {
@@ -436,7 +472,7 @@ extern "C" int fd23_ctx_create(const fd23_desc *desc, fd23_ctx **out) {
     std::vector<float> ones(kScaleBanks, 1.0f);
     hipMemcpy(c->scl, ones.data(), sizeof(float) * ones.size(), hipMemcpyHostToDevice);
     hipMemcpy(c->d_roff, c->h_roff.data(), sizeof(long) * c->h_roff.size(), hipMemcpyHostToDevice);
-    c->tile = (d.nshots >= 4) ? 4 : 0;
+    c->tile = default_tile(d);
     hipError_t e = hipDeviceSynchronize();
     if (e != hipSuccess) {
         free_ctx(c);

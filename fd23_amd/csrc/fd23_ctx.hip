@@ -1607,12 +1607,7 @@ static void launch_march_t(fd23_ctx *c, int k, int itrecord, bool events, bool c
     }
     const PsvMat5<C> m{(const C *)c->mat[0], (const C *)c->mat[1], (const C *)c->mat[2], (const C *)c->mat[3],
                        (const C *)c->mat[4]};
-    if (mw.W == 256)
-        hipLaunchKernelGGL((k_psv_march<S, 256>), dim3(round_up(mw.nwork, 8)), dim3(256 / NC), 0, c->stream, fa, fb, m,
-                           g, mw, ev, c->scl + kPrevScale, c->scl, amax);
-    else
-        hipLaunchKernelGGL((k_psv_march<S, 512>), dim3(round_up(mw.nwork, 8)), dim3(512 / NC), 0, c->stream, fa, fb, m,
-                           g, mw, ev, c->scl + kPrevScale, c->scl, amax);
+    march_launch<S>(c->stream, fa, fb, m, g, mw, ev, c->scl + kPrevScale, c->scl, amax);
     if (commit) enqueue_commit(c, false, true);
 }
 static void dispatch_march(fd23_ctx *c, int k, int itrecord, bool events = true, bool commit = false,

@@ -1331,7 +1331,7 @@ __global__ void k_record(S *const *comps, int ncomp, long sstride, const long *_
 // rescale kernel multiplies the stored data by the (exact) power-of-two
 // ratio of old to new scale.
 // ===========================================================================
-__global__ void k_scale_control(float *scl, unsigned *amax, int n, int lo, int hi, int target) {
+static __global__ void k_scale_control(float *scl, unsigned *amax, int n, int lo, int hi, int target) {
     __shared__ unsigned red[kAmaxSpread];
     const int t = threadIdx.x; // blockDim.x == kAmaxSpread
     for (int f = 0; f < n; f++) {
@@ -1363,7 +1363,7 @@ __global__ void k_scale_control(float *scl, unsigned *amax, int n, int lo, int h
 
 // the arrays a pass has rewritten now hold values in the next scales; save:
 // no array is left in an older scale
-__global__ void k_commit_scales(float *scl, unsigned mask, bool save) {
+static __global__ void k_commit_scales(float *scl, unsigned mask, bool save) {
     const int f = threadIdx.x;
     if (f >= kNextScale) return;
     const float cur = (mask >> f) & 1u ? scl[kNextScale + f] : scl[f];
@@ -1416,7 +1416,7 @@ static __global__ __launch_bounds__(256) void k_zero_regions(ZeroRegions z) {
 }
 
 // advance the step clock after a captured chunk of steps
-__global__ void k_tick(int *clock, int steps) {
+static __global__ void k_tick(int *clock, int steps) {
     if (threadIdx.x == 0) clock[0] += steps;
 }
 
@@ -1424,12 +1424,12 @@ __global__ void k_tick(int *clock, int steps) {
 struct PtrTable5 {
     void *p[5];
 };
-__global__ void k_set_ptrs(void **tab, PtrTable5 v, int n) {
+static __global__ void k_set_ptrs(void **tab, PtrTable5 v, int n) {
     if (threadIdx.x < n) tab[threadIdx.x] = v.p[threadIdx.x];
 }
 
 // set the step clock in stream order (no host round trip)
-__global__ void k_set_clock(int *clock, int it0) {
+static __global__ void k_set_clock(int *clock, int it0) {
     if (threadIdx.x == 0) clock[0] = it0;
 }
 

@@ -475,4 +475,10 @@ __global__ __launch_bounds__(MW / NC, 2) void k_psv_march(PsvFields<S> fa, PsvFi
         march_item<S, MW, false, false>(fa, fb, m, g, w, ev, sa, scl, amax, q, l);
 }
 
+// fd23_march.hip
+template <class S>
+void march_launch(hipStream_t stream, const PsvFields<S> &fa, const PsvFields<S> &fb, const PsvMat5<float> &m,
+                  const Grid &g, const MarchWork &w, const FusedEvents &ev, const float *sa, const float *scl,
+                  unsigned *amax);
+
 } // namespace fd23

@@ -150,9 +150,13 @@ def kernel_names(ctx, wl):
         if kind == _lib.TILE_BLOCK and wl.punch_after is None:
             n = ("fd23::k_sh_block<%s, %d, %d, %d>" % (t, seg, rz, blk // rz),)
             return (n, n)
+        if blk == -1 and wl.storage == 0 and wl.punch_after is None:  # the marching step and its frame's passes
+            n = tuple("fd23::k_sh_march<%d>" % w for w in (256, 512)) + \
+                tuple("fd23::k_sh_%s<float, 4, 1, true>" % p for p in ("stress", "velocity"))
+            return (n, n)
         if kind != _lib.TILE_TILED:  # a window runs tile 0's tiled kernels
             rz, spb = ctx.tile_shape(0)[:2]
-        return (("fd23::k_sh_stress<%s, %d, %d>" % (t, rz, spb),), ("fd23::k_sh_velocity<%s, %d, %d>" % (t, rz, spb),))
+        return tuple(("fd23::k_sh_%s<%s, %d, %d, false>" % (p, t, rz, spb),) for p in ("stress", "velocity"))
     # a first-arrival window runs the whole-grid tiled kernels (tile 0's
     # shape in place of a fused one)
     window = wl.punch_after is not None

@@ -88,8 +88,12 @@ enum { kTileTwo = 0, kTileFour = 1, kTileBlock2x16 = 20, kTileOne = 25, kTileBlo
 //  - the marching step where the five fields outgrow the 256 MB MALL, 200 MB
 //    of them (2000 x 1000 x 8 168 against 227, x 4 102 / 90; FP16 1400 x 900
 //    x 16 184 / 191), on grids mostly interior;
-//  - four rows per thread for large SH and 16-bit P-SV batches (SH 1024 x 512
-//    x 16 69 / 75, x 2 15.9 / 15.5; P-SV FP16 2000 x 1000 x 4 87 / 99); two
+//  - the SH marching step, FP32, from 3.5 M cells on grids still more
+//    interior, where it is ahead of four rows per thread by little at first
+//    (1400 x 900 x 3 34 / 36, 1024 x 512 x 16 60 / 68, 2048 x 1024 x 6 68 / 88,
+//    4096 x 2048 x 4 135 / 271; 512 x 256 x 64 69 / 66, 2000 x 1000 27 / 24);
+//  - four rows per thread for large SH and 16-bit P-SV batches (SH FP64 and
+//    16-bit, 1024 x 512 x 16 69 / 75 in FP32, x 2 15.9 / 15.5; P-SV FP16 2000 x 1000 x 4 87 / 99); two
 //    rows otherwise.
 static int default_tile(const fd23_desc &d) {
     const double N = (double)d.nx * d.nz * d.nshots;
@@ -103,11 +107,12 @@ static int default_tile(const fd23_desc &d) {
         if (groups(36, 20) <= 256) return kTileBlock2x16;
     }
     if (N <= (psv && half ? 2e5 : psv && f64 ? 6e5 : 3e5)) return kTileOne;
+    const double inner = std::max(0.0, d.nx - 2.0 * (d.npml + 16)) * std::max(0.0, d.nz - 1.5 * (d.npml + 16));
     if (psv) {
-        const double inner = std::max(0.0, d.nx - 2.0 * (d.npml + 16)) * std::max(0.0, d.nz - 1.5 * (d.npml + 16));
         if (!f64 && 5.0 * (half ? 2 : 4) * N >= 2e8 && inner >= 0.6 * d.nx * d.nz) return kTileMarch;
         return half && N >= 5e6 ? kTileFour : kTileTwo;
     }
+    if (!f64 && !half && N >= 3.5e6 && inner >= 0.75 * d.nx * d.nz) return kTileMarch;
     return N >= (half ? 1e6 : 2e6) ? kTileFour : kTileTwo;
 }
 
@@ -899,13 +904,13 @@ static bool march_rect(const fd23_ctx *c, MarchWork &w) {
     return true;
 }
 // The marching step runs in fd23_run for P-SV contexts with FP32, FP16 or
-// BF16 storage that have such a rectangle, without a box, a first-arrival
+// BF16 storage and SH contexts with FP32 that have such a rectangle, without a box, a first-arrival
 // window or idle slots (a slot that is left alone must keep its fields in
 // place), each shot's array within a buffer resource's 2 GiB.  Everything
 // else, and the last step of an odd run, takes the two passes.
 static bool use_march(const fd23_ctx *c) {
     MarchWork w;
-    return tile_march(c->tile) && is_psv(c) && c->d.storage != FD23_STORE_F64 && !c->box && !c->punch && !c->idle &&
+    return tile_march(c->tile) && (is_psv(c) ? c->d.storage != FD23_STORE_F64 : c->d.storage == FD23_STORE_F32) && !c->box && !c->punch && !c->idle &&
            (size_t)c->sstride * c->csize < 0x7fffffffu && march_rect(c, w);
 }
 static int pass_tile(const fd23_ctx *c) { return tile_fused(c->tile) || tile_block(c->tile) ? 0 : c->tile; }
@@ -1348,7 +1353,7 @@ static void launch_stress_t(fd23_ctx *c, const Events &ev, unsigned *amax) {
         ShPsi2<S> ps{(S *)c->psi[1], (S *)c->psi[3]};
         ShProf2<C> pr{prof_of<C>(c, 1), prof_of<C>(c, 3)};
         hipLaunchKernelGGL((k_sh_stress<S, RZ, SPB>), grid, block, 0, c->stream, f, m, ps, pr, g, w, ev, c->scl,
-                           amax);
+                           amax, f, ps);
     }
 }
 
@@ -1391,7 +1396,7 @@ static void launch_velocity_t(fd23_ctx *c, const Events &ev, unsigned *amax) {
         ShPsi2<S> ps{(S *)c->psi[0], (S *)c->psi[2]};
         ShProf2<C> pr{prof_of<C>(c, 0), prof_of<C>(c, 2)};
         hipLaunchKernelGGL((k_sh_velocity<S, RZ, SPB>), grid, block, 0, c->stream, f, (const C *)c->mat[0], ps,
-                           pr, g, w, ev, c->scl, amax);
+                           pr, g, w, ev, c->scl, amax, f, ps);
     }
 }
 
@@ -1555,33 +1560,52 @@ static void dispatch_fused(fd23_ctx *c, int k, int itrecord, bool record = true,
 // the other set (the first ones read the current set), over the tiles that
 // hold a cell of the frame or of the 12 cells inside it that the frame's
 // stencils need; the marching kernel then writes every cell of the rectangle
-// from the current set.  scaled storage: between the first
+// from the current set.  The frame's passes load their C-PML memory variables
+// and profile entries ahead of the barrier: read where they are used, each row
+// waited for two loads in turn (SH, one 2000 x 1000 shot: 7.7 us a pass, 6.0
+// so; P-SV, 8 shots of 4096 x 2048: 460 us a step, 454).  Scaled storage: between the first
 // step's passes their scales are committed as in the two-pass loop (commit),
 // the marching kernel still reads the current set in the previous ones.
+// the tiles that hold a cell outside the rectangle or up to `reach` cells
+// inside it
+static Work march_frame(const fd23_ctx *c, const MarchWork &mw, int reach) {
+    const int TZ = BY * 4;
+    Work f{};
+    f.ntx = (c->d.nx + TX - 1) / TX;
+    f.ntz = (c->d.nz + TZ - 1) / TZ;
+    f.ngroups = c->d.nshots;
+    f.kx0 = mw.x0, f.kx1 = mw.x1, f.kz0 = mw.z0, f.kz1 = mw.z1;
+    f.ix0 = (mw.x0 + reach + TX - 1) / TX, f.ix1 = (mw.x1 - reach) / TX;
+    f.iz0 = (mw.z0 + reach + TZ - 1) / TZ, f.iz1 = (mw.z1 - reach) / TZ;
+    if (f.ix1 <= f.ix0 || f.iz1 <= f.iz0) f.ix0 = f.ix1 = f.iz0 = f.iz1 = 0;
+    f.ntiles = f.ntx * f.ntz - (f.ix1 - f.ix0) * (f.iz1 - f.iz0);
+    f.nwork = f.ntiles * f.ngroups;
+    return f;
+}
+static FusedEvents march_events(const fd23_ctx *c, int k, int itrecord, bool events) {
+    FusedEvents ev{};
+    if (!events) return ev;
+    ev.clock = c->clock;
+    ev.k = k;
+    ev.itrecord = itrecord;
+    ev.tap_start = c->d_ftap_start;
+    ev.taps = c->d_ftaps;
+    ev.src = c->d_src;
+    ev.stf = c->d_stf;
+    ev.rec_start = c->d_frec_start;
+    ev.recs = c->d_frecs;
+    ev.seis = c->seis;
+    ev.max_frames = c->seis ? c->d.max_frames : 0;
+    ev.frame_size = (long)c->d.nshots * c->ncomp * c->d.max_rec;
+    return ev;
+}
 static void enqueue_commit(fd23_ctx *c, bool stress, bool save = true);
 template <class S>
 static void launch_march_t(fd23_ctx *c, int k, int itrecord, bool events, bool commit, unsigned *amax) {
     using C = float;
     const Grid g = make_grid(c);
     const MarchWork mw = march_work(c);
-    const int TZ = BY * 4;
-    Work w{};
-    w.ntx = (c->d.nx + TX - 1) / TX;
-    w.ntz = (c->d.nz + TZ - 1) / TZ;
-    w.ngroups = c->d.nshots;
-    w.kx0 = mw.x0, w.kx1 = mw.x1, w.kz0 = mw.z0, w.kz1 = mw.z1;
-    // the tiles that hold a cell outside the rectangle or up to `reach` cells
-    // inside it
-    auto frame = [&](int reach) {
-        Work f = w;
-        f.ix0 = (mw.x0 + reach + TX - 1) / TX, f.ix1 = (mw.x1 - reach) / TX;
-        f.iz0 = (mw.z0 + reach + TZ - 1) / TZ, f.iz1 = (mw.z1 - reach) / TZ;
-        if (f.ix1 <= f.ix0 || f.iz1 <= f.iz0) f.ix0 = f.ix1 = f.iz0 = f.iz1 = 0;
-        f.ntiles = w.ntx * w.ntz - (f.ix1 - f.ix0) * (f.iz1 - f.iz0);
-        f.nwork = f.ntiles * f.ngroups;
-        return f;
-    };
-    const Work wide = frame(kMarchReach), narrow = frame(0);
+    const Work wide = march_frame(c, mw, kMarchReach), narrow = march_frame(c, mw, 0);
     const dim3 gw(round_up(wide.nwork, 8)), gn(round_up(std::max(narrow.nwork, 1), 8)), block(TX, BY);
     auto fields = [](void *const *f) {
         return PsvFields<S>{(S *)f[0], (S *)f[1], (S *)f[2], (S *)f[3], (S *)f[4]};
@@ -1605,28 +1629,43 @@ static void launch_march_t(fd23_ctx *c, int k, int itrecord, bool events, bool c
                            vpsi(c->alt_psi));
         if (commit && !half) enqueue_commit(c, false, false);
     }
-    FusedEvents ev{};
-    if (events) {
-        ev.clock = c->clock;
-        ev.k = k;
-        ev.itrecord = itrecord;
-        ev.tap_start = c->d_ftap_start;
-        ev.taps = c->d_ftaps;
-        ev.src = c->d_src;
-        ev.stf = c->d_stf;
-        ev.rec_start = c->d_frec_start;
-        ev.recs = c->d_frecs;
-        ev.seis = c->seis;
-        ev.max_frames = c->seis ? c->d.max_frames : 0;
-        ev.frame_size = (long)c->d.nshots * c->ncomp * c->d.max_rec;
-    }
+    const FusedEvents ev = march_events(c, k, itrecord, events);
     const PsvMat5<C> m{(const C *)c->mat[0], (const C *)c->mat[1], (const C *)c->mat[2], (const C *)c->mat[3],
                        (const C *)c->mat[4]};
     march_launch<S>(c->stream, fa, fb, m, g, mw, ev, c->scl + kPrevScale, c->scl, amax);
     if (commit) enqueue_commit(c, false, true);
 }
+// the same for SH, FP32
+static void launch_sh_march(fd23_ctx *c, int k, int itrecord, bool events) {
+    const Grid g = make_grid(c);
+    const MarchWork mw = march_work(c);
+    const Work wide = march_frame(c, mw, kMarchReach), narrow = march_frame(c, mw, 0);
+    const dim3 gw(round_up(wide.nwork, 8)), gn(round_up(std::max(narrow.nwork, 1), 8)), block(TX, BY);
+    auto fields = [](void *const *f) { return ShFields<float>{(float *)f[0], (float *)f[1], (float *)f[2]}; };
+    auto psi = [](void *const *p, int i) { return ShPsi2<float>{(float *)p[i], (float *)p[i + 2]}; };
+    const ShFields<float> fa = fields(c->fields), fb = fields(c->alt_fields);
+    const ShStressMat<float> sm{(const float *)c->mat[1], (const float *)c->mat[2]};
+    const ShProf2<float> spr{prof_of<float>(c, 1), prof_of<float>(c, 3)}, vpr{prof_of<float>(c, 0), prof_of<float>(c, 2)};
+    for (int half = 0; half < 2; half++) {
+        const Events ev = events ? make_events(c, k + half, itrecord) : Events{};
+        const ShFields<float> f = half ? fb : fa;
+        void *const *p = half ? c->alt_psi : c->psi;
+        hipLaunchKernelGGL((k_sh_stress<float, 4, 1, true>), gw, block, 0, c->stream, f, sm, psi(p, 1), spr, g, wide, ev,
+                           c->scl, (unsigned *)nullptr, fb, psi(c->alt_psi, 1));
+        hipLaunchKernelGGL((k_sh_velocity<float, 4, 1, true>), half ? gn : gw, block, 0, c->stream, f,
+                           (const float *)c->mat[0], psi(p, 0), vpr, g, half ? narrow : wide, ev, c->scl,
+                           (unsigned *)nullptr, fb, psi(c->alt_psi, 0));
+    }
+    const ShMat3<float> m{(const float *)c->mat[0], (const float *)c->mat[1], (const float *)c->mat[2]};
+    sh_march_launch(c->stream, fa, fb, m, g, mw, march_events(c, k, itrecord, events));
+}
 static void dispatch_march(fd23_ctx *c, int k, int itrecord, bool events = true, bool commit = false,
                            bool track = false) {
+    if (!is_psv(c)) {
+        launch_sh_march(c, k, itrecord, events);
+        swap_sets(c);
+        return;
+    }
     unsigned *amax = track ? c->amax : nullptr;
     switch (c->d.storage) {
     case FD23_STORE_F16: launch_march_t<__half>(c, k, itrecord, events, commit, amax); break;
@@ -2218,7 +2257,7 @@ extern "C" int fd23_set_state(fd23_ctx *c, int shot, const void *buf, size_t byt
 // ---------------------------------------------------------------------------
 extern "C" int fd23_set_tile(fd23_ctx *c, int tile) {
     if (!c || tile < 0 || tile >= kNumTiles) return fail(FD23_EINVAL, "bad tile %d", tile);
-    if ((tile_fused(tile) || tile_march(tile)) && !is_psv(c)) return fail(FD23_EINVAL, "the fused step is P-SV only");
+    if (tile_fused(tile) && !is_psv(c)) return fail(FD23_EINVAL, "the fused step is P-SV only");
     if (tile_block(tile) && (is_psv(c) || scaled_storage(c)))
         return fail(FD23_EINVAL, "the block step is SH with FP32 or FP64 storage only");
     if (tile_fused(tile) && kTiles[tile].fr == 0 && scaled_storage(c))
@@ -2239,7 +2278,8 @@ extern "C" double fd23_bytes_per_step(const fd23_ctx *c) {
     const double nzp = (c->d.topabsorb ? 2.0 : 1.0) * c->d.npml * c->d.nx;
     // the fused step reads the five fields once and writes them once
     if (is_psv(c) && use_fused(c)) return S * (10 * wf * N + 8 * wf * (nxp + nzp)) + 5 * wm * N;
-    if (use_march(c)) return (S * (10 * wf * N + 8 * wf * (nxp + nzp)) + 5 * wm * N) / kTiles[c->tile].mk;
+    if (use_march(c) && is_psv(c)) return (S * (10 * wf * N + 8 * wf * (nxp + nzp)) + 5 * wm * N) / kTiles[c->tile].mk;
+    if (use_march(c)) return (S * (6 * wf * N + 4 * wf * (nxp + nzp)) + 3 * wm * N) / kTiles[c->tile].mk;
     // the block step reads the state (V Tx Tz, four psi) and the material
     // once per launch of bk steps and writes the state once
     if (use_block(c)) return (S * (6 * wf * N + 4 * wf * (nxp + nzp)) + 3 * wm * N) / kTiles[c->tile].bk;
@@ -2403,7 +2443,7 @@ extern "C" int fd23_autotune(fd23_ctx *c, int steps, double *best_ms) {
         // shapes that would run as another one: SH and a first-arrival
         // window run split shapes unsplit, the window and the box run fused
         // shapes as tile 0, and the window runs block shapes as tile 0
-        if (kTiles[t].split && (!is_psv(c) || c->punch)) continue;
+        if (kTiles[t].split && !tile_march(t) && (!is_psv(c) || c->punch)) continue;
         if (tile_fused(t) && (!is_psv(c) || c->box || c->punch)) continue;
         if (tile_block(t) && (is_psv(c) || scaled_storage(c) || c->punch)) continue;
         if (tile_fused(t) && kTiles[t].fr == 0 && scaled_storage(c)) continue;

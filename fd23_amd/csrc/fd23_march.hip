@@ -1,7 +1,8 @@
-// Instances of the marching P-SV kernel (a translation unit of its own: each
+// Instances of the marching kernels (a translation unit of its own: each
 // holds three or six unrolled row loops).
 #include "fd23.h"
 #include "fd_march.hpp"
+#include "fd_sh_march.hpp"
 
 namespace fd23 {
 
@@ -24,5 +25,12 @@ INSTANCE(float)
 INSTANCE(__half)
 INSTANCE(__hip_bfloat16)
 #undef INSTANCE
+
+void sh_march_launch(hipStream_t stream, const ShFields<float> &fa, const ShFields<float> &fb, const ShMat3<float> &m,
+                     const Grid &g, const MarchWork &w, const FusedEvents &ev) {
+    const dim3 grid((w.nwork + 7) / 8 * 8), block(w.W / NC);
+    if (w.W == 256) hipLaunchKernelGGL((k_sh_march<256>), grid, block, 0, stream, fa, fb, m, g, w, ev);
+    else hipLaunchKernelGGL((k_sh_march<512>), grid, block, 0, stream, fa, fb, m, g, w, ev);
+}
 
 } // namespace fd23

@@ -37,9 +37,6 @@ template <class S> struct ShPsi4 {
 template <class C> struct ShProf4 {
     Prof<C> Tx_x, V_x, Tz_z, V_z;
 };
-template <class C> struct ShMat3 {
-    const C *BV, *MUX, *MUZ;
-};
 struct BlockWork {
     int ntx, ntz;  // tiles in x and z
     int nwork;     // ntx*ntz*nshots (logical workgroups)

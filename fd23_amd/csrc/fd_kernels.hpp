@@ -317,6 +317,13 @@ template <class C> struct PsvStressMat {
 template <class S> struct PsvStressPsi {
     S *Ux, *Wx, *Uz, *Wz; // shot 0
 };
+// one profile entry, loaded ahead
+template <class C> struct PmlCoef {
+    C b, c, k;
+};
+template <class C> __device__ __forceinline__ PmlCoef<C> pml_coef(const Prof<C> &p, int i, bool in) {
+    return in ? PmlCoef<C>{p.b[i], p.c[i], p.k[i]} : PmlCoef<C>{C(0), C(0), C(0)};
+}
 template <class C> struct PsvStressProf {
     Prof<C> Ux, Wx, Uz, Wz;
 };
@@ -353,20 +360,21 @@ __device__ __forceinline__ void psv_stress_exact(const Grid &g, int ix, int iz, 
                                                  C lm, C mm, C ma, C &a, C &b, C &cc, const PsvStressPsi<S> &rd,
                                                  const PsvStressPsi<S> &wr, bool own,
                                                  const PsvStressProf<C> &pr, const PsiScl4 &sc, float (&mp)[4],
-                                                 C q0 = C(0), C q1 = C(0), C q2 = C(0), C q3 = C(0)) {
+                                                 C q0 = C(0), C q1 = C(0), C q2 = C(0), C q3 = C(0),
+                                                 const PmlCoef<C> *xv = nullptr, const PmlCoef<C> *zv = nullptr) {
     using ST = Store<S>;
     const int nx = g.nx, nz = g.nz, npml = g.npml;
     const C gam = lm + C(2.0) * mm;
     if (ix < npml || ix >= nx - npml) {
         const long pi = (long)shot * g.xpsi_stride + xpsi_idx(ix, iz, nx, npml);
-        C p1 = mad(pr.Ux.b[ix], PRE ? q0 : ST::ld(rd.Ux, pi, sc.r[0]), pr.Ux.c[ix] * ux);
+        C p1 = mad((PRE ? xv[0].b : pr.Ux.b[ix]), PRE ? q0 : ST::ld(rd.Ux, pi, sc.r[0]), (PRE ? xv[0].c : pr.Ux.c[ix]) * ux);
         if (own) ST::st(wr.Ux, pi, p1, sc.w[0]);
-        const C e1 = mad(ux, pr.Ux.k[ix], p1);
+        const C e1 = mad(ux, (PRE ? xv[0].k : pr.Ux.k[ix]), p1);
         a = mad(gam, e1, a);
         b = mad(lm, e1, b);
-        C p2 = mad(pr.Wx.b[ix], PRE ? q1 : ST::ld(rd.Wx, pi, sc.r[1]), pr.Wx.c[ix] * wx);
+        C p2 = mad((PRE ? xv[1].b : pr.Wx.b[ix]), PRE ? q1 : ST::ld(rd.Wx, pi, sc.r[1]), (PRE ? xv[1].c : pr.Wx.c[ix]) * wx);
         if (own) ST::st(wr.Wx, pi, p2, sc.w[1]);
-        cc = mad(ma, mad(wx, pr.Wx.k[ix], p2), cc);
+        cc = mad(ma, mad(wx, (PRE ? xv[1].k : pr.Wx.k[ix]), p2), cc);
         if (ST::scaled && own) {
             mp[0] = fmaxf(mp[0], fabsf((float)p1));
             mp[1] = fmaxf(mp[1], fabsf((float)p2));
@@ -377,14 +385,14 @@ __device__ __forceinline__ void psv_stress_exact(const Grid &g, int ix, int iz, 
     const bool topcell = iz < npml && g.top;
     if (topcell || iz >= nz - npml) {
         const long pi = (long)shot * g.zpsi_stride + zpsi_idx(ix, iz, nx, nz, npml, topcell);
-        C p1 = mad(pr.Wz.b[iz], PRE ? q2 : ST::ld(rd.Wz, pi, sc.r[3]), pr.Wz.c[iz] * wz);
+        C p1 = mad((PRE ? zv[0].b : pr.Wz.b[iz]), PRE ? q2 : ST::ld(rd.Wz, pi, sc.r[3]), (PRE ? zv[0].c : pr.Wz.c[iz]) * wz);
         if (own) ST::st(wr.Wz, pi, p1, sc.w[3]);
-        const C e1 = mad(wz, pr.Wz.k[iz], p1);
+        const C e1 = mad(wz, (PRE ? zv[0].k : pr.Wz.k[iz]), p1);
         a = mad(lm, e1, a);
         b = mad(gam, e1, b);
-        C p2 = mad(pr.Uz.b[iz], PRE ? q3 : ST::ld(rd.Uz, pi, sc.r[2]), pr.Uz.c[iz] * uz);
+        C p2 = mad((PRE ? zv[1].b : pr.Uz.b[iz]), PRE ? q3 : ST::ld(rd.Uz, pi, sc.r[2]), (PRE ? zv[1].c : pr.Uz.c[iz]) * uz);
         if (own) ST::st(wr.Uz, pi, p2, sc.w[2]);
-        cc = mad(ma, mad(uz, pr.Uz.k[iz], p2), cc);
+        cc = mad(ma, mad(uz, (PRE ? zv[1].k : pr.Uz.k[iz]), p2), cc);
         if (ST::scaled && own) {
             mp[2] = fmaxf(mp[2], fabsf((float)p1));
             mp[3] = fmaxf(mp[3], fabsf((float)p2));
@@ -480,6 +488,23 @@ __global__ __launch_bounds__(TX *BY) void k_psv_stress(PsvFields<S> f, PsvStress
         mua[r] = live ? Store<C>::ldb(rMUA, vmat, so, 1.f) : C(0);
     }
 
+    // edge-only kernels: so are the profile entries of the thread's column and
+    // rows, once for all shots; read where they are used, each of the rows
+    // waited for two loads in turn
+    PmlCoef<C> xv[2], zv[kPrePsi ? RZ : 1][2];
+    if constexpr (kPrePsi) {
+        const bool inx = gx < nx && (gx < g.npml || gx >= nx - g.npml);
+        xv[0] = pml_coef(pr.Ux, gx, inx);
+        xv[1] = pml_coef(pr.Wx, gx, inx);
+#pragma unroll
+        for (int r = 0; r < RZ; r++) {
+            const int iz = z0 + lz0 + r;
+            const bool inz = iz < nz && ((iz < g.npml && g.top) || iz >= nz - g.npml);
+            zv[r][0] = pml_coef(pr.Wz, iz, inz);
+            zv[r][1] = pml_coef(pr.Uz, iz, inz);
+        }
+    }
+
     const int sh0 = t.group * SPB;
     for (int s = 0; s < SPB; s++) {
         const int shot = sh0 + s;
@@ -559,7 +584,7 @@ __global__ __launch_bounds__(TX *BY) void k_psv_stress(PsvFields<S> f, PsvStress
                 if constexpr (kPrePsi)
                     psv_stress_exact<S, C, true>(g, ix, iz, shot, ux, uz, wx, wz, lam[r], mu[r], mua[r], txx[r],
                                                  tzz[r], txz[r], ps, po, true, pr, psc, mp, pq[0][r], pq[1][r],
-                                                 pq[2][r], pq[3][r]);
+                                                 pq[2][r], pq[3][r], xv, zv[r]);
                 else
                     psv_stress_exact<S, C>(g, ix, iz, shot, ux, uz, wx, wz, lam[r], mu[r], mua[r], txx[r], tzz[r],
                                            txz[r], ps, po, true, pr, psc, mp);
@@ -665,17 +690,18 @@ __device__ __forceinline__ void psv_velocity_exact(const Grid &g, int ix, int iz
                                                    C dxTxz, C dzTxz, C b_u, C b_w, C &u, C &ww,
                                                    const PsvVelPsi<S> &rd, const PsvVelPsi<S> &wr, bool own,
                                                    const PsvVelProf<C> &pr, const PsiScl4 &sc, float (&mp)[4],
-                                                   C q0 = C(0), C q1 = C(0), C q2 = C(0), C q3 = C(0)) {
+                                                   C q0 = C(0), C q1 = C(0), C q2 = C(0), C q3 = C(0),
+                                                   const PmlCoef<C> *xv = nullptr, const PmlCoef<C> *zv = nullptr) {
     using ST = Store<S>;
     const int nx = g.nx, nz = g.nz, npml = g.npml;
     if (ix < npml || ix >= nx - npml) {
         const long pi = (long)shot * g.xpsi_stride + xpsi_idx(ix, iz, nx, npml);
-        C p1 = mad(pr.Txx_x.b[ix], PRE ? q0 : ST::ld(rd.Txx_x, pi, sc.r[0]), pr.Txx_x.c[ix] * dxTxx);
+        C p1 = mad((PRE ? xv[0].b : pr.Txx_x.b[ix]), PRE ? q0 : ST::ld(rd.Txx_x, pi, sc.r[0]), (PRE ? xv[0].c : pr.Txx_x.c[ix]) * dxTxx);
         if (own) ST::st(wr.Txx_x, pi, p1, sc.w[0]);
-        u = mad(b_u, mad(dxTxx, pr.Txx_x.k[ix], p1), u);
-        C p2 = mad(pr.Txz_x.b[ix], PRE ? q1 : ST::ld(rd.Txz_x, pi, sc.r[1]), pr.Txz_x.c[ix] * dxTxz);
+        u = mad(b_u, mad(dxTxx, (PRE ? xv[0].k : pr.Txx_x.k[ix]), p1), u);
+        C p2 = mad((PRE ? xv[1].b : pr.Txz_x.b[ix]), PRE ? q1 : ST::ld(rd.Txz_x, pi, sc.r[1]), (PRE ? xv[1].c : pr.Txz_x.c[ix]) * dxTxz);
         if (own) ST::st(wr.Txz_x, pi, p2, sc.w[1]);
-        ww = mad(b_w, mad(dxTxz, pr.Txz_x.k[ix], p2), ww);
+        ww = mad(b_w, mad(dxTxz, (PRE ? xv[1].k : pr.Txz_x.k[ix]), p2), ww);
         if (ST::scaled && own) {
             mp[0] = fmaxf(mp[0], fabsf((float)p1));
             mp[1] = fmaxf(mp[1], fabsf((float)p2));
@@ -687,14 +713,14 @@ __device__ __forceinline__ void psv_velocity_exact(const Grid &g, int ix, int iz
     const bool topcell = iz < npml && g.top;
     if (topcell || iz >= nz - npml) {
         const long pi = (long)shot * g.zpsi_stride + zpsi_idx(ix, iz, nx, nz, npml, topcell);
-        C p1 = mad(pr.Txz_z.b[iz], PRE ? q2 : ST::ld(rd.Txz_z, pi, sc.r[2]), pr.Txz_z.c[iz] * dzTxz);
-        C p2 = mad(pr.Tzz_z.b[iz], PRE ? q3 : ST::ld(rd.Tzz_z, pi, sc.r[3]), pr.Tzz_z.c[iz] * dzTzz);
+        C p1 = mad((PRE ? zv[0].b : pr.Txz_z.b[iz]), PRE ? q2 : ST::ld(rd.Txz_z, pi, sc.r[2]), (PRE ? zv[0].c : pr.Txz_z.c[iz]) * dzTxz);
+        C p2 = mad((PRE ? zv[1].b : pr.Tzz_z.b[iz]), PRE ? q3 : ST::ld(rd.Tzz_z, pi, sc.r[3]), (PRE ? zv[1].c : pr.Tzz_z.c[iz]) * dzTzz);
         if (own) {
             ST::st(wr.Txz_z, pi, p1, sc.w[2]);
             ST::st(wr.Tzz_z, pi, p2, sc.w[3]);
         }
-        u = mad(b_u, mad(dzTxz, pr.Txz_z.k[iz], p1), u);
-        ww = mad(b_w, mad(dzTzz, pr.Tzz_z.k[iz], p2), ww);
+        u = mad(b_u, mad(dzTxz, (PRE ? zv[0].k : pr.Txz_z.k[iz]), p1), u);
+        ww = mad(b_w, mad(dzTzz, (PRE ? zv[1].k : pr.Tzz_z.k[iz]), p2), ww);
         if (ST::scaled && own) {
             mp[2] = fmaxf(mp[2], fabsf((float)p1));
             mp[3] = fmaxf(mp[3], fabsf((float)p2));
@@ -783,6 +809,23 @@ __global__ __launch_bounds__(TX *BY) void k_psv_velocity(PsvFields<S> f, PsvVelM
         bw[r] = live ? Store<C>::ldb(rBW, vmat, so, 1.f) : C(0);
     }
 
+    // edge-only kernels: so are the profile entries of the thread's column and
+    // rows, once for all shots; read where they are used, each of the rows
+    // waited for two loads in turn
+    PmlCoef<C> xv[2], zv[kPrePsi ? RZ : 1][2];
+    if constexpr (kPrePsi) {
+        const bool inx = gx < nx && (gx < g.npml || gx >= nx - g.npml);
+        xv[0] = pml_coef(pr.Txx_x, gx, inx);
+        xv[1] = pml_coef(pr.Txz_x, gx, inx);
+#pragma unroll
+        for (int r = 0; r < RZ; r++) {
+            const int iz = z0 + lz0 + r;
+            const bool inz = iz < nz && ((iz < g.npml && g.top) || iz >= nz - g.npml);
+            zv[r][0] = pml_coef(pr.Txz_z, iz, inz);
+            zv[r][1] = pml_coef(pr.Tzz_z, iz, inz);
+        }
+    }
+
     const int sh0 = t.group * SPB;
     for (int s = 0; s < SPB; s++) {
         const int shot = sh0 + s;
@@ -864,7 +907,7 @@ __global__ __launch_bounds__(TX *BY) void k_psv_velocity(PsvFields<S> f, PsvVelM
                 if constexpr (kPrePsi)
                     psv_velocity_exact<S, C, true>(g, ix, iz, shot, dxTxx, dzTzz, dxTxz, dzTxz, bu[r], bw[r],
                                                    nv[0][r], nv[1][r], ps, po, true, pr, psc, mp, pq[0][r],
-                                                   pq[1][r], pq[2][r], pq[3][r]);
+                                                   pq[1][r], pq[2][r], pq[3][r], xv, zv[r]);
                 else
                     psv_velocity_exact<S, C>(g, ix, iz, shot, dxTxx, dzTzz, dxTxz, dzTxz, bu[r], bw[r], nv[0][r],
                                              nv[1][r], ps, po, true, pr, psc, mp);
@@ -904,6 +947,9 @@ enum { SC_V = 0, SC_TX, SC_TZ, SC_PTX_X, SC_PV_X, SC_PTZ_Z, SC_PV_Z, SC_SH_N };
 template <class C> struct ShStressMat {
     const C *MUX, *MUZ;
 };
+template <class C> struct ShMat3 {
+    const C *BV, *MUX, *MUZ;
+};
 template <class S> struct ShPsi2 {
     S *x, *z; // (V_x, V_z) for stress, (Tx_x, Tz_z) for velocity
 };
@@ -911,19 +957,27 @@ template <class C> struct ShProf2 {
     Prof<C> x, z;
 };
 
-template <class S, int RZ, int SPB>
+// TO: over the tiles outside the work's interior ones (REGION_EDGE), new values
+// and C-PML memory written to the fields fo and po of the other buffer set
+template <class S, int RZ, int SPB, bool TO = false>
 __global__ __launch_bounds__(TX *BY) void k_sh_stress(ShFields<S> f, ShStressMat<typename Store<S>::C> m,
                                                       ShPsi2<S> ps, ShProf2<typename Store<S>::C> pr, Grid g,
                                                       Work w, Events ev, const float *__restrict__ scl,
-                                                      unsigned *__restrict__ amax) {
+                                                      unsigned *__restrict__ amax, ShFields<S> fo,
+                                                      ShPsi2<S> po) {
+    if (!TO) {
+        fo = f;
+        po = ps;
+    }
     using C = typename Store<S>::C;
     using ST = Store<S>;
+    constexpr bool kPrePsi = TO;
     constexpr int TZ = BY * RZ;
     constexpr int LW = TX + 2 * HALO;
     __shared__ C sV[(TZ + 2 * HALO) * LW];
 
     TileId t;
-    if (!map_tile<TZ>(w, t)) return;
+    if (!map_tile<TZ, TO ? REGION_EDGE : REGION_ALL>(w, t)) return;
     // a wavefront is one row of 64 threads, so threadIdx.y is wave-uniform
     const int tx = threadIdx.x, ty = __builtin_amdgcn_readfirstlane((int)threadIdx.y);
     const int x0 = t.x0, z0 = t.z0;
@@ -966,6 +1020,21 @@ __global__ __launch_bounds__(TX *BY) void k_sh_stress(ShFields<S> f, ShStressMat
         muz[r] = live ? Store<C>::ldb(rMUZ, vmat, so, 1.f) : C(0);
     }
 
+    // edge-only kernels: so are the profile entries of the thread's column and
+    // rows, once for all shots; read where they are used, each of the rows
+    // waited for two loads in turn
+    PmlCoef<C> xv[1], zv[kPrePsi ? RZ : 1][1];
+    if constexpr (kPrePsi) {
+        const bool inx = gx < nx && (gx < npml || gx >= nx - npml);
+        xv[0] = pml_coef(pr.x, gx, inx);
+#pragma unroll
+        for (int r = 0; r < RZ; r++) {
+            const int iz = z0 + lz0 + r;
+            const bool inz = iz < nz && ((iz < npml && g.top) || iz >= nz - npml);
+            zv[r][0] = pml_coef(pr.z, iz, inz);
+        }
+    }
+
     const int sh0 = t.group * SPB;
     for (int s = 0; s < SPB; s++) {
         const int shot = sh0 + s;
@@ -974,6 +1043,7 @@ __global__ __launch_bounds__(TX *BY) void k_sh_stress(ShFields<S> f, ShStressMat
         // buffer origin of this shot's arrays: element (row -HALO, column -HALO)
         const long org = (long)shot * g.sstride - (long)HALO * px - HALO;
         const BufRsrc bV = buf_rsrc(f.V + org), bX = buf_rsrc(f.Tx + org), bZ = buf_rsrc(f.Tz + org);
+        const BufRsrc oX = TO ? buf_rsrc(fo.Tx + org) : bX, oZ = TO ? buf_rsrc(fo.Tz + org) : bZ;
         Stage<S, TZ, true, true> rV;
         rV.loadb(bV, pxb, vcol, x0, z0, ty, sc_v);
         C vx[RZ], vz[RZ];
@@ -982,6 +1052,23 @@ __global__ __launch_bounds__(TX *BY) void k_sh_stress(ShFields<S> f, ShStressMat
             const unsigned so = (unsigned)(z0 + lz0 + r + HALO) * pxb;
             vx[r] = ST::ldb(bX, vcol, so, sc_x);
             vz[r] = ST::ldb(bZ, vcol, so, sc_z);
+        }
+        // this shot's C-PML memory variables, ahead of the barrier
+        C pq[2][kPrePsi ? RZ : 1];
+        if (kPrePsi && !interior) {
+#pragma unroll
+            for (int r = 0; r < RZ; r++) {
+                const int iz = z0 + lz0 + r;
+                pq[0][r] = pq[1][r] = C(0);
+                if (gx >= nx || iz >= nz || !(upd >> r & 1u)) continue;
+                if (gx < npml || gx >= nx - npml)
+                    pq[0][r] = ST::ld(ps.x, (long)shot * g.xpsi_stride + xpsi_idx(gx, iz, nx, npml),
+                                      ST::scaled ? scl[SC_PV_X] : 1.f);
+                const bool topcell = iz < npml && g.top;
+                if (topcell || iz >= nz - npml)
+                    pq[1][r] = ST::ld(ps.z, (long)shot * g.zpsi_stride + zpsi_idx(gx, iz, nx, nz, npml, topcell),
+                                      ST::scaled ? scl[SC_PV_Z] : 1.f);
+            }
         }
         if (s > 0) __syncthreads();
         rV.store(sV);
@@ -1017,9 +1104,9 @@ __global__ __launch_bounds__(TX *BY) void k_sh_stress(ShFields<S> f, ShStressMat
                 C tx_ = vx[r], tz_ = vz[r];
                 if (ix < npml || ix >= nx - npml) {
                     const long pi = (long)shot * g.xpsi_stride + xpsi_idx(ix, iz, nx, npml);
-                    C p = mad(pr.x.b[ix], ST::ld(ps.x, pi, sp_x), pr.x.c[ix] * dxV);
-                    ST::st(ps.x, pi, p, wp_x);
-                    tx_ = mad(mux[r], mad(dxV, pr.x.k[ix], p), tx_);
+                    C p = mad((kPrePsi ? xv[0].b : pr.x.b[ix]), kPrePsi ? pq[0][r] : ST::ld(ps.x, pi, sp_x), (kPrePsi ? xv[0].c : pr.x.c[ix]) * dxV);
+                    ST::st(po.x, pi, p, wp_x);
+                    tx_ = mad(mux[r], mad(dxV, (kPrePsi ? xv[0].k : pr.x.k[ix]), p), tx_);
                     if (ST::scaled) mp[0] = fmaxf(mp[0], fabsf((float)p));
                 } else {
                     tx_ = mad(mux[r], dxV, tx_);
@@ -1027,9 +1114,9 @@ __global__ __launch_bounds__(TX *BY) void k_sh_stress(ShFields<S> f, ShStressMat
                 const bool topcell = iz < npml && g.top;
                 if (topcell || iz >= nz - npml) {
                     const long pi = (long)shot * g.zpsi_stride + zpsi_idx(ix, iz, nx, nz, npml, topcell);
-                    C p = mad(pr.z.b[iz], ST::ld(ps.z, pi, sp_z), pr.z.c[iz] * dzV);
-                    ST::st(ps.z, pi, p, wp_z);
-                    tz_ = mad(muz[r], mad(dzV, pr.z.k[iz], p), tz_);
+                    C p = mad((kPrePsi ? zv[r][0].b : pr.z.b[iz]), kPrePsi ? pq[1][r] : ST::ld(ps.z, pi, sp_z), (kPrePsi ? zv[r][0].c : pr.z.c[iz]) * dzV);
+                    ST::st(po.z, pi, p, wp_z);
+                    tz_ = mad(muz[r], mad(dzV, (kPrePsi ? zv[r][0].k : pr.z.k[iz]), p), tz_);
                     if (ST::scaled) mp[1] = fmaxf(mp[1], fabsf((float)p));
                 } else {
                     tz_ = mad(muz[r], dzV, tz_);
@@ -1062,8 +1149,8 @@ __global__ __launch_bounds__(TX *BY) void k_sh_stress(ShFields<S> f, ShStressMat
             const int gz = z0 + lz0 + r;
             if (gx >= nx || gz >= nz) continue;
             const unsigned so = (unsigned)(gz + HALO) * pxb;
-            ST::stb(bX, vcol, so, vx[r], wi_x);
-            ST::stb(bZ, vcol, so, vz[r], wi_z);
+            ST::stb(oX, vcol, so, vx[r], wi_x);
+            ST::stb(oZ, vcol, so, vz[r], wi_z);
             if (ST::scaled && amax) { // the maxima are gathered on the step before a check
                 mx_x = fmaxf(mx_x, fabsf((float)vx[r]));
                 mx_z = fmaxf(mx_z, fabsf((float)vz[r]));
@@ -1082,20 +1169,26 @@ __global__ __launch_bounds__(TX *BY) void k_sh_stress(ShFields<S> f, ShStressMat
 // SH velocity pass (SH/fd/cu_fd.cu:172-273); Tz row 0 is first set to
 // -Tz row 1 (:226), so every read of Tz row 0 in this pass sees -Tz[1].
 // ===========================================================================
-template <class S, int RZ, int SPB>
+template <class S, int RZ, int SPB, bool TO = false>
 __global__ __launch_bounds__(TX *BY) void k_sh_velocity(ShFields<S> f, const typename Store<S>::C *__restrict__ BV,
                                                         ShPsi2<S> ps, ShProf2<typename Store<S>::C> pr, Grid g,
                                                         Work w, Events ev, const float *__restrict__ scl,
-                                                        unsigned *__restrict__ amax) {
+                                                        unsigned *__restrict__ amax, ShFields<S> fo,
+                                                        ShPsi2<S> po) {
+    if (!TO) {
+        fo = f;
+        po = ps;
+    }
     using C = typename Store<S>::C;
     using ST = Store<S>;
+    constexpr bool kPrePsi = TO;
     constexpr int TZ = BY * RZ;
     constexpr int LW = TX + 2 * HALO;
     __shared__ C sX[(TZ + 2 * HALO) * LW];
     __shared__ C sZ[(TZ + 2 * HALO) * LW];
 
     TileId t;
-    if (!map_tile<TZ>(w, t)) return;
+    if (!map_tile<TZ, TO ? REGION_EDGE : REGION_ALL>(w, t)) return;
     // a wavefront is one row of 64 threads, so threadIdx.y is wave-uniform
     const int tx = threadIdx.x, ty = __builtin_amdgcn_readfirstlane((int)threadIdx.y);
     const int x0 = t.x0, z0 = t.z0;
@@ -1138,6 +1231,21 @@ __global__ __launch_bounds__(TX *BY) void k_sh_velocity(ShFields<S> f, const typ
         bv[r] = live ? Store<C>::ldb(rBV, vmat, (unsigned)gz * pxm, 1.f) : C(0);
     }
 
+    // edge-only kernels: so are the profile entries of the thread's column and
+    // rows, once for all shots; read where they are used, each of the rows
+    // waited for two loads in turn
+    PmlCoef<C> xv[1], zv[kPrePsi ? RZ : 1][1];
+    if constexpr (kPrePsi) {
+        const bool inx = gx < nx && (gx < npml || gx >= nx - npml);
+        xv[0] = pml_coef(pr.x, gx, inx);
+#pragma unroll
+        for (int r = 0; r < RZ; r++) {
+            const int iz = z0 + lz0 + r;
+            const bool inz = iz < nz && ((iz < npml && g.top) || iz >= nz - npml);
+            zv[r][0] = pml_coef(pr.z, iz, inz);
+        }
+    }
+
     const int sh0 = t.group * SPB;
     for (int s = 0; s < SPB; s++) {
         const int shot = sh0 + s;
@@ -1148,7 +1256,8 @@ __global__ __launch_bounds__(TX *BY) void k_sh_velocity(ShFields<S> f, const typ
         const long base = (long)shot * g.sstride;
         // buffer origin of this shot's arrays: element (row -HALO, column -HALO)
         const long org = base - (long)HALO * px - HALO;
-        const BufRsrc bV = buf_rsrc(f.V + org), bX = buf_rsrc(f.Tx + org), bZ = buf_rsrc(f.Tz + org);
+        const BufRsrc bV = buf_rsrc(f.V + org), bX = buf_rsrc(fo.Tx + org), bZ = buf_rsrc(fo.Tz + org);
+        const BufRsrc oV = TO ? buf_rsrc(fo.V + org) : bV;
         Stage<S, TZ, false, true> rX;
         Stage<S, TZ, true, false> rZ;
         rX.loadb(bX, pxb, vcol, x0, z0, ty, sc_x);
@@ -1160,7 +1269,24 @@ __global__ __launch_bounds__(TX *BY) void k_sh_velocity(ShFields<S> f, const typ
         // HALO - z0) takes -Tz[row 1], and the tile owning row 0 writes it back
         const bool img = z0 - HALO <= 0 && z0 + TZ + HALO > 0;
         C img_v = C(0);
-        if (img && ty == 0 && img_open) img_v = -ST::ld(f.Tz, base + (long)px + gx, sc_z);
+        if (img && ty == 0 && img_open) img_v = -ST::ld(fo.Tz, base + (long)px + gx, sc_z);
+        // this shot's C-PML memory variables, ahead of the barrier
+        C pq[2][kPrePsi ? RZ : 1];
+        if (kPrePsi && !interior) {
+#pragma unroll
+            for (int r = 0; r < RZ; r++) {
+                const int iz = z0 + lz0 + r;
+                pq[0][r] = pq[1][r] = C(0);
+                if (gx >= nx || iz >= nz || !(upd >> r & 1u)) continue;
+                if (gx < npml || gx >= nx - npml)
+                    pq[0][r] = ST::ld(ps.x, (long)shot * g.xpsi_stride + xpsi_idx(gx, iz, nx, npml),
+                                      ST::scaled ? scl[SC_PTX_X] : 1.f);
+                const bool topcell = iz < npml && g.top;
+                if (topcell || iz >= nz - npml)
+                    pq[1][r] = ST::ld(ps.z, (long)shot * g.zpsi_stride + zpsi_idx(gx, iz, nx, nz, npml, topcell),
+                                      ST::scaled ? scl[SC_PTZ_Z] : 1.f);
+            }
+        }
         if (s > 0) __syncthreads();
         rX.store(sX);
         rZ.store(sZ);
@@ -1168,7 +1294,7 @@ __global__ __launch_bounds__(TX *BY) void k_sh_velocity(ShFields<S> f, const typ
             __syncthreads();
             if (ty == 0 && img_open) {
                 sZ[(HALO - z0) * LW + tx + HALO] = img_v;
-                if (z0 == 0 && gx < nx) ST::st(f.Tz, base + gx, img_v, inv_pow2(sc_z));
+                if (z0 == 0 && gx < nx) ST::st(fo.Tz, base + gx, img_v, inv_pow2(sc_z));
             }
         }
         __syncthreads();
@@ -1221,9 +1347,9 @@ __global__ __launch_bounds__(TX *BY) void k_sh_velocity(ShFields<S> f, const typ
                 C v = nv[0][r];
                 if (ix < npml || ix >= nx - npml) {
                     const long pi = (long)shot * g.xpsi_stride + xpsi_idx(ix, iz, nx, npml);
-                    C p = mad(pr.x.b[ix], ST::ld(ps.x, pi, sp_x), pr.x.c[ix] * Tx_x);
-                    ST::st(ps.x, pi, p, wp_x);
-                    v = mad(bv[r], mad(Tx_x, pr.x.k[ix], p), v);
+                    C p = mad((kPrePsi ? xv[0].b : pr.x.b[ix]), kPrePsi ? pq[0][r] : ST::ld(ps.x, pi, sp_x), (kPrePsi ? xv[0].c : pr.x.c[ix]) * Tx_x);
+                    ST::st(po.x, pi, p, wp_x);
+                    v = mad(bv[r], mad(Tx_x, (kPrePsi ? xv[0].k : pr.x.k[ix]), p), v);
                     if (ST::scaled) mp[0] = fmaxf(mp[0], fabsf((float)p));
                 } else {
                     v = mad(bv[r], Tx_x, v);
@@ -1231,9 +1357,9 @@ __global__ __launch_bounds__(TX *BY) void k_sh_velocity(ShFields<S> f, const typ
                 const bool topcell = iz < npml && g.top;
                 if (topcell || iz >= nz - npml) {
                     const long pi = (long)shot * g.zpsi_stride + zpsi_idx(ix, iz, nx, nz, npml, topcell);
-                    C p = mad(pr.z.b[iz], ST::ld(ps.z, pi, sp_z), pr.z.c[iz] * Tz_z);
-                    ST::st(ps.z, pi, p, wp_z);
-                    v = mad(bv[r], mad(Tz_z, pr.z.k[iz], p), v);
+                    C p = mad((kPrePsi ? zv[r][0].b : pr.z.b[iz]), kPrePsi ? pq[1][r] : ST::ld(ps.z, pi, sp_z), (kPrePsi ? zv[r][0].c : pr.z.c[iz]) * Tz_z);
+                    ST::st(po.z, pi, p, wp_z);
+                    v = mad(bv[r], mad(Tz_z, (kPrePsi ? zv[r][0].k : pr.z.k[iz]), p), v);
                     if (ST::scaled) mp[1] = fmaxf(mp[1], fabsf((float)p));
                 } else {
                     v = mad(bv[r], Tz_z, v);
@@ -1245,10 +1371,10 @@ __global__ __launch_bounds__(TX *BY) void k_sh_velocity(ShFields<S> f, const typ
         for (int r = 0; r < RZ; r++) {
             const int gz = z0 + lz0 + r;
             if (gx >= nx || gz >= nz) continue;
-            ST::stb(bV, vcol, (unsigned)(gz + HALO) * pxb, nv[0][r], wi_v);
+            ST::stb(oV, vcol, (unsigned)(gz + HALO) * pxb, nv[0][r], wi_v);
             if (ST::scaled && amax) mx_v = fmaxf(mx_v, fabsf((float)nv[0][r]));
         }
-        if (ev.clock) fused_record<C, RZ, 1>(ev, it, t.tile * g.nshots + shot, sX, sX, nv, lz0, ev.src[shot].t0, w, x0, z0);
+        if (ev.clock) fused_record<C, RZ, 1, TO>(ev, it, t.tile * g.nshots + shot, sX, sX, nv, lz0, ev.src[shot].t0, w, x0, z0);
     }
     if (ST::scaled) {
         amax_update(amax, SC_V, mx_v);

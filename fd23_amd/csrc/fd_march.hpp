@@ -418,17 +418,9 @@ __device__ __forceinline__ void march_item(const PsvFields<S> &fa, const PsvFiel
     }
 }
 
-
-template <class S, int MW>
-__global__ __launch_bounds__(MW / NC, 2) void k_psv_march(PsvFields<S> fa, PsvFields<S> fb, PsvMat5<float> m, Grid g,
-                                                          MarchWork w, FusedEvents ev, const float *__restrict__ sa,
-                                                          const float *__restrict__ scl,
-                                                          unsigned *__restrict__ amax) {
-    __shared__ MarchLds<MW> l;
-    const int qd = gridDim.x >> 3; // grid padded to a multiple of 8
-    const int L = (int)(blockIdx.x & 7) * qd + (int)(blockIdx.x >> 3);
-    if (L >= w.nwork) return;
-    MarchItem q;
+// work item L; whether a source or receiver is in it
+template <int MW>
+__device__ __forceinline__ bool march_find(const Grid &g, const MarchWork &w, const FusedEvents &ev, int L, MarchItem &q) {
     const int rest = L / g.nshots, seg = rest / w.nstrip;
     q.shot = L % g.nshots;
     q.strip = rest % w.nstrip;
@@ -466,8 +458,22 @@ __global__ __launch_bounds__(MW / NC, 2) void k_psv_march(PsvFields<S> fa, PsvFi
         }
     }
     const bool taps = (q.onA || q.onB) && q.trow1 >= q.za - kMarchReach && q.trow0 < q.zb + kMarchReach;
+    return taps || q.nextA != kNoRow || q.nextB != kNoRow;
+}
+
+template <class S, int MW>
+__global__ __launch_bounds__(MW / NC, 2) void k_psv_march(PsvFields<S> fa, PsvFields<S> fb, PsvMat5<float> m, Grid g,
+                                                          MarchWork w, FusedEvents ev, const float *__restrict__ sa,
+                                                          const float *__restrict__ scl,
+                                                          unsigned *__restrict__ amax) {
+    __shared__ MarchLds<MW> l;
+    const int qd = gridDim.x >> 3; // grid padded to a multiple of 8
+    const int L = (int)(blockIdx.x & 7) * qd + (int)(blockIdx.x >> 3);
+    if (L >= w.nwork) return;
+    MarchItem q;
+    const bool checked = march_find<MW>(g, w, ev, L, q);
     // amax is null on steps that no scale check follows
-    if (taps || q.nextA != kNoRow || q.nextB != kNoRow)
+    if (checked)
         march_item<S, MW, true, Store<S>::scaled>(fa, fb, m, g, w, ev, sa, scl, amax, q, l);
     else if (Store<S>::scaled && amax)
         march_item<S, MW, false, Store<S>::scaled>(fa, fb, m, g, w, ev, sa, scl, amax, q, l);
@@ -480,5 +486,9 @@ template <class S>
 void march_launch(hipStream_t stream, const PsvFields<S> &fa, const PsvFields<S> &fb, const PsvMat5<float> &m,
                   const Grid &g, const MarchWork &w, const FusedEvents &ev, const float *sa, const float *scl,
                   unsigned *amax);
+
+// SH (fd_sh_march.hpp), FP32
+void sh_march_launch(hipStream_t stream, const ShFields<float> &fa, const ShFields<float> &fb, const ShMat3<float> &m,
+                     const Grid &g, const MarchWork &w, const FusedEvents &ev);
 
 } // namespace fd23

@@ -280,16 +280,17 @@ int fd23_num_tiles(void);
  * tile-parallel step, FP32/FP64 storage only; or block_rows -1: the
  * marching step, seg_rows = steps per launch, the interior by a kernel
  * that marches down strips and the frame around it by two-pass kernels of
- * rz rows per thread, FP32/FP16/BF16 storage; 0 for tiled kinds);
+ * rz rows per thread, P-SV with FP32/FP16/BF16 storage and SH with FP32;
+ * 0 for tiled kinds);
  * FD23_TILE_BLOCK, the SH block step (seg_rows = K steps per launch over
  * regions of 64 columns x block_rows rows, rz rows per thread, each
  * region a tile plus a 7*K-cell halo that the launch recomputes, over two
- * buffer sets).  The fused step applies to fd23_run of P-SV contexts
- * without a box, the block step to fd23_run of SH contexts with FP32/FP64
+ * buffer sets).  The fused step applies to fd23_run of P-SV contexts (the
+ * marching step's of SH ones too) without a box, the block step to fd23_run of SH contexts with FP32/FP64
  * storage, both without a first-arrival window; the staged entry points,
  * the box and the window run the tiled kernels (tile 0's shape, or for the
- * marching step its frame's; so do contexts with idle slots or FP64
- * storage set to the marching step, and grids with no interior).  No
+ * marching step its frame's; so do contexts with idle slots or with
+ * other storage set to the marching step, and grids with no interior).  No
  * reference counterpart: the reference launches two kernels per step
  * (SH/main.cpp:93-141).                                                 */
 enum { FD23_TILE_TILED = 0, FD23_TILE_FUSED = 1, FD23_TILE_BLOCK = 2 };

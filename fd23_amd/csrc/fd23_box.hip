@@ -109,133 +109,142 @@ __device__ __forceinline__ int ring_depth(int i, int j, int bx, int bz) {
     return min(min(i, j), min(bx - 1 - i, bz - 1 - j));
 }
 
-// add (a = r + s) or sub (r = a - s) over one ring for fields [f0, f1)
+// the drive of field fi at box cell (i, j) at time t; stab: file drive, this
+// step's converted frames
 template <class C>
-__global__ void k_box_ring(BoxPar p, C *const *glob, C *resid, int f0, int f1, bool add, const int *clock, int k,
-                           int it_arg, double toff, const double *stab) {
+__device__ __forceinline__ C ring_drive(const BoxPar &p, int fi, int i, int j, double t, const double *stab) {
+    if (stab) return C(stab[((long)fi * p.bz + j) * p.bx + i]);
+    double ox, oz;
+    offsets(fi, ox, oz);
+    return C(drive(p, fi, p.x0 + i + ox, p.z0 + j + oz, t));
+}
+
+// add ring of the velocities (a = r + s) at the start of a chunk
+template <class C>
+__global__ void k_box_add(BoxPar p, C *const *glob, const C *resid, const int *clock, int k, int it_arg,
+                          const double *stab) {
     const int it = clock ? clock[0] + k : it_arg;
-    const double t = (it + toff) * p.dt;
+    const double t = (it + 0.5) * p.dt;
     const long nb = (long)p.bx * p.bz;
-    const int dlo = add ? 4 : 0, dhi = add ? 7 : 3;
-    const long total = nb * (f1 - f0) * p.nshots;
+    const long total = nb * 2 * p.nshots;
     for (long e = blockIdx.x * (long)blockDim.x + threadIdx.x; e < total; e += (long)gridDim.x * blockDim.x) {
         const long cell = e % nb;
-        const int fi = f0 + (int)((e / nb) % (f1 - f0));
-        const int shot = (int)(e / (nb * (f1 - f0)));
+        const int fi = (int)((e / nb) % 2);
+        const int shot = (int)(e / (nb * 2));
         const int i = (int)(cell % p.bx), j = (int)(cell / p.bx);
         const int d = ring_depth(i, j, p.bx, p.bz);
-        if (d < dlo || d > dhi) continue;
-        C s;
-        if (stab) { // file drive: this step's converted frames
-            s = C(stab[(long)fi * nb + cell]);
-        } else {
-            double ox, oz;
-            offsets(fi, ox, oz);
-            s = C(drive(p, fi, p.x0 + i + ox, p.z0 + j + oz, t));
-        }
-        C *a = glob[fi] + (long)shot * p.sstride + (long)(p.z0 + j) * p.px + (p.x0 + i);
-        C *r = resid + ((long)shot * 5 + fi) * nb + cell;
-        if (add)
-            *a = *r + s;
-        else
-            *r = *a - s;
+        if (d < 4 || d > 7) continue;
+        glob[fi][(long)shot * p.sstride + (long)(p.z0 + j) * p.px + (p.x0 + i)] =
+            resid[((long)shot * 5 + fi) * nb + cell] + ring_drive<C>(p, fi, i, j, t, stab);
     }
 }
 
-template <class C> __device__ __forceinline__ C rat(const C *f, int bx, int bz, int i, int j) {
-    return (i < 0 || i >= bx || j < 0 || j >= bz) ? C(0) : f[(long)j * bx + i];
-}
+// Residual grid passes (PSV/psv_clean_double/fd/cu_fd.cu:93-207): full order,
+// zero outside the box, homogeneous (lam, mu, b) already scaled.  A pass is
+// one kernel with the rings around it: the sub ring of the fields it
+// differentiates, staged with their halo (a workgroup computes the ring's
+// values of its halo for itself, none writes what another reads), and the add
+// ring of the fields it updates.  The step of a 640 x 401 FP64 grid is a chain
+// of dependent launches (38 us); as three kernels a pass, six of its eight
+// were rings and residual passes of 3.7 and 4.4 us each.
+constexpr int KX = 32, KZ = 8, KH = 4, KW = KX + 2 * KH, KN = KW * (KZ + 2 * KH);
 
-// residual grid passes (PSV/psv_clean_double/fd/cu_fd.cu:93-207): full
-// order, zero outside the box, homogeneous (lam, mu, b) already scaled
+struct BoxTile {
+    int i0, j0, shot;
+};
+__device__ __forceinline__ BoxTile box_tile(const BoxPar &p) {
+    const int ntx = (p.bx + KX - 1) / KX, ntz = (p.bz + KZ - 1) / KZ;
+    const int t = (int)blockIdx.x % (ntx * ntz);
+    return BoxTile{t % ntx * KX, t / ntx * KZ, (int)blockIdx.x / (ntx * ntz)};
+}
+// field fi with its halo: the residual grid's values, in the sub ring
+// (depth 0..3) a - s, which the owner stores; zero outside the box
 template <class C>
-__global__ void k_box_stress_r(BoxPar p, C *resid, const C *LAMg, const C *MUg, const C *MUAg) {
+__device__ __forceinline__ void stage_ring(const BoxPar &p, const BoxTile &b, int fi, const C *glob, C *resid, double t,
+                                           const double *stab, C *lds) {
     const long nb = (long)p.bx * p.bz;
+    C *r = resid + ((long)b.shot * 5 + fi) * nb;
+    for (int e = (int)threadIdx.x; e < KN; e += KX * KZ) {
+        const int li = e % KW - KH, lj = e / KW - KH, i = b.i0 + li, j = b.j0 + lj;
+        C v = C(0);
+        if (i >= 0 && i < p.bx && j >= 0 && j < p.bz) {
+            const long cell = (long)j * p.bx + i;
+            if (ring_depth(i, j, p.bx, p.bz) <= 3) {
+                v = glob[(long)b.shot * p.sstride + (long)(p.z0 + j) * p.px + (p.x0 + i)] -
+                    ring_drive<C>(p, fi, i, j, t, stab);
+                if (li >= 0 && li < KX && lj >= 0 && lj < KZ) r[cell] = v;
+            } else {
+                v = r[cell];
+            }
+        }
+        lds[e] = v;
+    }
+}
+template <class C>
+__global__ __launch_bounds__(KX *KZ) void k_box_stress_r(BoxPar p, C *const *glob, C *resid, const C *LAMg,
+                                                         const C *MUg, const C *MUAg, const int *clock, int k,
+                                                         int it_arg, const double *stab) {
+    __shared__ C sU[KN], sW[KN];
+    const int it = clock ? clock[0] + k : it_arg;
+    const BoxTile b = box_tile(p);
+    stage_ring(p, b, 0, glob[0], resid, (it + 0.5) * p.dt, stab, sU);
+    stage_ring(p, b, 1, glob[1], resid, (it + 0.5) * p.dt, stab, sW);
+    __syncthreads();
+    const int li = (int)threadIdx.x % KX, lj = (int)threadIdx.x / KX, i = b.i0 + li, j = b.j0 + lj;
+    if (i >= p.bx || j >= p.bz) return;
+    const int o = (lj + KH) * KW + li + KH;
     const C c0 = C(1225. / 1024.), c1 = C(245. / 3072.), c2 = C(49. / 5120.), c3 = C(5. / 7168.);
-    for (long e = blockIdx.x * (long)blockDim.x + threadIdx.x; e < nb * p.nshots; e += (long)gridDim.x * blockDim.x) {
-        const int shot = (int)(e / nb);
-        const long cell = e % nb;
-        const int i = (int)(cell % p.bx), j = (int)(cell / p.bx);
-        C *R = resid + (long)shot * 5 * nb;
-        const C *U = R, *W = R + nb;
-        C *Txx = R + 2 * nb, *Tzz = R + 3 * nb, *Txz = R + 4 * nb;
-        const int bx = p.bx, bz = p.bz;
-        auto dmx = [&](const C *f) {
-            C r = c0 * (rat(f, bx, bz, i, j) - rat(f, bx, bz, i - 1, j));
-            r = mad(-c1, rat(f, bx, bz, i + 1, j) - rat(f, bx, bz, i - 2, j), r);
-            r = mad(c2, rat(f, bx, bz, i + 2, j) - rat(f, bx, bz, i - 3, j), r);
-            return mad(-c3, rat(f, bx, bz, i + 3, j) - rat(f, bx, bz, i - 4, j), r);
-        };
-        auto dmz = [&](const C *f) {
-            C r = c0 * (rat(f, bx, bz, i, j) - rat(f, bx, bz, i, j - 1));
-            r = mad(-c1, rat(f, bx, bz, i, j + 1) - rat(f, bx, bz, i, j - 2), r);
-            r = mad(c2, rat(f, bx, bz, i, j + 2) - rat(f, bx, bz, i, j - 3), r);
-            return mad(-c3, rat(f, bx, bz, i, j + 3) - rat(f, bx, bz, i, j - 4), r);
-        };
-        auto dpx = [&](const C *f) {
-            C r = c0 * (rat(f, bx, bz, i + 1, j) - rat(f, bx, bz, i, j));
-            r = mad(-c1, rat(f, bx, bz, i + 2, j) - rat(f, bx, bz, i - 1, j), r);
-            r = mad(c2, rat(f, bx, bz, i + 3, j) - rat(f, bx, bz, i - 2, j), r);
-            return mad(-c3, rat(f, bx, bz, i + 4, j) - rat(f, bx, bz, i - 3, j), r);
-        };
-        auto dpz = [&](const C *f) {
-            C r = c0 * (rat(f, bx, bz, i, j + 1) - rat(f, bx, bz, i, j));
-            r = mad(-c1, rat(f, bx, bz, i, j + 2) - rat(f, bx, bz, i, j - 1), r);
-            r = mad(c2, rat(f, bx, bz, i, j + 3) - rat(f, bx, bz, i, j - 2), r);
-            return mad(-c3, rat(f, bx, bz, i, j + 4) - rat(f, bx, bz, i, j - 3), r);
-        };
-        const C ux = dmx(U), uz = dmz(U), wx = dpx(W), wz = dpz(W);
-        const long qg = (long)(p.z0 + j) * p.px + p.x0 + i;
-        const C lam = LAMg[qg], mu = MUg[qg], mua = MUAg[qg];
-        const C gam = lam + C(2.0) * mu;
-        const long q = (long)j * bx + i;
-        Txx[q] = Txx[q] + (gam * ux + lam * wz);
-        Tzz[q] = Tzz[q] + (lam * ux + gam * wz);
-        Txz[q] = Txz[q] + mua * (wx + uz);
+    const C ux = dm(&sU[o], 1, c0, c1, c2, c3), uz = dm(&sU[o], KW, c0, c1, c2, c3);
+    const C wx = dp(&sW[o], 1, c0, c1, c2, c3), wz = dp(&sW[o], KW, c0, c1, c2, c3);
+    const long qg = (long)(p.z0 + j) * p.px + p.x0 + i;
+    const C lam = LAMg[qg], mu = MUg[qg], mua = MUAg[qg];
+    const C gam = lam + C(2.0) * mu;
+    const long nb = (long)p.bx * p.bz, q = (long)j * p.bx + i;
+    C *T = resid + ((long)b.shot * 5 + 2) * nb + q;
+    C v[3];
+    v[0] = T[0] + (gam * ux + lam * wz);
+    v[1] = T[nb] + (lam * ux + gam * wz);
+    v[2] = T[2 * nb] + mua * (wx + uz);
+    const int d = ring_depth(i, j, p.bx, p.bz);
+#pragma unroll
+    for (int f = 0; f < 3; f++) {
+        T[f * nb] = v[f];
+        if (d >= 4 && d <= 7)
+            glob[2 + f][(long)b.shot * p.sstride + qg] = v[f] + ring_drive<C>(p, 2 + f, i, j, (it + 1.0) * p.dt, stab);
     }
 }
 
-template <class C> __global__ void k_box_velocity_r(BoxPar p, C *resid, const C *BUg, const C *BWg) {
-    const long nb = (long)p.bx * p.bz;
+// add: with the next step's add ring of the velocities
+template <class C>
+__global__ __launch_bounds__(KX *KZ) void k_box_velocity_r(BoxPar p, C *const *glob, C *resid, const C *BUg,
+                                                           const C *BWg, const int *clock, int k, int it_arg,
+                                                           const double *stab, bool add) {
+    __shared__ C sXX[KN], sZZ[KN], sXZ[KN];
+    const int it = clock ? clock[0] + k : it_arg;
+    const BoxTile b = box_tile(p);
+    stage_ring(p, b, 2, glob[2], resid, (it + 1.0) * p.dt, stab, sXX);
+    stage_ring(p, b, 3, glob[3], resid, (it + 1.0) * p.dt, stab, sZZ);
+    stage_ring(p, b, 4, glob[4], resid, (it + 1.0) * p.dt, stab, sXZ);
+    __syncthreads();
+    const int li = (int)threadIdx.x % KX, lj = (int)threadIdx.x / KX, i = b.i0 + li, j = b.j0 + lj;
+    if (i >= p.bx || j >= p.bz) return;
+    const int o = (lj + KH) * KW + li + KH;
     const C c0 = C(1225. / 1024.), c1 = C(245. / 3072.), c2 = C(49. / 5120.), c3 = C(5. / 7168.);
-    for (long e = blockIdx.x * (long)blockDim.x + threadIdx.x; e < nb * p.nshots; e += (long)gridDim.x * blockDim.x) {
-        const int shot = (int)(e / nb);
-        const long cell = e % nb;
-        const int i = (int)(cell % p.bx), j = (int)(cell / p.bx);
-        C *R = resid + (long)shot * 5 * nb;
-        C *U = R, *W = R + nb;
-        const C *Txx = R + 2 * nb, *Tzz = R + 3 * nb, *Txz = R + 4 * nb;
-        const int bx = p.bx, bz = p.bz;
-        auto dmx = [&](const C *f) {
-            C r = c0 * (rat(f, bx, bz, i, j) - rat(f, bx, bz, i - 1, j));
-            r = mad(-c1, rat(f, bx, bz, i + 1, j) - rat(f, bx, bz, i - 2, j), r);
-            r = mad(c2, rat(f, bx, bz, i + 2, j) - rat(f, bx, bz, i - 3, j), r);
-            return mad(-c3, rat(f, bx, bz, i + 3, j) - rat(f, bx, bz, i - 4, j), r);
-        };
-        auto dmz = [&](const C *f) {
-            C r = c0 * (rat(f, bx, bz, i, j) - rat(f, bx, bz, i, j - 1));
-            r = mad(-c1, rat(f, bx, bz, i, j + 1) - rat(f, bx, bz, i, j - 2), r);
-            r = mad(c2, rat(f, bx, bz, i, j + 2) - rat(f, bx, bz, i, j - 3), r);
-            return mad(-c3, rat(f, bx, bz, i, j + 3) - rat(f, bx, bz, i, j - 4), r);
-        };
-        auto dpx = [&](const C *f) {
-            C r = c0 * (rat(f, bx, bz, i + 1, j) - rat(f, bx, bz, i, j));
-            r = mad(-c1, rat(f, bx, bz, i + 2, j) - rat(f, bx, bz, i - 1, j), r);
-            r = mad(c2, rat(f, bx, bz, i + 3, j) - rat(f, bx, bz, i - 2, j), r);
-            return mad(-c3, rat(f, bx, bz, i + 4, j) - rat(f, bx, bz, i - 3, j), r);
-        };
-        auto dpz = [&](const C *f) {
-            C r = c0 * (rat(f, bx, bz, i, j + 1) - rat(f, bx, bz, i, j));
-            r = mad(-c1, rat(f, bx, bz, i, j + 2) - rat(f, bx, bz, i, j - 1), r);
-            r = mad(c2, rat(f, bx, bz, i, j + 3) - rat(f, bx, bz, i, j - 2), r);
-            return mad(-c3, rat(f, bx, bz, i, j + 4) - rat(f, bx, bz, i, j - 3), r);
-        };
-        const C dxTxx = dpx(Txx), dzTzz = dmz(Tzz), dxTxz = dmx(Txz), dzTxz = dpz(Txz);
-        const long qg = (long)(p.z0 + j) * p.px + p.x0 + i;
-        const C bu = BUg[qg], bw = BWg[qg];
-        const long q = (long)j * bx + i;
-        U[q] = U[q] + bu * (dxTxx + dzTxz);
-        W[q] = W[q] + bw * (dxTxz + dzTzz);
+    const C dxTxx = dp(&sXX[o], 1, c0, c1, c2, c3), dzTzz = dm(&sZZ[o], KW, c0, c1, c2, c3);
+    const C dxTxz = dm(&sXZ[o], 1, c0, c1, c2, c3), dzTxz = dp(&sXZ[o], KW, c0, c1, c2, c3);
+    const long qg = (long)(p.z0 + j) * p.px + p.x0 + i;
+    const C bu = BUg[qg], bw = BWg[qg];
+    const long nb = (long)p.bx * p.bz, q = (long)j * p.bx + i;
+    C *V = resid + (long)b.shot * 5 * nb + q;
+    C v[2];
+    v[0] = V[0] + bu * (dxTxx + dzTxz);
+    v[1] = V[nb] + bw * (dxTxz + dzTzz);
+    const int d = ring_depth(i, j, p.bx, p.bz);
+#pragma unroll
+    for (int f = 0; f < 2; f++) {
+        V[f * nb] = v[f];
+        if (add && d >= 4 && d <= 7)
+            glob[f][(long)b.shot * p.sstride + qg] = v[f] + ring_drive<C>(p, f, i, j, (it + 1 + 0.5) * p.dt, stab);
     }
 }
 
@@ -350,13 +359,29 @@ struct Box {
 
 Box *get(fd23_ctx *c) { return (Box *)fd23_ctx_box(c); }
 
-template <class C> int launch_ring(fd23_ctx *c, Box *bx, int f0, int f1, bool add, int k, double toff) {
-    const long total = (long)bx->p.bx * bx->p.bz * (f1 - f0) * bx->p.nshots;
+// one workgroup per tile and shot
+dim3 box_grid(const BoxPar &p) {
+    return dim3((unsigned)((p.bx + KX - 1) / KX * ((p.bz + KZ - 1) / KZ) * p.nshots));
+}
+template <class C> int launch_add(fd23_ctx *c, Box *bx, int k) {
+    const long total = (long)bx->p.bx * bx->p.bz * 2 * bx->p.nshots;
     const int nblk = (int)std::min<long>((total + 255) / 256, 2048);
-    hipLaunchKernelGGL((k_box_ring<C>), dim3(nblk), dim3(256), 0, fd23_ctx_stream(c), bx->p, (C *const *)bx->gtab,
-                       (C *)bx->resid, f0, f1, add, k >= 0 ? fd23_ctx_clock(c) : nullptr, k < 0 ? 0 : k,
-                       bx->staged_it, toff, bx->sdrive);
+    hipLaunchKernelGGL((k_box_add<C>), dim3(nblk), dim3(256), 0, fd23_ctx_stream(c), bx->p, (C *const *)bx->gtab,
+                       (const C *)bx->resid, k >= 0 ? fd23_ctx_clock(c) : nullptr, k < 0 ? 0 : k, bx->staged_it,
+                       bx->sdrive);
     return FD23_OK;
+}
+template <class C> void launch_stress_r(fd23_ctx *c, Box *b, int k) {
+    hipLaunchKernelGGL((k_box_stress_r<C>), box_grid(b->p), dim3(KX * KZ), 0, fd23_ctx_stream(c), b->p,
+                       (C *const *)b->gtab, (C *)b->resid, (const C *)fd23_ctx_material(c, 4),
+                       (const C *)fd23_ctx_material(c, 2), (const C *)fd23_ctx_material(c, 3),
+                       k >= 0 ? fd23_ctx_clock(c) : nullptr, k < 0 ? 0 : k, b->staged_it, b->sdrive);
+}
+template <class C> void launch_velocity_r(fd23_ctx *c, Box *b, int k, bool add) {
+    hipLaunchKernelGGL((k_box_velocity_r<C>), box_grid(b->p), dim3(KX * KZ), 0, fd23_ctx_stream(c), b->p,
+                       (C *const *)b->gtab, (C *)b->resid, (const C *)fd23_ctx_material(c, 0),
+                       (const C *)fd23_ctx_material(c, 1), k >= 0 ? fd23_ctx_clock(c) : nullptr, k < 0 ? 0 : k,
+                       b->staged_it, b->sdrive, add);
 }
 
 // the file drive of this step, ahead of its first ring
@@ -389,7 +414,8 @@ int fd23_box_launch_pre_stress(fd23_ctx *c, int k) {
         else
             launch_frames_drive<float>(c, b, k);
     }
-    return b->f64 ? launch_ring<double>(c, b, 0, 2, true, k, 0.5) : launch_ring<float>(c, b, 0, 2, true, k, 0.5);
+    if (k > 0 && !b->frames) return FD23_OK; // the step before has added them
+    return b->f64 ? launch_add<double>(c, b, k) : launch_add<float>(c, b, k);
 }
 
 // frames a run of steps [it0, it0+nt) needs: it0+nt+1
@@ -409,40 +435,19 @@ int fd23_box_check_run(fd23_ctx *c, int it0, int nt) {
 int fd23_box_launch_post_stress(fd23_ctx *c, int k) {
     Box *b = get(c);
     if (!b) return FD23_OK;
-    const long nb = (long)b->p.bx * b->p.bz * b->p.nshots;
-    const int nblk = (int)std::min<long>((nb + 255) / 256, 2048);
-    if (b->f64) {
-        launch_ring<double>(c, b, 0, 2, false, k, 0.5);
-        hipLaunchKernelGGL((k_box_stress_r<double>), dim3(nblk), dim3(256), 0, fd23_ctx_stream(c), b->p,
-                           (double *)b->resid, (const double *)fd23_ctx_material(c, 4),
-                           (const double *)fd23_ctx_material(c, 2), (const double *)fd23_ctx_material(c, 3));
-        launch_ring<double>(c, b, 2, 5, true, k, 1.0);
-    } else {
-        launch_ring<float>(c, b, 0, 2, false, k, 0.5);
-        hipLaunchKernelGGL((k_box_stress_r<float>), dim3(nblk), dim3(256), 0, fd23_ctx_stream(c), b->p,
-                           (float *)b->resid, (const float *)fd23_ctx_material(c, 4),
-                           (const float *)fd23_ctx_material(c, 2), (const float *)fd23_ctx_material(c, 3));
-        launch_ring<float>(c, b, 2, 5, true, k, 1.0);
-    }
+    if (b->f64) launch_stress_r<double>(c, b, k);
+    else launch_stress_r<float>(c, b, k);
     return FD23_OK;
 }
 
-int fd23_box_launch_post_velocity(fd23_ctx *c, int k) {
+// more: the chunk goes on with step k+1, whose pre_stress adds nothing then
+// (the drive of the source frames is converted only at that step's start)
+int fd23_box_launch_post_velocity(fd23_ctx *c, int k, bool more) {
     Box *b = get(c);
     if (!b) return FD23_OK;
-    const long nb = (long)b->p.bx * b->p.bz * b->p.nshots;
-    const int nblk = (int)std::min<long>((nb + 255) / 256, 2048);
-    if (b->f64) {
-        launch_ring<double>(c, b, 2, 5, false, k, 1.0);
-        hipLaunchKernelGGL((k_box_velocity_r<double>), dim3(nblk), dim3(256), 0, fd23_ctx_stream(c), b->p,
-                           (double *)b->resid, (const double *)fd23_ctx_material(c, 0),
-                           (const double *)fd23_ctx_material(c, 1));
-    } else {
-        launch_ring<float>(c, b, 2, 5, false, k, 1.0);
-        hipLaunchKernelGGL((k_box_velocity_r<float>), dim3(nblk), dim3(256), 0, fd23_ctx_stream(c), b->p,
-                           (float *)b->resid, (const float *)fd23_ctx_material(c, 0),
-                           (const float *)fd23_ctx_material(c, 1));
-    }
+    const bool add = more && !b->frames;
+    if (b->f64) launch_velocity_r<double>(c, b, k, add);
+    else launch_velocity_r<float>(c, b, k, add);
     if (k < 0) b->staged_it++;
     return FD23_OK;
 }

@@ -277,7 +277,7 @@ struct fd23_ctx {
 // implemented in fd23_box.hip
 int fd23_box_launch_pre_stress(fd23_ctx *c, int k);
 int fd23_box_launch_post_stress(fd23_ctx *c, int k);
-int fd23_box_launch_post_velocity(fd23_ctx *c, int k);
+int fd23_box_launch_post_velocity(fd23_ctx *c, int k, bool more);
 void fd23_box_free(fd23_ctx *c);
 void fd23_box_set_step(fd23_ctx *c, int it);
 int fd23_box_check_run(fd23_ctx *c, int it0, int nt);
@@ -1950,7 +1950,7 @@ extern "C" int fd23_step_velocity(fd23_ctx *c) {
         enqueue_commit(c, false);
         if (++c->staged_steps % kScaleEvery == 0) enqueue_scale_control(c);
     }
-    if (c->box && (r = fd23_box_launch_post_velocity(c, -1))) return r;
+    if (c->box && (r = fd23_box_launch_post_velocity(c, -1, false))) return r;
     return check_launch();
 }
 extern "C" int fd23_record(fd23_ctx *c, int it, int itrecord) {
@@ -1962,8 +1962,9 @@ extern "C" int fd23_record(fd23_ctx *c, int it, int itrecord) {
     return check_launch();
 }
 
-// step k of a chunk: the step index is clock[0] + k on the device
-static int enqueue_step(fd23_ctx *c, int k, int itrecord) {
+// step k of a chunk, `left` steps remaining with it: the step index is
+// clock[0] + k on the device
+static int enqueue_step(fd23_ctx *c, int k, int left, int itrecord) {
     int r;
     const Events ev = make_events(c, k, itrecord);
     // a scale check ends every kScaleEvery-th step of a chunk, so the passes
@@ -1985,7 +1986,7 @@ static int enqueue_step(fd23_ctx *c, int k, int itrecord) {
     if (c->box && (r = fd23_box_launch_post_stress(c, k))) return r;
     dispatch_pass(c, false, ev, track);
     if (commit) enqueue_commit(c, false);
-    if (c->box && (r = fd23_box_launch_post_velocity(c, k))) return r;
+    if (c->box && (r = fd23_box_launch_post_velocity(c, k, left > 1))) return r;
     if (scaled_storage(c) && (k + 1) % kScaleEvery == 0) enqueue_scale_control(c);
     return FD23_OK;
 }
@@ -2012,7 +2013,7 @@ static int enqueue_launch(fd23_ctx *c, int k, int left, int itrecord, int *taken
         return FD23_OK;
     }
     *taken = 1;
-    return enqueue_step(c, k, itrecord);
+    return enqueue_step(c, k, left, itrecord);
 }
 
 // The graph of a chunk of `steps` steps starting on the current buffer set.
@@ -2071,7 +2072,7 @@ static int get_graph(fd23_ctx *c, int itrecord, int steps, fd23_ctx::Chunk *out)
             for (int i = 0; i < n && r == FD23_OK; i++) {
                 c->chain = i;
                 c->stream = i ? c->chain_stream[i - 1] : main;
-                r = enqueue_step(c, s, itrecord);
+                r = enqueue_step(c, s, steps - s, itrecord);
                 c->stream = main;
             }
         c->chain = -1;

@@ -107,20 +107,8 @@ __global__ __launch_bounds__(TX *NW) void k_sh_block(ShFields<S> fa, ShFields<S>
     const int tid = ty * TX + tx;
     const int key = tile * g.nshots + shot;
 
-    // Every global load of the launch is issued before the first barrier,
-    // in two dependent levels, so that the steps wait on no global memory.
-    // Level 1: the heads of the (tile, shot) lists, the step, the source.
-    int it0 = 0, e0 = 0, e1 = 0, r0 = 0, r1 = 0;
-    SrcInfo si{};
-    if (ev.clock) {
-        it0 = ev.clock[0] + ev.k;
-        e0 = ev.tap_start[key];
-        e1 = ev.tap_start[key + 1];
-        r0 = ev.rec_start[key];
-        r1 = ev.rec_start[key + 1];
-        si = ev.src[shot];
-    }
-
+    // Every global load of the launch is issued before the first barrier, so
+    // that the steps wait on no global memory.
     // The region's fields, material, C-PML memory and profiles, with no
     // branch around a load: coordinates are clamped into the grid and a
     // cell off the C-PML reads element 0 of a psi array; cells outside the
@@ -156,8 +144,35 @@ __global__ __launch_bounds__(TX *NW) void k_sh_block(ShFields<S> fa, ShFields<S>
         pVz[r] = pa.V_z[zi];
     }
 
-    // Level 2: the region's source taps (lane i of every wavefront holds list
-    // entry min(i, n-1), read back with readlane; the lists end with one
+    // The heads of the (tile, shot) lists, the step and the source, behind the
+    // loads above: these are scalar loads, which return out of order, and the
+    // next kernel argument that is used waits for all of them (ahead of the
+    // fields a second memory latency: 256 x 128 5.0 -> 4.7 us a step).
+    __builtin_amdgcn_sched_barrier(0);
+    int it0 = 0, e0 = 0, e1 = 0, r0 = 0, r1 = 0;
+    SrcInfo si{};
+    if (ev.clock) {
+        it0 = ev.clock[0] + ev.k;
+        e0 = ev.tap_start[key];
+        e1 = ev.tap_start[key + 1];
+        r0 = ev.rec_start[key];
+        r1 = ev.rec_start[key + 1];
+        si = ev.src[shot];
+    }
+
+    // LDS: cells outside the region 0 (the rows above and below, the
+    // columns left and right)
+    for (int i = tid; i < LH * LW; i += TX * NW) {
+        const int r = i / LW, col = i - r * LW;
+        if (r < HALO || r >= LH - HALO || col < HALO || col >= LW - HALO) {
+            sV[i] = C(0);
+            sX[i] = C(0);
+            sZ[i] = C(0);
+        }
+    }
+
+    // Behind those, the region's source taps (lane i of every wavefront holds
+    // list entry min(i, n-1), read back with readlane; the lists end with one
     // spare entry, so an empty list reads that), the source samples of the
     // launch's steps, the thread's first receiver.  Nothing waits for them
     // before the first stress half needs the taps.
@@ -197,16 +212,7 @@ __global__ __launch_bounds__(TX *NW) void k_sh_block(ShFields<S> fa, ShFields<S>
         muz[r] = in ? muz[r] : C(0);
     }
 
-    // LDS: cells outside the region 0 (the rows above and below, the
-    // columns left and right), the region's V, the z profiles
-    for (int i = tid; i < LH * LW; i += TX * NW) {
-        const int r = i / LW, col = i - r * LW;
-        if (r < HALO || r >= LH - HALO || col < HALO || col >= LW - HALO) {
-            sV[i] = C(0);
-            sX[i] = C(0);
-            sZ[i] = C(0);
-        }
-    }
+    // LDS: the region's V, the z profiles
 #pragma unroll
     for (int r = 0; r < CZ; r++) sV[(lz0 + r + HALO) * LW + tx + HALO] = v[r];
     if (tid < B::RH) {
@@ -239,9 +245,17 @@ __global__ __launch_bounds__(TX *NW) void k_sh_block(ShFields<S> fa, ShFields<S>
         if (j >= w.nsub) break;
         const int it = it0 + j;
         const int nt_ = son[j] ? ntap : 0; // taps active this step
+        // the rows that the tile still depends on: V of 7 rows around it per
+        // step after this one, and Tx, Tz of the rows z-3..z+4 that V of those
+        // reads.  Other rows are left stale (uniform per wavefront; half of the
+        // rows of the two-step shapes; 256 x 128 5.2 -> 5.0 us a step)
+        const int left = kBlockReach * (w.nsub - 1 - j);
+        const bool need_s = lz0 + CZ > H - left - 3 && lz0 < H + B::OZ + left + 4;
+        const bool need_v = lz0 + CZ > H - left && lz0 < H + B::OZ + left;
 
         // ---- stress half: Tx, Tz from V (k_sh_stress)
-        if (wint) {
+        if (!need_s) {
+        } else if (wint) {
 #pragma unroll
             for (int r = 0; r < CZ; r++) {
                 const C *pv = &sV[(lz0 + r + HALO) * LW + tx + HALO];
@@ -293,10 +307,12 @@ __global__ __launch_bounds__(TX *NW) void k_sh_block(ShFields<S> fa, ShFields<S>
                 else sz[r] = apply_tap(sz[r], tp, sval[j]);
             }
         }
+        if (need_s) {
 #pragma unroll
-        for (int r = 0; r < CZ; r++) {
-            sX[(lz0 + r + HALO) * LW + tx + HALO] = sx[r];
-            sZ[(lz0 + r + HALO) * LW + tx + HALO] = sz[r];
+            for (int r = 0; r < CZ; r++) {
+                sX[(lz0 + r + HALO) * LW + tx + HALO] = sx[r];
+                sZ[(lz0 + r + HALO) * LW + tx + HALO] = sz[r];
+            }
         }
         __syncthreads();
         if (img) {
@@ -322,7 +338,8 @@ __global__ __launch_bounds__(TX *NW) void k_sh_block(ShFields<S> fa, ShFields<S>
         }
 
         // ---- velocity half: V from Tx, Tz (k_sh_velocity)
-        if (wint) {
+        if (!need_v) {
+        } else if (wint) {
 #pragma unroll
             for (int r = 0; r < CZ; r++) {
                 const int o = (lz0 + r + HALO) * LW + tx + HALO;
@@ -361,8 +378,10 @@ __global__ __launch_bounds__(TX *NW) void k_sh_block(ShFields<S> fa, ShFields<S>
         // V of the region is read again by the next stress half only, after
         // the barrier below; the stress half's reads of sV ended at the
         // barrier above
+        if (need_v) {
 #pragma unroll
-        for (int r = 0; r < CZ; r++) sV[(lz0 + r + HALO) * LW + tx + HALO] = v[r];
+            for (int r = 0; r < CZ; r++) sV[(lz0 + r + HALO) * LW + tx + HALO] = v[r];
+        }
 
         __syncthreads();
         // receivers of the tile (the lists hold tile cells only), one per

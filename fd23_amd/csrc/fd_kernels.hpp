@@ -227,6 +227,32 @@ template <class C, class T> __device__ __forceinline__ C apply_tap(C v, const T 
     return C((double)v + tp.q * sv * tp.m);
 }
 
+// The step and the heads of a (tile, shot)'s lists, read once the tile's own
+// loads are in flight: scalar loads return out of order, so the next use of
+// any kernel argument waits for all of them, and read at the kernel's start
+// (or behind the material, selected to 0 off the grid) they put a second
+// memory latency ahead of the fields (us a step: P-SV 301 x 223 7.8, 7.6
+// behind them; 2000 x 1000 32.6 and 31.3; 64 shots of 1024 x 512 492 and 475;
+// SH 6 shots of 2048 x 1024 96 and 92).
+struct ListHeads {
+    int it, tap0, tap1, rec0, rec1, t0;
+};
+__device__ __forceinline__ ListHeads list_heads(const Events &ev, int key, int shot, bool rec) {
+    ListHeads h{};
+    __builtin_amdgcn_sched_barrier(0);
+    if (ev.clock) {
+        h.it = ev.clock[0] + ev.k;
+        h.tap0 = ev.tap_start[key];
+        h.tap1 = ev.tap_start[key + 1];
+        if (rec) {
+            h.rec0 = ev.rec_start[key];
+            h.rec1 = ev.rec_start[key + 1];
+            h.t0 = ev.src[shot].t0;
+        }
+    }
+    return h;
+}
+
 // ---------------------------------------------------------------------------
 // tile staging through registers: all loads first, LDS writes afterwards
 //  ZH: the 4-row halos above/below (all TX columns)
@@ -437,11 +463,12 @@ __global__ __launch_bounds__(TX *BY) void k_psv_stress(PsvFields<S> f, PsvStress
     bool interior = REGION == REGION_INTERIOR  ? true
                     : REGION == REGION_EDGE    ? false
                                                : tile_interior(g, x0, z0, TZ);
-    const int it = ev.clock ? ev.clock[0] + ev.k : 0;
+    int it = 0; // set with the list heads below; a window needs it first
     // first-arrival window: the interior-only kernel is never launched with
     // one; a tile with a closed block takes the exact path, which masks rows
     const bool pun = REGION != REGION_INTERIOR && punch_on(g, ev); // uniform
     if (pun) {
+        it = ev.clock[0] + ev.k;
         const int tw = tile_window<SPB>(g, ev, t, it);
         if (tw == kTileIdle) return;
         interior = interior && tw == kTileOpen;
@@ -468,7 +495,7 @@ __global__ __launch_bounds__(TX *BY) void k_psv_stress(PsvFields<S> f, PsvStress
         psc.w[0] = inv_pow2(scl[kNextScale + SC_PU_X]); psc.w[1] = inv_pow2(scl[kNextScale + SC_PW_X]);
         psc.w[2] = inv_pow2(scl[kNextScale + SC_PU_Z]); psc.w[3] = inv_pow2(scl[kNextScale + SC_PW_Z]);
     }
-    constexpr bool kPrePsi = REGION == REGION_EDGE;
+    constexpr bool kPrePsi = REGION == REGION_EDGE || (REGION == REGION_ALL && RZ == 1 && !ST::scaled);
 
     // buffer addressing: byte pitch of a row and this lane's column
     constexpr unsigned SZ = sizeof(S);
@@ -480,29 +507,10 @@ __global__ __launch_bounds__(TX *BY) void k_psv_stress(PsvFields<S> f, PsvStress
     C lam[RZ], mu[RZ], mua[RZ];
 #pragma unroll
     for (int r = 0; r < RZ; r++) {
-        const int gz = z0 + lz0 + r;
-        const bool live = gx < nx && gz < nz;
-        const unsigned so = (unsigned)gz * pxm;
-        lam[r] = live ? Store<C>::ldb(rLAM, vmat, so, 1.f) : C(0);
-        mu[r] = live ? Store<C>::ldb(rMU, vmat, so, 1.f) : C(0);
-        mua[r] = live ? Store<C>::ldb(rMUA, vmat, so, 1.f) : C(0);
-    }
-
-    // edge-only kernels: so are the profile entries of the thread's column and
-    // rows, once for all shots; read where they are used, each of the rows
-    // waited for two loads in turn
-    PmlCoef<C> xv[2], zv[kPrePsi ? RZ : 1][2];
-    if constexpr (kPrePsi) {
-        const bool inx = gx < nx && (gx < g.npml || gx >= nx - g.npml);
-        xv[0] = pml_coef(pr.Ux, gx, inx);
-        xv[1] = pml_coef(pr.Wx, gx, inx);
-#pragma unroll
-        for (int r = 0; r < RZ; r++) {
-            const int iz = z0 + lz0 + r;
-            const bool inz = iz < nz && ((iz < g.npml && g.top) || iz >= nz - g.npml);
-            zv[r][0] = pml_coef(pr.Wz, iz, inz);
-            zv[r][1] = pml_coef(pr.Uz, iz, inz);
-        }
+        const unsigned so = (unsigned)min(z0 + lz0 + r, nz - 1) * pxm;
+        lam[r] = Store<C>::ldb(rLAM, vmat, so, 1.f);
+        mu[r] = Store<C>::ldb(rMU, vmat, so, 1.f);
+        mua[r] = Store<C>::ldb(rMUA, vmat, so, 1.f);
     }
 
     const int sh0 = t.group * SPB;
@@ -527,10 +535,12 @@ __global__ __launch_bounds__(TX *BY) void k_psv_stress(PsvFields<S> f, PsvStress
             tzz[r] = ST::ldb(bZZ, vcol, so, sc_zz);
             txz[r] = ST::ldb(bXZ, vcol, so, sc_xz);
         }
-        // edge-only kernels: this shot's C-PML memory variables (U_x W_x
-        // W_z U_z) are loaded with the fields, ahead of the barrier
+        // edge-only kernels and one row per thread: this shot's C-PML memory
+        // variables (U_x W_x W_z U_z) are loaded with the fields, ahead of the
+        // barrier (FP64 640 x 401 11.9 -> 11.1 us a step; with more rows of whole
+        // tiles, or 16-bit storage, the registers cost more than the latency)
         C pq[4][kPrePsi ? RZ : 1];
-        if constexpr (kPrePsi) {
+        if (kPrePsi && !interior) {
 #pragma unroll
             for (int r = 0; r < RZ; r++) {
                 const int iz = z0 + lz0 + r;
@@ -549,6 +559,22 @@ __global__ __launch_bounds__(TX *BY) void k_psv_stress(PsvFields<S> f, PsvStress
                 }
             }
         }
+        // and the profile entries of the thread's column and rows
+        PmlCoef<C> xv[2], zv[kPrePsi ? RZ : 1][2];
+        if (kPrePsi && !interior) {
+            const bool inx = gx < nx && (gx < g.npml || gx >= nx - g.npml);
+            xv[0] = pml_coef(pr.Ux, gx, inx);
+            xv[1] = pml_coef(pr.Wx, gx, inx);
+#pragma unroll
+            for (int r = 0; r < RZ; r++) {
+                const int iz = z0 + lz0 + r;
+                const bool inz = iz < nz && ((iz < g.npml && g.top) || iz >= nz - g.npml);
+                zv[r][0] = pml_coef(pr.Wz, iz, inz);
+                zv[r][1] = pml_coef(pr.Uz, iz, inz);
+            }
+        }
+        const ListHeads h = list_heads(ev, t.tile * g.nshots + shot, shot, false);
+        it = h.it;
         if (s > 0) __syncthreads();
         rU.store(sU);
         rW.store(sW);
@@ -593,11 +619,9 @@ __global__ __launch_bounds__(TX *BY) void k_psv_stress(PsvFields<S> f, PsvStress
         // fused source injection: the owner of a tap cell adds it after the
         // cell's own update, taps in the reference's order
         if (ev.clock) {
-            const int key = t.tile * g.nshots + shot;
-            const int e0 = ev.tap_start[key], e1 = ev.tap_start[key + 1];
             double sv;
-            if (e1 > e0 && src_sample(ev.src[shot], ev.stf, it, sv)) {
-                for (int e = e0; e < e1; e++) {
+            if (h.tap1 > h.tap0 && src_sample(ev.src[shot], ev.stf, it, sv)) {
+                for (int e = h.tap0; e < h.tap1; e++) {
                     const TapT tp = ev.taps[e];
                     const int lx = tp.cell % TX, lz = tp.cell / TX;
                     if (lx != tx || lz < lz0 || lz >= lz0 + RZ) continue;
@@ -642,10 +666,10 @@ __global__ __launch_bounds__(TX *BY) void k_psv_stress(PsvFields<S> f, PsvStress
 // the tile's receivers read them.  Uniform per workgroup.  KEPT: receivers
 // in the work's kept rectangle are recorded by another kernel.
 template <class C, int RZ, int NV, bool KEPT = false>
-__device__ __forceinline__ void fused_record(const Events &ev, int it, int key, C *park0, C *park1,
-                                             const C (&val)[NV][RZ], int lz0, int t0, const Work &w, int x0, int z0) {
-    const int e0 = ev.rec_start[key], e1 = ev.rec_start[key + 1];
-    const int ts = it - t0; // step of the shot
+__device__ __forceinline__ void fused_record(const Events &ev, const ListHeads &h, C *park0, C *park1,
+                                             const C (&val)[NV][RZ], int lz0, const Work &w, int x0, int z0) {
+    const int e0 = h.rec0, e1 = h.rec1;
+    const int ts = h.it - h.t0; // step of the shot
     if (e1 <= e0 || ts < 0 || ts % ev.itrecord != 0) return;
     const int frame = ts / ev.itrecord;
     if (frame >= ev.max_frames) return;
@@ -765,11 +789,12 @@ __global__ __launch_bounds__(TX *BY) void k_psv_velocity(PsvFields<S> f, PsvVelM
     bool interior = REGION == REGION_INTERIOR  ? true
                     : REGION == REGION_EDGE    ? false
                                                : tile_interior(g, x0, z0, TZ);
-    const int it = ev.clock ? ev.clock[0] + ev.k : 0;
+    int it = 0; // set with the list heads below; a window needs it first
     // first-arrival window: the interior-only kernel is never launched with
     // one; a tile with a closed block takes the exact path, which masks rows
     const bool pun = REGION != REGION_INTERIOR && punch_on(g, ev); // uniform
     if (pun) {
+        it = ev.clock[0] + ev.k;
         const int tw = tile_window<SPB>(g, ev, t, it);
         if (tw == kTileIdle) return;
         interior = interior && tw == kTileOpen;
@@ -791,7 +816,7 @@ __global__ __launch_bounds__(TX *BY) void k_psv_velocity(PsvFields<S> f, PsvVelM
         psc.w[0] = inv_pow2(scl[kNextScale + SC_PTXX_X]); psc.w[1] = inv_pow2(scl[kNextScale + SC_PTXZ_X]);
         psc.w[2] = inv_pow2(scl[kNextScale + SC_PTXZ_Z]); psc.w[3] = inv_pow2(scl[kNextScale + SC_PTZZ_Z]);
     }
-    constexpr bool kPrePsi = REGION == REGION_EDGE;
+    constexpr bool kPrePsi = REGION == REGION_EDGE || (REGION == REGION_ALL && RZ == 1 && !ST::scaled);
 
     // buffer addressing: byte pitch of a row and this lane's column
     constexpr unsigned SZ = sizeof(S);
@@ -802,28 +827,9 @@ __global__ __launch_bounds__(TX *BY) void k_psv_velocity(PsvFields<S> f, PsvVelM
     C bu[RZ], bw[RZ];
 #pragma unroll
     for (int r = 0; r < RZ; r++) {
-        const int gz = z0 + lz0 + r;
-        const bool live = gx < nx && gz < nz;
-        const unsigned so = (unsigned)gz * pxm;
-        bu[r] = live ? Store<C>::ldb(rBU, vmat, so, 1.f) : C(0);
-        bw[r] = live ? Store<C>::ldb(rBW, vmat, so, 1.f) : C(0);
-    }
-
-    // edge-only kernels: so are the profile entries of the thread's column and
-    // rows, once for all shots; read where they are used, each of the rows
-    // waited for two loads in turn
-    PmlCoef<C> xv[2], zv[kPrePsi ? RZ : 1][2];
-    if constexpr (kPrePsi) {
-        const bool inx = gx < nx && (gx < g.npml || gx >= nx - g.npml);
-        xv[0] = pml_coef(pr.Txx_x, gx, inx);
-        xv[1] = pml_coef(pr.Txz_x, gx, inx);
-#pragma unroll
-        for (int r = 0; r < RZ; r++) {
-            const int iz = z0 + lz0 + r;
-            const bool inz = iz < nz && ((iz < g.npml && g.top) || iz >= nz - g.npml);
-            zv[r][0] = pml_coef(pr.Txz_z, iz, inz);
-            zv[r][1] = pml_coef(pr.Tzz_z, iz, inz);
-        }
+        const unsigned so = (unsigned)min(z0 + lz0 + r, nz - 1) * pxm;
+        bu[r] = Store<C>::ldb(rBU, vmat, so, 1.f);
+        bw[r] = Store<C>::ldb(rBW, vmat, so, 1.f);
     }
 
     const int sh0 = t.group * SPB;
@@ -854,7 +860,7 @@ __global__ __launch_bounds__(TX *BY) void k_psv_velocity(PsvFields<S> f, PsvVelM
         // edge-only kernels: this shot's C-PML memory variables (Txx_x
         // Txz_x Txz_z Tzz_z) are loaded with the fields, ahead of the barrier
         C pq[4][kPrePsi ? RZ : 1];
-        if constexpr (kPrePsi) {
+        if (kPrePsi && !interior) {
 #pragma unroll
             for (int r = 0; r < RZ; r++) {
                 const int iz = z0 + lz0 + r;
@@ -873,6 +879,22 @@ __global__ __launch_bounds__(TX *BY) void k_psv_velocity(PsvFields<S> f, PsvVelM
                 }
             }
         }
+        // and the profile entries of the thread's column and rows
+        PmlCoef<C> xv[2], zv[kPrePsi ? RZ : 1][2];
+        if (kPrePsi && !interior) {
+            const bool inx = gx < nx && (gx < g.npml || gx >= nx - g.npml);
+            xv[0] = pml_coef(pr.Txx_x, gx, inx);
+            xv[1] = pml_coef(pr.Txz_x, gx, inx);
+#pragma unroll
+            for (int r = 0; r < RZ; r++) {
+                const int iz = z0 + lz0 + r;
+                const bool inz = iz < nz && ((iz < g.npml && g.top) || iz >= nz - g.npml);
+                zv[r][0] = pml_coef(pr.Txz_z, iz, inz);
+                zv[r][1] = pml_coef(pr.Tzz_z, iz, inz);
+            }
+        }
+        const ListHeads h = list_heads(ev, t.tile * g.nshots + shot, shot, true);
+        it = h.it;
         if (s > 0) __syncthreads();
         rXX.store(sXX);
         rZZ.store(sZZ);
@@ -926,7 +948,7 @@ __global__ __launch_bounds__(TX *BY) void k_psv_velocity(PsvFields<S> f, PsvVelM
             }
         }
         if (ev.clock)
-            fused_record<C, RZ, 2, TO>(ev, it, t.tile * g.nshots + shot, sXX, sZZ, nv, lz0, ev.src[shot].t0, w, x0, z0);
+            fused_record<C, RZ, 2, TO>(ev, h, sXX, sZZ, nv, lz0, w, x0, z0);
     }
     if (ST::scaled) {
         amax_update(amax, SC_U, mx_u);
@@ -971,7 +993,7 @@ __global__ __launch_bounds__(TX *BY) void k_sh_stress(ShFields<S> f, ShStressMat
     }
     using C = typename Store<S>::C;
     using ST = Store<S>;
-    constexpr bool kPrePsi = TO;
+    constexpr bool kPrePsi = TO || (RZ == 1 && !ST::scaled);
     constexpr int TZ = BY * RZ;
     constexpr int LW = TX + 2 * HALO;
     __shared__ C sV[(TZ + 2 * HALO) * LW];
@@ -985,11 +1007,12 @@ __global__ __launch_bounds__(TX *BY) void k_sh_stress(ShFields<S> f, ShStressMat
     const int gx = x0 + tx;
     const int lz0 = ty * RZ;
     bool interior = tile_interior(g, x0, z0, TZ);
-    const int it = ev.clock ? ev.clock[0] + ev.k : 0;
+    int it = 0; // set with the list heads below; a window needs it first
     // first-arrival window: a tile with a closed block takes the exact
     // path, which masks rows
     const bool pun = punch_on(g, ev); // uniform
     if (pun) {
+        it = ev.clock[0] + ev.k;
         const int tw = tile_window<SPB>(g, ev, t, it);
         if (tw == kTileIdle) return;
         interior = interior && tw == kTileOpen;
@@ -1013,26 +1036,9 @@ __global__ __launch_bounds__(TX *BY) void k_sh_stress(ShFields<S> f, ShStressMat
     C mux[RZ], muz[RZ];
 #pragma unroll
     for (int r = 0; r < RZ; r++) {
-        const int gz = z0 + lz0 + r;
-        const bool live = gx < nx && gz < nz;
-        const unsigned so = (unsigned)gz * pxm;
-        mux[r] = live ? Store<C>::ldb(rMUX, vmat, so, 1.f) : C(0);
-        muz[r] = live ? Store<C>::ldb(rMUZ, vmat, so, 1.f) : C(0);
-    }
-
-    // edge-only kernels: so are the profile entries of the thread's column and
-    // rows, once for all shots; read where they are used, each of the rows
-    // waited for two loads in turn
-    PmlCoef<C> xv[1], zv[kPrePsi ? RZ : 1][1];
-    if constexpr (kPrePsi) {
-        const bool inx = gx < nx && (gx < npml || gx >= nx - npml);
-        xv[0] = pml_coef(pr.x, gx, inx);
-#pragma unroll
-        for (int r = 0; r < RZ; r++) {
-            const int iz = z0 + lz0 + r;
-            const bool inz = iz < nz && ((iz < npml && g.top) || iz >= nz - npml);
-            zv[r][0] = pml_coef(pr.z, iz, inz);
-        }
+        const unsigned so = (unsigned)min(z0 + lz0 + r, nz - 1) * pxm;
+        mux[r] = Store<C>::ldb(rMUX, vmat, so, 1.f);
+        muz[r] = Store<C>::ldb(rMUZ, vmat, so, 1.f);
     }
 
     const int sh0 = t.group * SPB;
@@ -1070,6 +1076,20 @@ __global__ __launch_bounds__(TX *BY) void k_sh_stress(ShFields<S> f, ShStressMat
                                       ST::scaled ? scl[SC_PV_Z] : 1.f);
             }
         }
+        // and the profile entries of the thread's column and rows
+        PmlCoef<C> xv[1], zv[kPrePsi ? RZ : 1][1];
+        if (kPrePsi && !interior) {
+            const bool inx = gx < nx && (gx < npml || gx >= nx - npml);
+            xv[0] = pml_coef(pr.x, gx, inx);
+#pragma unroll
+            for (int r = 0; r < RZ; r++) {
+                const int iz = z0 + lz0 + r;
+                const bool inz = iz < nz && ((iz < npml && g.top) || iz >= nz - npml);
+                zv[r][0] = pml_coef(pr.z, iz, inz);
+            }
+        }
+        const ListHeads h = list_heads(ev, t.tile * g.nshots + shot, shot, false);
+        it = h.it;
         if (s > 0) __syncthreads();
         rV.store(sV);
         __syncthreads();
@@ -1127,11 +1147,9 @@ __global__ __launch_bounds__(TX *BY) void k_sh_stress(ShFields<S> f, ShStressMat
         // fused SH source, stress taps (Tx, Tz); a point force on V is added
         // by the velocity pass, which is the only pass that writes V
         if (ev.clock) {
-            const int key = t.tile * g.nshots + shot;
-            const int e0 = ev.tap_start[key], e1 = ev.tap_start[key + 1];
             double sv;
-            if (e1 > e0 && src_sample(ev.src[shot], ev.stf, it, sv)) {
-                for (int e = e0; e < e1; e++) {
+            if (h.tap1 > h.tap0 && src_sample(ev.src[shot], ev.stf, it, sv)) {
+                for (int e = h.tap0; e < h.tap1; e++) {
                     const TapT tp = ev.taps[e];
                     const int lx = tp.cell % TX, lz = tp.cell / TX;
                     if (tp.field == 0 || lx != tx || lz < lz0 || lz >= lz0 + RZ) continue;
@@ -1181,7 +1199,7 @@ __global__ __launch_bounds__(TX *BY) void k_sh_velocity(ShFields<S> f, const typ
     }
     using C = typename Store<S>::C;
     using ST = Store<S>;
-    constexpr bool kPrePsi = TO;
+    constexpr bool kPrePsi = TO || (RZ == 1 && !ST::scaled);
     constexpr int TZ = BY * RZ;
     constexpr int LW = TX + 2 * HALO;
     __shared__ C sX[(TZ + 2 * HALO) * LW];
@@ -1196,11 +1214,12 @@ __global__ __launch_bounds__(TX *BY) void k_sh_velocity(ShFields<S> f, const typ
     const int gx = x0 + tx;
     const int lz0 = ty * RZ;
     bool interior = tile_interior(g, x0, z0, TZ);
-    const int it = ev.clock ? ev.clock[0] + ev.k : 0;
+    int it = 0; // set with the list heads below; a window needs it first
     // first-arrival window: a tile with a closed block takes the exact
     // path, which masks rows
     const bool pun = punch_on(g, ev); // uniform
     if (pun) {
+        it = ev.clock[0] + ev.k;
         const int tw = tile_window<SPB>(g, ev, t, it);
         if (tw == kTileIdle) return;
         interior = interior && tw == kTileOpen;
@@ -1226,24 +1245,7 @@ __global__ __launch_bounds__(TX *BY) void k_sh_velocity(ShFields<S> f, const typ
     C bv[RZ];
 #pragma unroll
     for (int r = 0; r < RZ; r++) {
-        const int gz = z0 + lz0 + r;
-        const bool live = gx < nx && gz < nz;
-        bv[r] = live ? Store<C>::ldb(rBV, vmat, (unsigned)gz * pxm, 1.f) : C(0);
-    }
-
-    // edge-only kernels: so are the profile entries of the thread's column and
-    // rows, once for all shots; read where they are used, each of the rows
-    // waited for two loads in turn
-    PmlCoef<C> xv[1], zv[kPrePsi ? RZ : 1][1];
-    if constexpr (kPrePsi) {
-        const bool inx = gx < nx && (gx < npml || gx >= nx - npml);
-        xv[0] = pml_coef(pr.x, gx, inx);
-#pragma unroll
-        for (int r = 0; r < RZ; r++) {
-            const int iz = z0 + lz0 + r;
-            const bool inz = iz < nz && ((iz < npml && g.top) || iz >= nz - npml);
-            zv[r][0] = pml_coef(pr.z, iz, inz);
-        }
+        bv[r] = Store<C>::ldb(rBV, vmat, (unsigned)min(z0 + lz0 + r, nz - 1) * pxm, 1.f);
     }
 
     const int sh0 = t.group * SPB;
@@ -1287,6 +1289,20 @@ __global__ __launch_bounds__(TX *BY) void k_sh_velocity(ShFields<S> f, const typ
                                       ST::scaled ? scl[SC_PTZ_Z] : 1.f);
             }
         }
+        // and the profile entries of the thread's column and rows
+        PmlCoef<C> xv[1], zv[kPrePsi ? RZ : 1][1];
+        if (kPrePsi && !interior) {
+            const bool inx = gx < nx && (gx < npml || gx >= nx - npml);
+            xv[0] = pml_coef(pr.x, gx, inx);
+#pragma unroll
+            for (int r = 0; r < RZ; r++) {
+                const int iz = z0 + lz0 + r;
+                const bool inz = iz < nz && ((iz < npml && g.top) || iz >= nz - npml);
+                zv[r][0] = pml_coef(pr.z, iz, inz);
+            }
+        }
+        const ListHeads h = list_heads(ev, t.tile * g.nshots + shot, shot, true);
+        it = h.it;
         if (s > 0) __syncthreads();
         rX.store(sX);
         rZ.store(sZ);
@@ -1301,11 +1317,9 @@ __global__ __launch_bounds__(TX *BY) void k_sh_velocity(ShFields<S> f, const typ
         // fused SH point force (cu_point_force): V += source before the
         // cell's velocity update, as the reference injects between passes
         if (ev.clock) {
-            const int key = t.tile * g.nshots + shot;
-            const int e0 = ev.tap_start[key], e1 = ev.tap_start[key + 1];
             double sv;
-            if (e1 > e0 && src_sample(ev.src[shot], ev.stf, it, sv)) {
-                for (int e = e0; e < e1; e++) {
+            if (h.tap1 > h.tap0 && src_sample(ev.src[shot], ev.stf, it, sv)) {
+                for (int e = h.tap0; e < h.tap1; e++) {
                     const TapT tp = ev.taps[e];
                     const int lx = tp.cell % TX, lz = tp.cell / TX;
                     if (tp.field != 0 || lx != tx || lz < lz0 || lz >= lz0 + RZ) continue;
@@ -1374,7 +1388,7 @@ __global__ __launch_bounds__(TX *BY) void k_sh_velocity(ShFields<S> f, const typ
             ST::stb(oV, vcol, (unsigned)(gz + HALO) * pxb, nv[0][r], wi_v);
             if (ST::scaled && amax) mx_v = fmaxf(mx_v, fabsf((float)nv[0][r]));
         }
-        if (ev.clock) fused_record<C, RZ, 1, TO>(ev, it, t.tile * g.nshots + shot, sX, sX, nv, lz0, ev.src[shot].t0, w, x0, z0);
+        if (ev.clock) fused_record<C, RZ, 1, TO>(ev, h, sX, sX, nv, lz0, w, x0, z0);
     }
     if (ST::scaled) {
         amax_update(amax, SC_V, mx_v);

@@ -144,74 +144,111 @@ __global__ void k_box_add(BoxPar p, C *const *glob, const C *resid, const int *c
 // one kernel with the rings around it: the sub ring of the fields it
 // differentiates, staged with their halo (a workgroup computes the ring's
 // values of its halo for itself, none writes what another reads), and the add
-// ring of the fields it updates.  The step of a 640 x 401 FP64 grid is a chain
-// of dependent launches (38 us); as three kernels a pass, six of its eight
-// were rings and residual passes of 3.7 and 4.4 us each.
+// ring of the fields it updates.  What bounds a step is its chain of dependent
+// launches and memory latencies: 60 steps of 640 x 401 in FP64, with the reset
+// and the readback, took 3.36 ms with the rings and the residual passes as
+// kernels of their own (eight launches a step, rings 3.7 and residual passes
+// 4.4 us), 2.83 fused and 2.27 with the loads below issued together.
+//
+// A thread stages its own cell, one of the four rows above or below the tile,
+// and the first 64 one of the four columns beside it; every load is issued
+// before the first is used.
 constexpr int KX = 32, KZ = 8, KH = 4, KW = KX + 2 * KH, KN = KW * (KZ + 2 * KH);
 
-struct BoxTile {
-    int i0, j0, shot;
+// a cell to be staged: where it is in the tile and in the arrays (clamped
+// into the box), and whether it is in the box and in its sub ring (depth 0..3)
+struct Spot {
+    int i, j, lds;
+    bool in, ring;
+    long cell, q;
 };
+struct BoxTile {
+    int i0, j0, shot, tx, tz;
+    Spot own, row, col;
+};
+__device__ __forceinline__ Spot box_spot(const BoxPar &p, const BoxTile &b, int li, int lj) {
+    Spot s;
+    s.i = b.i0 + li;
+    s.j = b.j0 + lj;
+    s.lds = (lj + KH) * KW + li + KH;
+    s.in = s.i >= 0 && s.i < p.bx && s.j >= 0 && s.j < p.bz;
+    s.ring = s.in && ring_depth(s.i, s.j, p.bx, p.bz) <= 3;
+    const int ci = min(max(s.i, 0), p.bx - 1), cj = min(max(s.j, 0), p.bz - 1);
+    s.cell = (long)cj * p.bx + ci;
+    s.q = (long)(p.z0 + cj) * p.px + p.x0 + ci;
+    return s;
+}
 __device__ __forceinline__ BoxTile box_tile(const BoxPar &p) {
     const int ntx = (p.bx + KX - 1) / KX, ntz = (p.bz + KZ - 1) / KZ;
-    const int t = (int)blockIdx.x % (ntx * ntz);
-    return BoxTile{t % ntx * KX, t / ntx * KZ, (int)blockIdx.x / (ntx * ntz)};
+    const int t = (int)blockIdx.x % (ntx * ntz), tid = (int)threadIdx.x;
+    BoxTile b;
+    b.i0 = t % ntx * KX;
+    b.j0 = t / ntx * KZ;
+    b.shot = (int)blockIdx.x / (ntx * ntz);
+    b.tx = tid % KX;
+    b.tz = tid / KX;
+    b.own = box_spot(p, b, b.tx, b.tz);
+    b.row = box_spot(p, b, b.tx, b.tz < KH ? b.tz - KH : b.tz + KZ - KH);
+    b.col = box_spot(p, b, (tid & 7) < KH ? (tid & 7) - KH : (tid & 7) + KX - KH, (tid >> 3) & (KZ - 1));
+    return b;
 }
-// field fi with its halo: the residual grid's values, in the sub ring
-// (depth 0..3) a - s, which the owner stores; zero outside the box
+// a staged value as loaded, from the global grid in the sub ring
+template <class C> __device__ __forceinline__ C spot_load(const Spot &s, const C *glob, const C *r) {
+    return *(s.ring ? glob + s.q : r + s.cell);
+}
+// a - s in the sub ring, zero outside the box
 template <class C>
-__device__ __forceinline__ void stage_ring(const BoxPar &p, const BoxTile &b, int fi, const C *glob, C *resid, double t,
-                                           const double *stab, C *lds) {
-    const long nb = (long)p.bx * p.bz;
-    C *r = resid + ((long)b.shot * 5 + fi) * nb;
-    for (int e = (int)threadIdx.x; e < KN; e += KX * KZ) {
-        const int li = e % KW - KH, lj = e / KW - KH, i = b.i0 + li, j = b.j0 + lj;
-        C v = C(0);
-        if (i >= 0 && i < p.bx && j >= 0 && j < p.bz) {
-            const long cell = (long)j * p.bx + i;
-            if (ring_depth(i, j, p.bx, p.bz) <= 3) {
-                v = glob[(long)b.shot * p.sstride + (long)(p.z0 + j) * p.px + (p.x0 + i)] -
-                    ring_drive<C>(p, fi, i, j, t, stab);
-                if (li >= 0 && li < KX && lj >= 0 && lj < KZ) r[cell] = v;
-            } else {
-                v = r[cell];
-            }
-        }
-        lds[e] = v;
-    }
+__device__ __forceinline__ C spot_value(const BoxPar &p, const Spot &s, int fi, C v, double t, const double *stab) {
+    if (s.ring) v = v - ring_drive<C>(p, fi, s.i, s.j, t, stab);
+    return s.in ? v : C(0);
 }
+
 template <class C>
 __global__ __launch_bounds__(KX *KZ) void k_box_stress_r(BoxPar p, C *const *glob, C *resid, const C *LAMg,
                                                          const C *MUg, const C *MUAg, const int *clock, int k,
                                                          int it_arg, const double *stab) {
-    __shared__ C sU[KN], sW[KN];
-    const int it = clock ? clock[0] + k : it_arg;
+    __shared__ C sV[2][KN];
     const BoxTile b = box_tile(p);
-    stage_ring(p, b, 0, glob[0], resid, (it + 0.5) * p.dt, stab, sU);
-    stage_ring(p, b, 1, glob[1], resid, (it + 0.5) * p.dt, stab, sW);
-    __syncthreads();
-    const int li = (int)threadIdx.x % KX, lj = (int)threadIdx.x / KX, i = b.i0 + li, j = b.j0 + lj;
-    if (i >= p.bx || j >= p.bz) return;
-    const int o = (lj + KH) * KW + li + KH;
-    const C c0 = C(1225. / 1024.), c1 = C(245. / 3072.), c2 = C(49. / 5120.), c3 = C(5. / 7168.);
-    const C ux = dm(&sU[o], 1, c0, c1, c2, c3), uz = dm(&sU[o], KW, c0, c1, c2, c3);
-    const C wx = dp(&sW[o], 1, c0, c1, c2, c3), wz = dp(&sW[o], KW, c0, c1, c2, c3);
-    const long qg = (long)(p.z0 + j) * p.px + p.x0 + i;
-    const C lam = LAMg[qg], mu = MUg[qg], mua = MUAg[qg];
-    const C gam = lam + C(2.0) * mu;
-    const long nb = (long)p.bx * p.bz, q = (long)j * p.bx + i;
-    C *T = resid + ((long)b.shot * 5 + 2) * nb + q;
-    C v[3];
-    v[0] = T[0] + (gam * ux + lam * wz);
-    v[1] = T[nb] + (lam * ux + gam * wz);
-    v[2] = T[2 * nb] + mua * (wx + uz);
-    const int d = ring_depth(i, j, p.bx, p.bz);
+    const bool side = threadIdx.x < 8 * KZ;
+    const long nb = (long)p.bx * p.bz, shift = (long)b.shot * p.sstride;
+    C *R = resid + (long)b.shot * 5 * nb, *T = R + 2 * nb + b.own.cell;
+    C own[2], row[2], col[2], v[3];
 #pragma unroll
-    for (int f = 0; f < 3; f++) {
-        T[f * nb] = v[f];
-        if (d >= 4 && d <= 7)
-            glob[2 + f][(long)b.shot * p.sstride + qg] = v[f] + ring_drive<C>(p, 2 + f, i, j, (it + 1.0) * p.dt, stab);
+    for (int f = 0; f < 2; f++) {
+        own[f] = spot_load(b.own, (const C *)glob[f] + shift, R + f * nb);
+        row[f] = spot_load(b.row, (const C *)glob[f] + shift, R + f * nb);
+        col[f] = spot_load(b.col, (const C *)glob[f] + shift, R + f * nb);
     }
+#pragma unroll
+    for (int f = 0; f < 3; f++) v[f] = T[f * nb];
+    const C lam = LAMg[b.own.q], mu = MUg[b.own.q], mua = MUAg[b.own.q];
+    const int it = clock ? clock[0] + k : it_arg;
+    const double tv = (it + 0.5) * p.dt;
+#pragma unroll
+    for (int f = 0; f < 2; f++) {
+        own[f] = spot_value(p, b.own, f, own[f], tv, stab);
+        if (b.own.ring) R[f * nb + b.own.cell] = own[f];
+        sV[f][b.own.lds] = own[f];
+        sV[f][b.row.lds] = spot_value(p, b.row, f, row[f], tv, stab);
+        if (side) sV[f][b.col.lds] = spot_value(p, b.col, f, col[f], tv, stab);
+    }
+    __syncthreads();
+    if (!b.own.in) return;
+    const C c0 = C(1225. / 1024.), c1 = C(245. / 3072.), c2 = C(49. / 5120.), c3 = C(5. / 7168.);
+    const C *U = &sV[0][b.own.lds], *W = &sV[1][b.own.lds];
+    const C ux = dm(U, 1, c0, c1, c2, c3), uz = dm(U, KW, c0, c1, c2, c3);
+    const C wx = dp(W, 1, c0, c1, c2, c3), wz = dp(W, KW, c0, c1, c2, c3);
+    const C gam = lam + C(2.0) * mu;
+    v[0] = v[0] + (gam * ux + lam * wz);
+    v[1] = v[1] + (lam * ux + gam * wz);
+    v[2] = v[2] + mua * (wx + uz);
+#pragma unroll
+    for (int f = 0; f < 3; f++) T[f * nb] = v[f];
+    const int d = ring_depth(b.own.i, b.own.j, p.bx, p.bz);
+    if (d < 4 || d > 7) return;
+#pragma unroll
+    for (int f = 0; f < 3; f++)
+        glob[2 + f][shift + b.own.q] = v[f] + ring_drive<C>(p, 2 + f, b.own.i, b.own.j, (it + 1.0) * p.dt, stab);
 }
 
 // add: with the next step's add ring of the velocities
@@ -219,33 +256,46 @@ template <class C>
 __global__ __launch_bounds__(KX *KZ) void k_box_velocity_r(BoxPar p, C *const *glob, C *resid, const C *BUg,
                                                            const C *BWg, const int *clock, int k, int it_arg,
                                                            const double *stab, bool add) {
-    __shared__ C sXX[KN], sZZ[KN], sXZ[KN];
-    const int it = clock ? clock[0] + k : it_arg;
+    __shared__ C sT[3][KN];
     const BoxTile b = box_tile(p);
-    stage_ring(p, b, 2, glob[2], resid, (it + 1.0) * p.dt, stab, sXX);
-    stage_ring(p, b, 3, glob[3], resid, (it + 1.0) * p.dt, stab, sZZ);
-    stage_ring(p, b, 4, glob[4], resid, (it + 1.0) * p.dt, stab, sXZ);
-    __syncthreads();
-    const int li = (int)threadIdx.x % KX, lj = (int)threadIdx.x / KX, i = b.i0 + li, j = b.j0 + lj;
-    if (i >= p.bx || j >= p.bz) return;
-    const int o = (lj + KH) * KW + li + KH;
-    const C c0 = C(1225. / 1024.), c1 = C(245. / 3072.), c2 = C(49. / 5120.), c3 = C(5. / 7168.);
-    const C dxTxx = dp(&sXX[o], 1, c0, c1, c2, c3), dzTzz = dm(&sZZ[o], KW, c0, c1, c2, c3);
-    const C dxTxz = dm(&sXZ[o], 1, c0, c1, c2, c3), dzTxz = dp(&sXZ[o], KW, c0, c1, c2, c3);
-    const long qg = (long)(p.z0 + j) * p.px + p.x0 + i;
-    const C bu = BUg[qg], bw = BWg[qg];
-    const long nb = (long)p.bx * p.bz, q = (long)j * p.bx + i;
-    C *V = resid + (long)b.shot * 5 * nb + q;
-    C v[2];
-    v[0] = V[0] + bu * (dxTxx + dzTxz);
-    v[1] = V[nb] + bw * (dxTxz + dzTzz);
-    const int d = ring_depth(i, j, p.bx, p.bz);
+    const bool side = threadIdx.x < 8 * KZ;
+    const long nb = (long)p.bx * p.bz, shift = (long)b.shot * p.sstride;
+    C *R = resid + (long)b.shot * 5 * nb, *V = R + b.own.cell;
+    C own[3], row[3], col[3], v[2];
 #pragma unroll
-    for (int f = 0; f < 2; f++) {
-        V[f * nb] = v[f];
-        if (add && d >= 4 && d <= 7)
-            glob[f][(long)b.shot * p.sstride + qg] = v[f] + ring_drive<C>(p, f, i, j, (it + 1 + 0.5) * p.dt, stab);
+    for (int f = 0; f < 3; f++) {
+        own[f] = spot_load(b.own, (const C *)glob[2 + f] + shift, R + (2 + f) * nb);
+        row[f] = spot_load(b.row, (const C *)glob[2 + f] + shift, R + (2 + f) * nb);
+        col[f] = spot_load(b.col, (const C *)glob[2 + f] + shift, R + (2 + f) * nb);
     }
+#pragma unroll
+    for (int f = 0; f < 2; f++) v[f] = V[f * nb];
+    const C bu = BUg[b.own.q], bw = BWg[b.own.q];
+    const int it = clock ? clock[0] + k : it_arg;
+    const double tt = (it + 1.0) * p.dt;
+#pragma unroll
+    for (int f = 0; f < 3; f++) {
+        own[f] = spot_value(p, b.own, 2 + f, own[f], tt, stab);
+        if (b.own.ring) R[(2 + f) * nb + b.own.cell] = own[f];
+        sT[f][b.own.lds] = own[f];
+        sT[f][b.row.lds] = spot_value(p, b.row, 2 + f, row[f], tt, stab);
+        if (side) sT[f][b.col.lds] = spot_value(p, b.col, 2 + f, col[f], tt, stab);
+    }
+    __syncthreads();
+    if (!b.own.in) return;
+    const C c0 = C(1225. / 1024.), c1 = C(245. / 3072.), c2 = C(49. / 5120.), c3 = C(5. / 7168.);
+    const C *Txx = &sT[0][b.own.lds], *Tzz = &sT[1][b.own.lds], *Txz = &sT[2][b.own.lds];
+    const C dxTxx = dp(Txx, 1, c0, c1, c2, c3), dzTzz = dm(Tzz, KW, c0, c1, c2, c3);
+    const C dxTxz = dm(Txz, 1, c0, c1, c2, c3), dzTxz = dp(Txz, KW, c0, c1, c2, c3);
+    v[0] = v[0] + bu * (dxTxx + dzTxz);
+    v[1] = v[1] + bw * (dxTxz + dzTzz);
+#pragma unroll
+    for (int f = 0; f < 2; f++) V[f * nb] = v[f];
+    const int d = ring_depth(b.own.i, b.own.j, p.bx, p.bz);
+    if (!add || d < 4 || d > 7) return;
+#pragma unroll
+    for (int f = 0; f < 2; f++)
+        glob[f][shift + b.own.q] = v[f] + ring_drive<C>(p, f, b.own.i, b.own.j, (it + 1 + 0.5) * p.dt, stab);
 }
 
 // force the box medium into the global material (the reference's

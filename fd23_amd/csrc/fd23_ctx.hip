@@ -79,22 +79,22 @@ enum { kTileTwo = 0, kTileFour = 1, kTileBlock2x16 = 20, kTileOne = 25, kTileBlo
 // programs), from its cells N = nx*nz*nshots and storage.  Each line is where
 // the faster of two shapes changes, us per step of 64 replayed steps:
 //  - SH, FP32/FP64: the two-step block shapes while their workgroups (one per
-//    36 x 8 or 36 x 20 cells) fit one per CU: 256 x 128 5.3 against 7.1 (tile
-//    25) and 8.5 (tile 0), 400 x 200 6.0 / 7.2 / 8.7; past that 256 x 128 x 8
-//    10.8 / 9.0 / 9.0;
-//  - one row per thread up to 300 K cells (P-SV FP32 256 x 128 7.8 against
-//    10.2, 512 x 256 x 2 10.2 / 11.3, 1024 x 512 14.9 / 14.2), 200 K with
-//    16-bit P-SV storage, 600 K in FP64 (1024 x 512 21.5 / 23.2);
+//    36 x 8 or 36 x 20 cells) fit one per CU: 256 x 128 4.7 against 6.0 (tile
+//    25) and 7.7 (tile 0), 400 x 200 5.3 / 6.5 / 8.0; past that 256 x 128 x 8
+//    9.6 / 8.6 / 8.6;
+//  - one row per thread up to 300 K cells (P-SV FP32 256 x 128 6.9 against
+//    9.8, 512 x 256 x 2 10.0 / 11.2, 1024 x 512 14.5 / 13.4), 200 K with
+//    16-bit P-SV storage, 600 K in FP64 (1024 x 512 19.1 / 22.6);
 //  - the marching step where the five fields outgrow the 256 MB MALL, 200 MB
-//    of them (2000 x 1000 x 8 168 against 227, x 4 102 / 90; FP16 1400 x 900
-//    x 16 184 / 191), on grids mostly interior;
+//    of them (2000 x 1000 x 8 161 against 231, x 4 99 / 87; FP16 1400 x 900
+//    x 16 176 / 176), on grids mostly interior;
 //  - the SH marching step, FP32, from 3.5 M cells on grids still more
-//    interior, where it is ahead of four rows per thread by little at first
-//    (1400 x 900 x 3 34 / 36, 1024 x 512 x 16 60 / 68, 2048 x 1024 x 6 68 / 88,
-//    4096 x 2048 x 4 135 / 271; 512 x 256 x 64 69 / 66, 2000 x 1000 27 / 24);
+//    interior, where it is no faster than four rows per thread at first
+//    (1400 x 900 x 3 34 / 33, 1024 x 512 x 16 59 / 64, 2048 x 1024 x 6 68 / 82,
+//    4096 x 2048 x 4 133 / 265; 512 x 256 x 64 69 / 64, 2000 x 1000 27 / 23);
 //  - four rows per thread for large SH and 16-bit P-SV batches (SH FP64 and
-//    16-bit, 1024 x 512 x 16 69 / 75 in FP32, x 2 15.9 / 15.5; P-SV FP16 2000 x 1000 x 4 87 / 99); two
-//    rows otherwise.
+//    16-bit, 1024 x 512 x 16 64 / 69 in FP32, x 2 15.2 / 14.6; P-SV FP16 2000 x
+//    1000 x 4 85 / 90); two rows otherwise.
 static int default_tile(const fd23_desc &d) {
     const double N = (double)d.nx * d.nz * d.nshots;
     const bool psv = d.wave == FD23_WAVE_PSV, f64 = d.storage == FD23_STORE_F64;

@@ -430,7 +430,7 @@ extern "C" int fd23_ctx_create(const fd23_desc *desc, fd23_ctx **out) {
     const size_t S = d.nshots;
     // every array of the context is a part of one zeroed allocation, and the
     // chains' streams wait for their first use: with 28 allocations and four
-    // streams per context a burst of nine small requests took 26.7 ms, 20.0
+    // streams per context a burst of six small requests took 26.7 ms, 20.0
     // with one of each
     Parts parts;
     for (int f = 0; f < c->nfield; f++)

@@ -78,13 +78,15 @@ enum { kTileTwo = 0, kTileFour = 1, kTileBlock2x16 = 20, kTileOne = 25, kTileBlo
 // The shape of a context that is not tuned (the serving engine, the par-file
 // programs), from its cells N = nx*nz*nshots and storage.  Each line is where
 // the faster of two shapes changes, us per step of 64 replayed steps:
-//  - SH, FP32/FP64: the two-step block shapes while their workgroups (one per
+//  - SH, FP32: the two-step block shapes while their workgroups (one per
 //    36 x 8 or 36 x 20 cells) fit one per CU: 256 x 128 4.7 against 6.0 (tile
 //    25) and 7.7 (tile 0), 400 x 200 5.3 / 6.5 / 8.0; past that 256 x 128 x 8
-//    9.6 / 8.6 / 8.6;
+//    9.6 / 8.6 / 8.6.  Not in FP64, whose block instances spill 82 and 225
+//    registers: 256 x 128 9.8 / 6.3 / 8.5, 400 x 200 25.3 / 7.0 / 8.7;
 //  - one row per thread up to 300 K cells (P-SV FP32 256 x 128 6.9 against
-//    9.8, 512 x 256 x 2 10.0 / 11.2, 1024 x 512 14.5 / 13.4), 200 K with
-//    16-bit P-SV storage, 600 K in FP64 (1024 x 512 19.1 / 22.6);
+//    9.8, 512 x 256 x 2 10.0 / 11.2, 1024 x 512 14.5 / 13.4; SH FP64 512 x
+//    256 x 2 9.2 / 9.9, 1024 x 512 13.9 / 12.9), 200 K with 16-bit P-SV
+//    storage, 600 K in P-SV FP64 (1024 x 512 18.9 / 21.9);
 //  - the marching step where the five fields outgrow the 256 MB MALL, 200 MB
 //    of them (2000 x 1000 x 8 161 against 231, x 4 99 / 87; FP16 1400 x 900
 //    x 16 176 / 176), on grids mostly interior;
@@ -92,14 +94,16 @@ enum { kTileTwo = 0, kTileFour = 1, kTileBlock2x16 = 20, kTileOne = 25, kTileBlo
 //    interior, where it is no faster than four rows per thread at first
 //    (1400 x 900 x 3 34 / 33, 1024 x 512 x 16 59 / 64, 2048 x 1024 x 6 68 / 82,
 //    4096 x 2048 x 4 133 / 265; 512 x 256 x 64 69 / 64, 2000 x 1000 27 / 23);
-//  - four rows per thread for large SH and 16-bit P-SV batches (SH FP64 and
-//    16-bit, 1024 x 512 x 16 64 / 69 in FP32, x 2 15.2 / 14.6; P-SV FP16 2000 x
-//    1000 x 4 85 / 90); two rows otherwise.
+//  - four rows per thread for SH batches in FP32 from 2 M cells (1024 x 512 x
+//    16 64 / 69, x 2 15.2 / 14.6) and in 16 bits from 1 M (1024 x 512 x 2 16.4
+//    / 16.4, x 4 24.7 / 25.8, x 16 58.6 / 72.9), and for 16-bit P-SV batches
+//    from 5 M (2000 x 1000 x 4 85 / 90); two rows otherwise, in FP64 at any
+//    size (SH 2000 x 1000 34.0 / 37.6, 4096 x 2048 124 / 128).
 static int default_tile(const fd23_desc &d) {
     const double N = (double)d.nx * d.nz * d.nshots;
     const bool psv = d.wave == FD23_WAVE_PSV, f64 = d.storage == FD23_STORE_F64;
     const bool half = d.storage == FD23_STORE_F16 || d.storage == FD23_STORE_BF16;
-    if (!psv && !half) {
+    if (!psv && !half && !f64) {
         auto groups = [&](int ox, int oz) {
             return (double)((d.nx + ox - 1) / ox) * ((d.nz + oz - 1) / oz) * d.nshots;
         };
@@ -113,7 +117,7 @@ static int default_tile(const fd23_desc &d) {
         return half && N >= 5e6 ? kTileFour : kTileTwo;
     }
     if (!f64 && !half && N >= 3.5e6 && inner >= 0.75 * d.nx * d.nz) return kTileMarch;
-    return N >= (half ? 1e6 : 2e6) ? kTileFour : kTileTwo;
+    return !f64 && N >= (half ? 1e6 : 2e6) ? kTileFour : kTileTwo;
 }
 
 extern "C" int fd23_num_tiles(void) { return kNumTiles; }

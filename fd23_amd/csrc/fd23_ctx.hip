@@ -99,11 +99,12 @@ enum { kTileTwo = 0, kTileFour = 1, kTileBlock2x16 = 20, kTileOne = 25, kTileBlo
 //    / 16.4, x 4 24.7 / 25.8, x 16 58.6 / 72.9), and for 16-bit P-SV batches
 //    from 5 M (2000 x 1000 x 4 85 / 90); two rows otherwise, in FP64 at any
 //    size (SH 2000 x 1000 34.0 / 37.6, 4096 x 2048 124 / 128).
-static int default_tile(const fd23_desc &d) {
+// in_place: among the shapes that need no second buffer set.
+static int default_tile(const fd23_desc &d, bool in_place = false) {
     const double N = (double)d.nx * d.nz * d.nshots;
     const bool psv = d.wave == FD23_WAVE_PSV, f64 = d.storage == FD23_STORE_F64;
     const bool half = d.storage == FD23_STORE_F16 || d.storage == FD23_STORE_BF16;
-    if (!psv && !half && !f64) {
+    if (!in_place && !psv && !half && !f64) {
         auto groups = [&](int ox, int oz) {
             return (double)((d.nx + ox - 1) / ox) * ((d.nz + oz - 1) / oz) * d.nshots;
         };
@@ -113,10 +114,10 @@ static int default_tile(const fd23_desc &d) {
     if (N <= (psv && half ? 2e5 : psv && f64 ? 6e5 : 3e5)) return kTileOne;
     const double inner = std::max(0.0, d.nx - 2.0 * (d.npml + 16)) * std::max(0.0, d.nz - 1.5 * (d.npml + 16));
     if (psv) {
-        if (!f64 && 5.0 * (half ? 2 : 4) * N >= 2e8 && inner >= 0.6 * d.nx * d.nz) return kTileMarch;
+        if (!in_place && !f64 && 5.0 * (half ? 2 : 4) * N >= 2e8 && inner >= 0.6 * d.nx * d.nz) return kTileMarch;
         return half && N >= 5e6 ? kTileFour : kTileTwo;
     }
-    if (!f64 && !half && N >= 3.5e6 && inner >= 0.75 * d.nx * d.nz) return kTileMarch;
+    if (!in_place && !f64 && !half && N >= 3.5e6 && inner >= 0.75 * d.nx * d.nz) return kTileMarch;
     return !f64 && N >= (half ? 1e6 : 2e6) ? kTileFour : kTileTwo;
 }
 
@@ -250,6 +251,7 @@ struct fd23_ctx {
     void *seis = nullptr;
 
     int tile = 0;
+    bool untuned = true; // the tile is default_tile's
     // idle shot slots 0..63 (fd23_set_shot_slot): a kernel argument of the
     // graph loop's launches, so a change invalidates the captured graphs
     unsigned long long idle = 0;
@@ -1206,12 +1208,28 @@ static int ensure_alt(fd23_ctx *c) {
     for (int f = 0; f < c->nfield; f++)
         parts.add(c->alt_alloc[f], ((size_t)c->d.nshots * c->sstride + 2 * kGuard) * c->esize);
     for (int p = 0; p < c->npsi; p++) parts.add(c->alt_psi[p], psi_bytes(c, p));
-    if (hipMalloc(&c->alt_arena, parts.total) != hipSuccess) return fail(FD23_ENOMEM, "fused buffer set");
+    if (hipMalloc(&c->alt_arena, parts.total) != hipSuccess) {
+        c->alt_arena = nullptr;
+        (void)hipGetLastError(); // not the next launch's
+        return fail(FD23_ENOMEM, "fused buffer set");
+    }
     HIPCHK(hipMemsetAsync(c->alt_arena, 0, parts.total, c->stream));
     parts.place(c->alt_arena);
     for (int f = 0; f < c->nfield; f++)
         c->alt_fields[f] = (char *)c->alt_alloc[f] + (size_t)(kGuard + (long)HALO * c->px) * c->esize;
     HIPCHK(hipStreamSynchronize(c->stream));
+    return FD23_OK;
+}
+
+// The second set where the context's shape runs with one.  A context whose
+// shape nobody chose does without: where the set does not fit, it goes on with
+// the passes, in place.
+static int ensure_sets(fd23_ctx *c) {
+    if (!use_fused(c) && !use_march(c) && !use_block(c)) return FD23_OK;
+    const int r = ensure_alt(c);
+    if (r != FD23_ENOMEM || !c->untuned) return r;
+    c->tile = default_tile(c->d, true);
+    fd23_ctx_invalidate_graphs(c);
     return FD23_OK;
 }
 
@@ -2119,9 +2137,10 @@ static int run_prologue(fd23_ctx *c, int it0, int nt, int itrecord) {
     if ((c->box || c->punch) && !slots_default(c))
         return fail(FD23_EINVAL, "the box and the first-arrival window run every shot from step 0");
     if (c->box && (r = fd23_box_check_run(c, it0, nt))) return r;
+    if ((r = ensure_sets(c))) return r;
     if ((r = build_events(c))) return r;
-    if ((use_fused(c) || use_march(c)) && ((r = ensure_alt(c)) || (r = build_fused_events(c)))) return r;
-    if (use_block(c) && ((r = ensure_alt(c)) || (r = build_block_events(c)))) return r;
+    if ((use_fused(c) || use_march(c)) && (r = build_fused_events(c))) return r;
+    if (use_block(c) && (r = build_block_events(c))) return r;
     return init_scales(c);
 }
 
@@ -2267,6 +2286,7 @@ extern "C" int fd23_set_tile(fd23_ctx *c, int tile) {
         return fail(FD23_EINVAL, "the block step is SH with FP32 or FP64 storage only");
     if (tile_fused(tile) && kTiles[tile].fr == 0 && scaled_storage(c))
         return fail(FD23_EINVAL, "the tile-parallel fused step keeps FP32 or FP64 storage");
+    c->untuned = false;
     if (c->tile != tile) {
         c->tile = tile;
         fd23_ctx_invalidate_graphs(c);
@@ -2296,15 +2316,14 @@ extern "C" int fd23_time_passes(fd23_ctx *c, int nsteps, double *stress_ms, doub
     int r = ready(c);
     if (r) return r;
     if (nsteps < 1 || nsteps > 4096) return fail(FD23_EINVAL, "nsteps must be in [1, 4096]");
+    if ((r = ensure_sets(c))) return r;
+    const bool sc = scaled_storage(c);
+    const bool fused = use_fused(c), block = use_block(c), march = use_march(c);
+    if (fused && (r = build_fused_events(c))) return r;
     hipEvent_t e0, e1, e2;
     HIPCHK(hipEventCreate(&e0));
     HIPCHK(hipEventCreate(&e1));
     HIPCHK(hipEventCreate(&e2));
-    const bool sc = scaled_storage(c);
-    const bool fused = use_fused(c), block = use_block(c), march = use_march(c);
-    if (march && (r = ensure_alt(c))) return r;
-    if (fused && ((r = ensure_alt(c)) || (r = build_fused_events(c)))) return r;
-    if (block && (r = ensure_alt(c))) return r;
     if (block) {
         // nsteps block launches of bk steps back to back (no sources or
         // receivers): the first value is the time per step, the second 0
@@ -2418,7 +2437,10 @@ extern "C" int fd23_autotune(fd23_ctx *c, int steps, double *best_ms) {
     std::vector<size_t> sizes;
     auto snap = [&](void *p, size_t n) -> int {
         void *q = nullptr;
-        if (hipMalloc(&q, n) != hipSuccess) return fail(FD23_ENOMEM, "autotune snapshot");
+        if (hipMalloc(&q, n) != hipSuccess) {
+            (void)hipGetLastError();
+            return fail(FD23_ENOMEM, "autotune snapshot");
+        }
         hipMemcpyAsync(q, p, n, hipMemcpyDeviceToDevice, c->stream);
         saved.push_back(q);
         sizes.push_back(n);
@@ -2440,6 +2462,8 @@ extern "C" int fd23_autotune(fd23_ctx *c, int steps, double *best_ms) {
     HIPCHK(hipMemcpy(scl_saved, c->scl, sizeof scl_saved, hipMemcpyDeviceToHost));
     HIPCHK(hipMemcpy(amax_saved.data(), c->amax, sizeof(unsigned) * amax_saved.size(), hipMemcpyDeviceToHost));
     const int orig = c->tile, orig_set = c->cur;
+    const bool untuned = c->untuned;
+    c->untuned = false; // the candidates run as they are
     int best = orig;
     double bt = 1e30;
     std::vector<std::pair<double, int>> timed; // pass time, shape
@@ -2519,6 +2543,7 @@ extern "C" int fd23_autotune(fd23_ctx *c, int steps, double *best_ms) {
     hipStreamSynchronize(c->stream);
     for (auto p : saved) hipFree(p);
     c->tile = orig;
+    c->untuned = untuned;
     if (r) return r;
     fd23_set_tile(c, best);
     if (best_ms) *best_ms = bt;

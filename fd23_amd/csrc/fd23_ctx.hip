@@ -1097,7 +1097,7 @@ static int build_fused_events(fd23_ctx *c) {
                 if (x < x0 || x >= x1 || z < z0 || z >= z1) continue;
                 const int st = (x - x0) / own, sg = (z - z0) / H;
                 rb[((size_t)sg * nstrip + st) * S + s].push_back(
-                    RecF{z, x - x0 - st * own + halo, comp, (int)(base + r)});
+                    RecF{z, x - x0 - st * own + halo, comp, (int)(base + r), 0, kNoRow});
             }
         }
     }
@@ -1113,10 +1113,15 @@ static int build_fused_events(fd23_ctx *c) {
         std::stable_sort(rb[k].begin(), rb[k].end(), [](const RecF &a, const RecF &b) { return a.row < b.row; });
         rs[k] = (int)recs.size();
         recs.insert(recs.end(), rb[k].begin(), rb[k].end());
+        for (int e = (int)recs.size() - 1, end = e + 1; e >= rs[k]; e--) {
+            if (e + 1 < (int)recs.size() && recs[e + 1].row != recs[e].row) end = e + 1;
+            recs[e].next = end;
+            if (end < (int)recs.size()) recs[e].nextrow = recs[end].row;
+        }
     }
     rs[rb.size()] = (int)recs.size();
     if (taps.empty()) taps.push_back(TapF{-1, -1, 0, 0, 0.0, 0.0});
-    if (recs.empty()) recs.push_back(RecF{-1, -1, 0, 0});
+    if (recs.empty()) recs.push_back(RecF{-1, -1, 0, 0, 0, kNoRow});
     int r;
     if ((r = upload_vec(c, c->d_ftap_start, c->ftap_start_cap, ts))) return r;
     if ((r = upload_vec(c, c->d_frec_start, c->frec_start_cap, rs))) return r;

@@ -33,7 +33,13 @@ struct TapF {                      // a source tap seen by one strip
 };
 struct RecF {                      // a receiver inside one (segment, strip)
     int row, lane, comp, out;
+    // the list entry behind its row's last, and that one's row (or kNoRow): a
+    // row's end found by reading on, entry after entry, held a line of 3000
+    // receivers up by 80 us (P-SV, 2 shots of 3000 x 1800 187 us a step, 145
+    // so; SH, one shot 61 and 40)
+    int next, nextrow;
 };
+constexpr int kNoRow = -(1 << 30); // below every row an iteration computes
 struct FusedEvents {
     const int *clock;              // step = clock[0] + k
     int k, itrecord;

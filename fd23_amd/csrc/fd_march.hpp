@@ -116,7 +116,18 @@ __device__ __forceinline__ void store2(BufRsrc r, unsigned vo, unsigned so, cons
     }
 }
 
-constexpr int kNoRow = -(1 << 30); // below every row an iteration computes
+// a list read at a uniform index, through the scalar cache: a vector load
+// there would wait for the rows loaded ahead
+template <class T> __device__ __forceinline__ const __attribute__((address_space(4))) T *uniform(const T *p) {
+    return (const __attribute__((address_space(4))) T *)p;
+}
+__device__ __forceinline__ RecF uniform_rec(const RecF *p, int e) {
+    const auto *r = uniform(p) + e;
+    return RecF{r->row, r->lane, r->comp, r->out, r->next, r->nextrow};
+}
+// receivers of a row that are not worth two barriers and a vector load (a
+// borehole's one per row: SH, 2 shots of 2000 x 1000 40 us a step, 46 with)
+constexpr int kFewRecs = 4;
 
 // a work item, and what happens in it: source taps [t0, t1) of rows
 // trow0..trow1, active in the first (onA) or second step (onB); receivers
@@ -189,23 +200,32 @@ __device__ __forceinline__ void march_item(const PsvFields<S> &fa, const PsvFiel
         }
     };
     auto record = [&](int step, int &r, const C (&u)[NC], const C (&ww)[NC]) -> int {
-        const int row = ev.recs[r].row;
+        const int e0 = r;
+        RecF rc = uniform_rec(ev.recs, e0);
+        const int e1 = rc.next, row = rc.nextrow;
+        r = e1;
+        C *seis = (C *)ev.seis + (long)(step / ev.itrecord) * ev.frame_size;
+        if (e1 - e0 <= kFewRecs) { // straight from the registers of the columns' threads
+            for (int e = e0;;) {
+#pragma unroll
+                for (int i = 0; i < NC; i++)
+                    if (rc.lane == lc + i) seis[rc.out] = rc.comp == 0 ? u[i] : ww[i];
+                if (++e >= e1) return row;
+                rc = uniform_rec(ev.recs, e);
+            }
+        }
 #pragma unroll
         for (int i = 0; i < NC; i++) {
             l.park[0][lc + i] = u[i];
             l.park[1][lc + i] = ww[i];
         }
         __syncthreads();
-        int e1 = r;
-        while (e1 < q.r1 && ev.recs[e1].row == row) e1++;
-        C *seis = (C *)ev.seis + (long)(step / ev.itrecord) * ev.frame_size;
-        for (int e = r + (int)threadIdx.x; e < e1; e += MT) {
+        for (int e = e0 + (int)threadIdx.x; e < e1; e += MT) {
             const RecF rc = ev.recs[e];
             seis[rc.out] = l.park[rc.comp == 0 ? 0 : 1][rc.lane];
         }
         __syncthreads();
-        r = e1;
-        return r < q.r1 ? ev.recs[r].row : kNoRow;
+        return row;
     };
 
     int rA = q.r, rB = q.r, nextA = q.nextA, nextB = q.nextB;
@@ -452,7 +472,7 @@ __device__ __forceinline__ bool march_find(const Grid &g, const MarchWork &w, co
         q.ts = it - si.t0;
         auto recorded = [&](int t) { return t >= 0 && t % ev.itrecord == 0 && t / ev.itrecord < ev.max_frames; };
         if (q.r < q.r1) {
-            const int row = ev.recs[q.r].row;
+            const int row = uniform(ev.recs)[q.r].row;
             q.nextA = recorded(q.ts) ? row : kNoRow;
             q.nextB = recorded(q.ts + 1) ? row : kNoRow;
         }

@@ -59,20 +59,29 @@ __device__ __forceinline__ void sh_march_item(const ShFields<float> &fa, const S
         }
     };
     auto record = [&](int step, int &r, const C (&v)[NC]) -> int {
-        const int row = ev.recs[r].row;
+        const int e0 = r;
+        RecF rc = uniform_rec(ev.recs, e0);
+        const int e1 = rc.next, row = rc.nextrow;
+        r = e1;
+        C *seis = (C *)ev.seis + (long)(step / ev.itrecord) * ev.frame_size;
+        if (e1 - e0 <= kFewRecs) {
+            for (int e = e0;;) {
+#pragma unroll
+                for (int i = 0; i < NC; i++)
+                    if (rc.lane == lc + i) seis[rc.out] = v[i];
+                if (++e >= e1) return row;
+                rc = uniform_rec(ev.recs, e);
+            }
+        }
 #pragma unroll
         for (int i = 0; i < NC; i++) l.park[lc + i] = v[i];
         __syncthreads();
-        int e1 = r;
-        while (e1 < q.r1 && ev.recs[e1].row == row) e1++;
-        C *seis = (C *)ev.seis + (long)(step / ev.itrecord) * ev.frame_size;
-        for (int e = r + (int)threadIdx.x; e < e1; e += MT) {
+        for (int e = e0 + (int)threadIdx.x; e < e1; e += MT) {
             const RecF rc = ev.recs[e];
             seis[rc.out] = l.park[rc.lane];
         }
         __syncthreads();
-        r = e1;
-        return r < q.r1 ? ev.recs[r].row : kNoRow;
+        return row;
     };
 
     int rA = q.r, rB = q.r, nextA = q.nextA, nextB = q.nextB;

@@ -188,14 +188,19 @@ __device__ __forceinline__ void march_item(const PsvFields<S> &fa, const PsvFiel
 
     auto inject = [&](int row, double sv, C (&a)[NC], C (&b)[NC], C (&c)[NC]) {
         for (int e = q.t0; e < q.t1; e++) {
-            const TapF tp = ev.taps[e];
-            if (tp.row != row) continue;
+            const auto *t = uniform(ev.taps) + e;
+            if (t->row != row) continue;
+            const TapF tp{t->row, t->lane, t->field, t->mode, t->m, t->q};
 #pragma unroll
             for (int i = 0; i < NC; i++) {
-                if (tp.lane != lc + i) continue;
-                if (tp.field == 2) a[i] = apply_tap(a[i], tp, sv);
-                else if (tp.field == 3) b[i] = apply_tap(b[i], tp, sv);
-                else c[i] = apply_tap(c[i], tp, sv);
+                // selects: with a branch per field the compiler takes the address
+                // of the one that is changed, and all three live in scratch memory,
+                // whose reloads wait for the rows ahead (2 shots of 3000 x 1800
+                // with a source at mid-depth 143 us a step, 113 so, 106 without)
+                const bool mine = tp.lane == lc + i;
+                a[i] = mine && tp.field == 2 ? apply_tap(a[i], tp, sv) : a[i];
+                b[i] = mine && tp.field == 3 ? apply_tap(b[i], tp, sv) : b[i];
+                c[i] = mine && tp.field == 4 ? apply_tap(c[i], tp, sv) : c[i];
             }
         }
     };
@@ -460,10 +465,11 @@ __device__ __forceinline__ bool march_find(const Grid &g, const MarchWork &w, co
         if (q.t1 > q.t0) {
             q.onA = src_sample(si, ev.stf, it, q.svA);
             q.onB = src_sample(si, ev.stf, it + 1, q.svB);
-            q.trow0 = q.trow1 = ev.taps[q.t0].row;
+            q.trow0 = q.trow1 = uniform(ev.taps)[q.t0].row;
             for (int e = q.t0 + 1; e < q.t1; e++) {
-                q.trow0 = min(q.trow0, ev.taps[e].row);
-                q.trow1 = max(q.trow1, ev.taps[e].row);
+                const int row = uniform(ev.taps)[e].row;
+                q.trow0 = min(q.trow0, row);
+                q.trow1 = max(q.trow1, row);
             }
         }
         const int rkey = (seg * w.nstrip + q.strip) * g.nshots + q.shot;

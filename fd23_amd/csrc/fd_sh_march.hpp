@@ -51,8 +51,9 @@ __device__ __forceinline__ void sh_march_item(const ShFields<float> &fa, const S
 
     auto inject = [&](int row, double sv, int field, C (&a)[NC]) {
         for (int e = q.t0; e < q.t1; e++) {
-            const TapF tp = ev.taps[e];
-            if (tp.row != row || tp.field != field) continue;
+            const auto *t = uniform(ev.taps) + e;
+            if (t->row != row || t->field != field) continue;
+            const TapF tp{t->row, t->lane, t->field, t->mode, t->m, t->q};
 #pragma unroll
             for (int i = 0; i < NC; i++)
                 if (tp.lane == lc + i) a[i] = apply_tap(a[i], tp, sv);

@@ -46,3 +46,12 @@ def test_receiver_line_at_depth(wave, shots, bound):
     deep = seconds(wave, nx, nz, shots, _lib.STORE_F32, 8, nz // 2)
     print("receiver line at depth", deep / near, flush=True)
     assert deep < bound * near
+
+
+# stresses in scratch memory: 1.37 times
+def test_source_at_depth():
+    nx, nz = 3000, 1800
+    near = seconds(_lib.WAVE_PSV, nx, nz, 2, _lib.STORE_F32, 8, 4)
+    deep = seconds(_lib.WAVE_PSV, nx, nz, 2, _lib.STORE_F32, nz // 2, 4)
+    print("source at depth", deep / near, flush=True)
+    assert deep < 1.22 * near

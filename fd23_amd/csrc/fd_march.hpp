@@ -498,10 +498,16 @@ __global__ __launch_bounds__(MW / NC, 2) void k_psv_march(PsvFields<S> fa, PsvFi
     if (L >= w.nwork) return;
     MarchItem q;
     const bool checked = march_find<MW>(g, w, ev, L, q);
-    // amax is null on steps that no scale check follows
-    if (checked)
+    // amax is null on steps that no scale check follows, three launches
+    // of four: they run the bodies without the maxima, whose checked
+    // one spills 40 registers in 16 bits (FP16, 4 shots of 3000 x 1800 with
+    // sources at mid-depth 246 us a step, 198 so)
+    const bool track = Store<S>::scaled && amax;
+    if (checked && track)
         march_item<S, MW, true, Store<S>::scaled>(fa, fb, m, g, w, ev, sa, scl, amax, q, l);
-    else if (Store<S>::scaled && amax)
+    else if (checked)
+        march_item<S, MW, true, false>(fa, fb, m, g, w, ev, sa, scl, amax, q, l);
+    else if (track)
         march_item<S, MW, false, Store<S>::scaled>(fa, fb, m, g, w, ev, sa, scl, amax, q, l);
     else
         march_item<S, MW, false, false>(fa, fb, m, g, w, ev, sa, scl, amax, q, l);

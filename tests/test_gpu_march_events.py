@@ -55,3 +55,13 @@ def test_source_at_depth():
     deep = seconds(_lib.WAVE_PSV, nx, nz, 2, _lib.STORE_F32, nz // 2, 4)
     print("source at depth", deep / near, flush=True)
     assert deep < 1.22 * near
+
+
+# maxima gathered on every step: 1.52 and 1.49 times
+@pytest.mark.parametrize("storage", [_lib.STORE_F16, _lib.STORE_BF16])
+def test_source_at_depth_in_16_bits(storage):
+    nx, nz = 3000, 1800
+    near = seconds(_lib.WAVE_PSV, nx, nz, 4, storage, 8, 4)
+    deep = seconds(_lib.WAVE_PSV, nx, nz, 4, storage, nz // 2, 4)
+    print("source at depth", storage, deep / near, flush=True)
+    assert deep < 1.38 * near

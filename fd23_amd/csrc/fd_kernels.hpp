@@ -234,12 +234,22 @@ template <class C, class T> __device__ __forceinline__ C apply_tap(C v, const T 
 // memory latency ahead of the fields (us a step: P-SV 301 x 223 7.8, 7.6
 // behind them; 2000 x 1000 32.6 and 31.3; 64 shots of 1024 x 512 492 and 475;
 // SH 6 shots of 2048 x 1024 96 and 92).
+//
+// Not where several shots of four rows each leave no register for them: in
+// P-SV with 16- or 64-bit storage, and SH in FP64 with four shots or more, the
+// heads ahead of the barrier cost one of three wavefronts per SIMD (4 shots of
+// 1400 x 900, us a step: FP16 2 shots per workgroup 102, 90 behind it, 4 shots
+// 113 and 101; FP64 155 / 146 and 166 / 161; SH FP64 4 shots 94 / 88).
+template <class S, int RZ, int SPB, bool WHOLE, bool PSV> constexpr bool late_heads() {
+    return WHOLE && RZ == 4 && (PSV ? SPB > 1 && sizeof(S) != 4 : SPB > 2 && sizeof(S) == 8);
+}
 struct ListHeads {
     int it, tap0, tap1, rec0, rec1, t0;
 };
+template <bool BEHIND = true>
 __device__ __forceinline__ ListHeads list_heads(const Events &ev, int key, int shot, bool rec) {
     ListHeads h{};
-    __builtin_amdgcn_sched_barrier(0);
+    if (BEHIND) __builtin_amdgcn_sched_barrier(0);
     if (ev.clock) {
         h.it = ev.clock[0] + ev.k;
         h.tap0 = ev.tap_start[key];
@@ -463,7 +473,9 @@ __global__ __launch_bounds__(TX *BY) void k_psv_stress(PsvFields<S> f, PsvStress
     bool interior = REGION == REGION_INTERIOR  ? true
                     : REGION == REGION_EDGE    ? false
                                                : tile_interior(g, x0, z0, TZ);
-    int it = 0; // set with the list heads below; a window needs it first
+    constexpr bool kLate = late_heads<S, RZ, SPB, REGION == REGION_ALL && !TO, true>();
+    // set with the list heads below; a window needs it first
+    int it = kLate && ev.clock ? ev.clock[0] + ev.k : 0;
     // first-arrival window: the interior-only kernel is never launched with
     // one; a tile with a closed block takes the exact path, which masks rows
     const bool pun = REGION != REGION_INTERIOR && punch_on(g, ev); // uniform
@@ -508,9 +520,10 @@ __global__ __launch_bounds__(TX *BY) void k_psv_stress(PsvFields<S> f, PsvStress
 #pragma unroll
     for (int r = 0; r < RZ; r++) {
         const unsigned so = (unsigned)min(z0 + lz0 + r, nz - 1) * pxm;
-        lam[r] = Store<C>::ldb(rLAM, vmat, so, 1.f);
-        mu[r] = Store<C>::ldb(rMU, vmat, so, 1.f);
-        mua[r] = Store<C>::ldb(rMUA, vmat, so, 1.f);
+        const bool live = !kLate || (gx < nx && z0 + lz0 + r < nz);
+        lam[r] = live ? Store<C>::ldb(rLAM, vmat, so, 1.f) : C(0);
+        mu[r] = live ? Store<C>::ldb(rMU, vmat, so, 1.f) : C(0);
+        mua[r] = live ? Store<C>::ldb(rMUA, vmat, so, 1.f) : C(0);
     }
 
     const int sh0 = t.group * SPB;
@@ -573,8 +586,11 @@ __global__ __launch_bounds__(TX *BY) void k_psv_stress(PsvFields<S> f, PsvStress
                 zv[r][1] = pml_coef(pr.Uz, iz, inz);
             }
         }
-        const ListHeads h = list_heads(ev, t.tile * g.nshots + shot, shot, false);
-        it = h.it;
+        ListHeads h{};
+        if (!kLate) {
+            h = list_heads(ev, t.tile * g.nshots + shot, shot, false);
+            it = h.it;
+        }
         if (s > 0) __syncthreads();
         rU.store(sU);
         rW.store(sW);
@@ -619,6 +635,7 @@ __global__ __launch_bounds__(TX *BY) void k_psv_stress(PsvFields<S> f, PsvStress
         // fused source injection: the owner of a tap cell adds it after the
         // cell's own update, taps in the reference's order
         if (ev.clock) {
+            if (kLate) h = list_heads<false>(ev, t.tile * g.nshots + shot, shot, false);
             double sv;
             if (h.tap1 > h.tap0 && src_sample(ev.src[shot], ev.stf, it, sv)) {
                 for (int e = h.tap0; e < h.tap1; e++) {
@@ -789,7 +806,9 @@ __global__ __launch_bounds__(TX *BY) void k_psv_velocity(PsvFields<S> f, PsvVelM
     bool interior = REGION == REGION_INTERIOR  ? true
                     : REGION == REGION_EDGE    ? false
                                                : tile_interior(g, x0, z0, TZ);
-    int it = 0; // set with the list heads below; a window needs it first
+    constexpr bool kLate = late_heads<S, RZ, SPB, REGION == REGION_ALL && !TO, true>();
+    // set with the list heads below; a window needs it first
+    int it = kLate && ev.clock ? ev.clock[0] + ev.k : 0;
     // first-arrival window: the interior-only kernel is never launched with
     // one; a tile with a closed block takes the exact path, which masks rows
     const bool pun = REGION != REGION_INTERIOR && punch_on(g, ev); // uniform
@@ -828,8 +847,9 @@ __global__ __launch_bounds__(TX *BY) void k_psv_velocity(PsvFields<S> f, PsvVelM
 #pragma unroll
     for (int r = 0; r < RZ; r++) {
         const unsigned so = (unsigned)min(z0 + lz0 + r, nz - 1) * pxm;
-        bu[r] = Store<C>::ldb(rBU, vmat, so, 1.f);
-        bw[r] = Store<C>::ldb(rBW, vmat, so, 1.f);
+        const bool live = !kLate || (gx < nx && z0 + lz0 + r < nz);
+        bu[r] = live ? Store<C>::ldb(rBU, vmat, so, 1.f) : C(0);
+        bw[r] = live ? Store<C>::ldb(rBW, vmat, so, 1.f) : C(0);
     }
 
     const int sh0 = t.group * SPB;
@@ -893,8 +913,11 @@ __global__ __launch_bounds__(TX *BY) void k_psv_velocity(PsvFields<S> f, PsvVelM
                 zv[r][1] = pml_coef(pr.Tzz_z, iz, inz);
             }
         }
-        const ListHeads h = list_heads(ev, t.tile * g.nshots + shot, shot, true);
-        it = h.it;
+        ListHeads h{};
+        if (!kLate) {
+            h = list_heads(ev, t.tile * g.nshots + shot, shot, true);
+            it = h.it;
+        }
         if (s > 0) __syncthreads();
         rXX.store(sXX);
         rZZ.store(sZZ);
@@ -947,8 +970,10 @@ __global__ __launch_bounds__(TX *BY) void k_psv_velocity(PsvFields<S> f, PsvVelM
                 mx_w = fmaxf(mx_w, fabsf((float)nv[1][r]));
             }
         }
-        if (ev.clock)
+        if (ev.clock) {
+            if (kLate) h = list_heads<false>(ev, t.tile * g.nshots + shot, shot, true);
             fused_record<C, RZ, 2, TO>(ev, h, sXX, sZZ, nv, lz0, w, x0, z0);
+        }
     }
     if (ST::scaled) {
         amax_update(amax, SC_U, mx_u);
@@ -1007,7 +1032,9 @@ __global__ __launch_bounds__(TX *BY) void k_sh_stress(ShFields<S> f, ShStressMat
     const int gx = x0 + tx;
     const int lz0 = ty * RZ;
     bool interior = tile_interior(g, x0, z0, TZ);
-    int it = 0; // set with the list heads below; a window needs it first
+    constexpr bool kLate = late_heads<S, RZ, SPB, !TO, false>();
+    // set with the list heads below; a window needs it first
+    int it = kLate && ev.clock ? ev.clock[0] + ev.k : 0;
     // first-arrival window: a tile with a closed block takes the exact
     // path, which masks rows
     const bool pun = punch_on(g, ev); // uniform
@@ -1037,8 +1064,9 @@ __global__ __launch_bounds__(TX *BY) void k_sh_stress(ShFields<S> f, ShStressMat
 #pragma unroll
     for (int r = 0; r < RZ; r++) {
         const unsigned so = (unsigned)min(z0 + lz0 + r, nz - 1) * pxm;
-        mux[r] = Store<C>::ldb(rMUX, vmat, so, 1.f);
-        muz[r] = Store<C>::ldb(rMUZ, vmat, so, 1.f);
+        const bool live = !kLate || (gx < nx && z0 + lz0 + r < nz);
+        mux[r] = live ? Store<C>::ldb(rMUX, vmat, so, 1.f) : C(0);
+        muz[r] = live ? Store<C>::ldb(rMUZ, vmat, so, 1.f) : C(0);
     }
 
     const int sh0 = t.group * SPB;
@@ -1088,8 +1116,11 @@ __global__ __launch_bounds__(TX *BY) void k_sh_stress(ShFields<S> f, ShStressMat
                 zv[r][0] = pml_coef(pr.z, iz, inz);
             }
         }
-        const ListHeads h = list_heads(ev, t.tile * g.nshots + shot, shot, false);
-        it = h.it;
+        ListHeads h{};
+        if (!kLate) {
+            h = list_heads(ev, t.tile * g.nshots + shot, shot, false);
+            it = h.it;
+        }
         if (s > 0) __syncthreads();
         rV.store(sV);
         __syncthreads();
@@ -1147,6 +1178,7 @@ __global__ __launch_bounds__(TX *BY) void k_sh_stress(ShFields<S> f, ShStressMat
         // fused SH source, stress taps (Tx, Tz); a point force on V is added
         // by the velocity pass, which is the only pass that writes V
         if (ev.clock) {
+            if (kLate) h = list_heads<false>(ev, t.tile * g.nshots + shot, shot, false);
             double sv;
             if (h.tap1 > h.tap0 && src_sample(ev.src[shot], ev.stf, it, sv)) {
                 for (int e = h.tap0; e < h.tap1; e++) {
@@ -1214,7 +1246,9 @@ __global__ __launch_bounds__(TX *BY) void k_sh_velocity(ShFields<S> f, const typ
     const int gx = x0 + tx;
     const int lz0 = ty * RZ;
     bool interior = tile_interior(g, x0, z0, TZ);
-    int it = 0; // set with the list heads below; a window needs it first
+    constexpr bool kLate = late_heads<S, RZ, SPB, !TO, false>();
+    // set with the list heads below; a window needs it first
+    int it = kLate && ev.clock ? ev.clock[0] + ev.k : 0;
     // first-arrival window: a tile with a closed block takes the exact
     // path, which masks rows
     const bool pun = punch_on(g, ev); // uniform
@@ -1245,7 +1279,8 @@ __global__ __launch_bounds__(TX *BY) void k_sh_velocity(ShFields<S> f, const typ
     C bv[RZ];
 #pragma unroll
     for (int r = 0; r < RZ; r++) {
-        bv[r] = Store<C>::ldb(rBV, vmat, (unsigned)min(z0 + lz0 + r, nz - 1) * pxm, 1.f);
+        const bool live = !kLate || (gx < nx && z0 + lz0 + r < nz);
+        bv[r] = live ? Store<C>::ldb(rBV, vmat, (unsigned)min(z0 + lz0 + r, nz - 1) * pxm, 1.f) : C(0);
     }
 
     const int sh0 = t.group * SPB;
@@ -1301,8 +1336,11 @@ __global__ __launch_bounds__(TX *BY) void k_sh_velocity(ShFields<S> f, const typ
                 zv[r][0] = pml_coef(pr.z, iz, inz);
             }
         }
-        const ListHeads h = list_heads(ev, t.tile * g.nshots + shot, shot, true);
-        it = h.it;
+        ListHeads h{};
+        if (!kLate) {
+            h = list_heads(ev, t.tile * g.nshots + shot, shot, true);
+            it = h.it;
+        }
         if (s > 0) __syncthreads();
         rX.store(sX);
         rZ.store(sZ);
@@ -1317,6 +1355,7 @@ __global__ __launch_bounds__(TX *BY) void k_sh_velocity(ShFields<S> f, const typ
         // fused SH point force (cu_point_force): V += source before the
         // cell's velocity update, as the reference injects between passes
         if (ev.clock) {
+            if (kLate) h = list_heads<false>(ev, t.tile * g.nshots + shot, shot, false);
             double sv;
             if (h.tap1 > h.tap0 && src_sample(ev.src[shot], ev.stf, it, sv)) {
                 for (int e = h.tap0; e < h.tap1; e++) {
@@ -1388,7 +1427,10 @@ __global__ __launch_bounds__(TX *BY) void k_sh_velocity(ShFields<S> f, const typ
             ST::stb(oV, vcol, (unsigned)(gz + HALO) * pxb, nv[0][r], wi_v);
             if (ST::scaled && amax) mx_v = fmaxf(mx_v, fabsf((float)nv[0][r]));
         }
-        if (ev.clock) fused_record<C, RZ, 1, TO>(ev, h, sX, sX, nv, lz0, w, x0, z0);
+        if (ev.clock) {
+            if (kLate) h = list_heads<false>(ev, t.tile * g.nshots + shot, shot, true);
+            fused_record<C, RZ, 1, TO>(ev, h, sX, sX, nv, lz0, w, x0, z0);
+        }
     }
     if (ST::scaled) {
         amax_update(amax, SC_V, mx_v);

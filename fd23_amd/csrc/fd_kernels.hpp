@@ -1018,7 +1018,7 @@ __global__ __launch_bounds__(TX *BY) void k_sh_stress(ShFields<S> f, ShStressMat
     }
     using C = typename Store<S>::C;
     using ST = Store<S>;
-    constexpr bool kPrePsi = TO || (RZ == 1 && !ST::scaled);
+    constexpr bool kPrePsi = TO || (RZ == 1 && sizeof(S) == 8);
     constexpr int TZ = BY * RZ;
     constexpr int LW = TX + 2 * HALO;
     __shared__ C sV[(TZ + 2 * HALO) * LW];
@@ -1087,7 +1087,9 @@ __global__ __launch_bounds__(TX *BY) void k_sh_stress(ShFields<S> f, ShStressMat
             vx[r] = ST::ldb(bX, vcol, so, sc_x);
             vz[r] = ST::ldb(bZ, vcol, so, sc_z);
         }
-        // this shot's C-PML memory variables, ahead of the barrier
+        // this shot's C-PML memory variables, ahead of the barrier (of whole grids
+        // with one row per thread in FP64 only: 256 x 128 7.0 -> 6.3 us a step; in
+        // FP32 the registers cost 4 shots of 1400 x 900 62 -> 72)
         C pq[2][kPrePsi ? RZ : 1];
         if (kPrePsi && !interior) {
 #pragma unroll
@@ -1231,7 +1233,7 @@ __global__ __launch_bounds__(TX *BY) void k_sh_velocity(ShFields<S> f, const typ
     }
     using C = typename Store<S>::C;
     using ST = Store<S>;
-    constexpr bool kPrePsi = TO || (RZ == 1 && !ST::scaled);
+    constexpr bool kPrePsi = TO || (RZ == 1 && sizeof(S) == 8);
     constexpr int TZ = BY * RZ;
     constexpr int LW = TX + 2 * HALO;
     __shared__ C sX[(TZ + 2 * HALO) * LW];

@@ -67,3 +67,10 @@ def test_passes_of_several_shots_keep_three_wavefronts():
     got.update(instances(r"k_sh_(stress|velocity)IdLi4ELi[48]E"))
     for n, k in got.items():
         assert k[".vgpr_count"] <= 168, (n, k[".vgpr_count"])
+
+
+def test_one_row_sh_passes_stay_small():
+    """One row per thread in FP32, bound by memory on large grids: no registers
+    for values loaded ahead (33 without, 38 with them)."""
+    for n, k in instances(r"k_sh_(stress|velocity)IfLi1ELi1E").items():
+        assert k[".vgpr_count"] <= 33, (n, k[".vgpr_count"])

@@ -262,8 +262,10 @@ struct fd23_ctx {
     struct Chunk {
         hipGraphExec_t exec;
         bool flips;
+        long used; // the context's count of uses at the last one
     };
     std::map<std::tuple<int, int, int>, Chunk> graphs;
+    long uses = 0;
     // a buffer that captured launches name has moved, or what they hold by
     // value has changed: they are captured again
     bool stale = false;
@@ -2072,15 +2074,35 @@ static int ensure_chains(fd23_ctx *c) {
     return FD23_OK;
 }
 
+// Runs of ever new lengths don't pile graphs up: at kMaxGraphs the half not
+// used for longest goes.  A run needs four at most, so those it has just
+// replayed, and those that fd23_prepare has just captured for it, stay.
+static const size_t kMaxGraphs = 16;
+static void drop_old_graphs(fd23_ctx *c) {
+    std::vector<long> used;
+    for (auto &kv : c->graphs) used.push_back(kv.second.used);
+    std::nth_element(used.begin(), used.begin() + kMaxGraphs / 2, used.end());
+    const long keep = used[kMaxGraphs / 2];
+    hipStreamSynchronize(c->stream); // a replay may still run
+    for (auto it = c->graphs.begin(); it != c->graphs.end();) {
+        if (it->second.used >= keep) {
+            ++it;
+            continue;
+        }
+        hipGraphExecDestroy(it->second.exec);
+        it = c->graphs.erase(it);
+    }
+}
+
 static int get_graph(fd23_ctx *c, int itrecord, int steps, fd23_ctx::Chunk *out) {
     const auto key = std::make_tuple(itrecord, steps, c->cur);
     auto it = c->graphs.find(key);
     if (it != c->graphs.end()) {
+        it->second.used = ++c->uses;
         *out = it->second;
         return FD23_OK;
     }
-    // a run needs four at most; runs of ever new lengths don't pile them up
-    if (c->graphs.size() >= 16) fd23_ctx_invalidate_graphs(c);
+    if (c->graphs.size() >= kMaxGraphs) drop_old_graphs(c);
     const int cur0 = c->cur;
     hipGraph_t graph;
     if (use_chains(c)) {
@@ -2121,7 +2143,7 @@ static int get_graph(fd23_ctx *c, int itrecord, int steps, fd23_ctx::Chunk *out)
     e = hipGraphInstantiate(&exec, graph, nullptr, nullptr, 0);
     hipGraphDestroy(graph);
     if (e != hipSuccess) return fail(FD23_EHIP, "graph instantiate: %s", hipGetErrorString(e));
-    c->graphs[key] = fd23_ctx::Chunk{exec, flips};
+    c->graphs[key] = fd23_ctx::Chunk{exec, flips, ++c->uses};
     *out = c->graphs[key];
     return FD23_OK;
 }

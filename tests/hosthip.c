@@ -9,7 +9,7 @@ typedef struct {
 } dim3_;
 
 long hh_room = 1L << 40;   /* bytes hipMalloc may still give */
-long hh_graphs, hh_launches, hh_mallocs, hh_copied;
+long hh_graphs, hh_held, hh_launches, hh_mallocs, hh_copied;
 int hh_error;              /* the error hipGetLastError returns next */
 
 static int failed(int e) {
@@ -98,10 +98,11 @@ int hipStreamEndCapture(void *s, void **g) { return (void)s, made(g); }
 int hipGraphInstantiate(void **x, void *g, void *n, char *l, size_t b) {
     (void)g, (void)n, (void)l, (void)b;
     hh_graphs++;
+    hh_held++;
     return made(x);
 }
 int hipGraphDestroy(void *g) { return (void)g, 0; }
-int hipGraphExecDestroy(void *x) { return (void)x, 0; }
+int hipGraphExecDestroy(void *x) { return (void)x, hh_held--, 0; }
 int hipGraphLaunch(void *x, void *s) { return (void)x, (void)s, 0; }
 int hipEventCreate(void **e) { return made(e); }
 int hipEventCreateWithFlags(void **e, unsigned f) { return (void)f, made(e); }

@@ -65,6 +65,16 @@ def block_bytes(wl, k):
     return S * (6 * wf * N + 4 * wf * (nxp + nzp)) + 3 * wf * N
 
 
+def march_bytes(wl):
+    """Algorithmic bytes of one marching launch: the state read once and written
+    once, the material read once (None where no marching step exists)."""
+    from fd23_amd import _lib
+
+    if wl.wave == _lib.WAVE_PSV:
+        return fused_bytes(wl) if wl.storage != _lib.STORE_F64 else None
+    return block_bytes(wl, 2) if wl.storage == _lib.STORE_F32 else None
+
+
 def pass_bytes(wl, ctx_bytes_per_step=None):
     """Algorithmic bytes of the stress and velocity passes of one step."""
     from fd23_amd import _lib
@@ -121,12 +131,15 @@ def run_gpu(wl, steps, warmup, autotune=True, tile=None, passes=True, chains=Non
     seis = ctx.seismograms(0, 0, warmup + steps)
     finite = bool(np.isfinite(seis).all())
     kind = ctx.tile_kind()
-    fused = kind == _lib.TILE_FUSED and wl.wave == _lib.WAVE_PSV and wl.punch_after is None
     # steps per launch of the SH block step, 0 when another path runs
     block = ctx.tile_shape()[2] if kind == _lib.TILE_BLOCK and wl.punch_after is None else 0
-    # steps per launch of the marching P-SV step (it is one of the fused shapes)
-    march = ctx.tile_shape()[2] if fused and ctx.tile_shape()[3] == -1 else 0
-    names = kernel_names(ctx, wl)
+    # steps per launch of the marching step (one of the fused shapes, SH and
+    # P-SV), 0 on a context set to it that runs the two passes instead
+    shape = ctx.tile_shape()
+    whole = march_bytes(wl) if shape[3] == -1 else None
+    march = shape[2] if whole and abs(ctx.bytes_per_step() * shape[2] - whole) < 1.0 else 0
+    fused = kind == _lib.TILE_FUSED and wl.wave == _lib.WAVE_PSV and wl.punch_after is None and shape[3] != -1
+    names = kernel_names(ctx, wl, march > 0)
     s_ms, v_ms = ctx.time_passes(20) if passes else (None, None)
     ctx.close()
     return dict(elapsed=el, stress_ms=s_ms, vel_ms=v_ms, tile=tile, tune_ms=tune_ms, finite=finite, fused=fused,
@@ -136,11 +149,12 @@ def run_gpu(wl, steps, warmup, autotune=True, tile=None, passes=True, chains=Non
 STORE_TYPE = {0: "float", 1: "__half", 2: "__hip_bfloat16", 3: "double"}
 
 
-def kernel_names(ctx, wl):
+def kernel_names(ctx, wl, march=False):
     """Kernels of the (stress, velocity) passes as profilers print them, a
     tuple per pass: split tile shapes launch the interior tiles and the edge
     tiles of a P-SV pass as two instances of one kernel; the fused step and
-    the SH block step are one kernel for both."""
+    the SH block step are one kernel for both.  march: the context runs the
+    marching step, whose kernel is one of two widths, and its frame's passes."""
     from fd23_amd import _lib
 
     rz, spb, seg, blk = ctx.tile_shape()
@@ -150,18 +164,18 @@ def kernel_names(ctx, wl):
         if kind == _lib.TILE_BLOCK and wl.punch_after is None:
             n = ("fd23::k_sh_block<%s, %d, %d, %d>" % (t, seg, rz, blk // rz),)
             return (n, n)
-        if blk == -1 and wl.storage == 0 and wl.punch_after is None:  # the marching step and its frame's passes
+        if march:
             n = tuple("fd23::k_sh_march<%d>" % w for w in (256, 512)) + \
                 tuple("fd23::k_sh_%s<float, 4, 1, true>" % p for p in ("stress", "velocity"))
             return (n, n)
-        if kind != _lib.TILE_TILED:  # a window runs tile 0's tiled kernels
+        if kind != _lib.TILE_TILED and blk != -1:  # a window runs tile 0's tiled kernels
             rz, spb = ctx.tile_shape(0)[:2]
         return tuple(("fd23::k_sh_%s<%s, %d, %d, false>" % (p, t, rz, spb),) for p in ("stress", "velocity"))
     # a first-arrival window runs the whole-grid tiled kernels (tile 0's
     # shape in place of a fused one)
     window = wl.punch_after is not None
-    if kind == _lib.TILE_FUSED and not window:
-        if blk == -1:  # the marching step: its interior kernel and its frame's two passes
+    if kind == _lib.TILE_FUSED and not window and (march or blk != -1):
+        if march:
             n = tuple("fd23::k_psv_march<%s, %d>" % (t, w) for w in (256, 512)) + \
                 tuple("fd23::k_psv_%s<%s, 4, 1, 2, true>" % (p, t) for p in ("stress", "velocity"))
             return (n, n)
@@ -169,7 +183,7 @@ def kernel_names(ctx, wl):
         n = ("fd23::k_psv_fused_tile<%s, %d>" % (t, seg // 4),) if blk == 0 else \
             ("fd23::k_psv_fused<%s, %d, %d>" % (t, seg, blk),)
         return (n, n)
-    if kind == _lib.TILE_FUSED:
+    if kind == _lib.TILE_FUSED and blk != -1:
         rz, spb = ctx.tile_shape(0)[:2]
     regions = (1, 2) if ctx.tile_split() and not window else (0,)
     return tuple(tuple("fd23::k_psv_%s<%s, %d, %d, %d>" % (p, t, rz, spb, region) for region in regions)
@@ -569,7 +583,7 @@ def measure_line(wl, steps, warmup, autotune=True, tile=None, chains=None):
     if r["march"]:
         # time_passes reports the time per step; a launch (the interior kernel
         # and its frame) reads and writes the state once for `march` steps
-        name, nbytes, kms, kname = "march", fused_bytes(wl), r["stress_ms"] * r["march"], r["kernels"][0]
+        name, nbytes, kms, kname = "march", march_bytes(wl), r["stress_ms"] * r["march"], r["kernels"][0]
         step_bytes = nbytes / r["march"]
     elif r["fused"]:
         name, nbytes, kms, kname = "fused", fused_bytes(wl), r["stress_ms"], r["kernels"][0]
@@ -586,6 +600,7 @@ def measure_line(wl, steps, warmup, autotune=True, tile=None, chains=None):
         name, nbytes, kms, kname = "velocity", vb, r["vel_ms"], r["kernels"][1]
         step_bytes = sb + vb
     achieved = nbytes / (kms * 1e-3) / 1e9
+    whole = r["march"] or r["fused"] or r["block"]  # steps timed as a whole
     sname = {v: k for k, v in STORAGE.items()}[wl.storage]
     out = {
         "metric": "Gcell-updates/s",
@@ -611,8 +626,8 @@ def measure_line(wl, steps, warmup, autotune=True, tile=None, chains=None):
                      "unit": "GB/s", "frac": round(achieved / HBM_PEAK_GBS, 4),
                      "traffic": measured_traffic(workload_id(wl), kname), "kernel_name": list(kname),
                      "kernel_ms": round(kms, 5), "algorithmic_bytes": nbytes,
-                     "stress_ms": None if r["fused"] or r["block"] else round(r["stress_ms"], 5),
-                     "velocity_ms": None if r["fused"] or r["block"] else round(r["vel_ms"], 5)},
+                     "stress_ms": None if whole else round(r["stress_ms"], 5),
+                     "velocity_ms": None if whole else round(r["vel_ms"], 5)},
         "finite": r["finite"],
     }
     if wl.punch_after is not None:

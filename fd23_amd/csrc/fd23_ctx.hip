@@ -516,6 +516,18 @@ extern "C" int fd23_ctx_destroy(fd23_ctx *c) {
 // a tenth of its 250 us on the link.
 static const size_t kStageBytes = (size_t)4 << 20;
 
+// A launch with a status of its own: hipGetLastError also returns what a call
+// of another part of the program has left, and takes it from it.
+template <class T> struct Same {
+    using type = T;
+};
+template <class... P>
+static hipError_t launch(void (*kernel)(P...), dim3 grid, dim3 block, hipStream_t stream,
+                         typename Same<P>::type... args) {
+    void *a[] = {(void *)&args...};
+    return hipLaunchKernel((const void *)kernel, grid, block, a, 0, stream);
+}
+
 template <class S> static int rows_xfer_t(fd23_ctx *c, void *dev, long pitch, long w, long h, void *host, float scale,
                                           bool to_host) {
     using C = typename Store<S>::C;
@@ -535,14 +547,11 @@ template <class S> static int rows_xfer_t(fd23_ctx *c, void *dev, long pitch, lo
         S *d = (S *)dev + r * pitch;
         char *p = (char *)host + (size_t)r * row;
         if (to_host) {
-            hipLaunchKernelGGL((k_pack_rows<S>), grid, block, 0, c->stream, (C *)c->stage, d, pitch, w, n, scale);
-            HIPCHK(hipGetLastError());
+            HIPCHK(launch(k_pack_rows<S>, grid, block, c->stream, (C *)c->stage, d, pitch, w, n, scale));
             HIPCHK(hipMemcpyAsync(p, c->stage, (size_t)n * row, hipMemcpyDeviceToHost, c->stream));
         } else {
             HIPCHK(hipMemcpyAsync(c->stage, p, (size_t)n * row, hipMemcpyHostToDevice, c->stream));
-            hipLaunchKernelGGL((k_unpack_rows<S>), grid, block, 0, c->stream, d, (const C *)c->stage, pitch, w, n,
-                               scale);
-            HIPCHK(hipGetLastError());
+            HIPCHK(launch(k_unpack_rows<S>, grid, block, c->stream, d, (const C *)c->stage, pitch, w, n, scale));
         }
     }
     HIPCHK(hipStreamSynchronize(c->stream));
@@ -867,8 +876,7 @@ extern "C" int fd23_reset_shot(fd23_ctx *c, int shot) {
         region((char *)c->seis + shot * mine, (long)frame, mine, c->d.max_frames);
     }
     if (n == 0) return FD23_OK;
-    hipLaunchKernelGGL(k_zero_regions, dim3(std::min(most, 256u), n), dim3(256), 0, c->stream, z);
-    HIPCHK(hipGetLastError());
+    HIPCHK(launch(k_zero_regions, dim3(std::min(most, 256u), n), dim3(256), c->stream, z));
     return FD23_OK;
 }
 

@@ -1,0 +1,32 @@
+"""Host transfers and resets beside other parts of a program (no GPU: the
+runtime is replaced)."""
+import pytest
+
+from hosthip import run
+
+CALLS = """
+c = context(%s, 130, 70, 2, %s)
+c.run(0, 6, 1)
+def calls(c):
+    for s in range(2):
+        state = c.get_state(s)
+        c.set_state(state, s)
+        for f in (("U", "Txz") if c.wave == PSV else ("V", "Tz")):
+            c.set_field(f, c.field(f, s), s)
+        for k in range(c.ncomp):
+            c.seismograms(s, k, 6)
+        c.reset_shot(s)
+    c.set_material([c.material(i) for i in range(5 if c.wave == PSV else 3)])
+"""
+KINDS = [("PSV", "F32"), ("PSV", "F16"), ("PSV", "F64"), ("SH", "F32"), ("SH", "BF16")]
+
+
+@pytest.mark.parametrize("kind", KINDS)
+def test_errors_of_others_stay_theirs(kind):
+    """An error that another call has left (an allocation that failed) is neither
+    reported by a transfer or a reset nor taken away."""
+    run(CALLS % kind + """
+hh.hh_error = 2
+calls(c)
+assert hh.hh_error == 2
+""")

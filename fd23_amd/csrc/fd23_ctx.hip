@@ -272,8 +272,9 @@ struct fd23_ctx {
     MarchWork march_lists{}; // the geometry the marching step's lists were built for
     const FusedEvents *trial = nullptr; // while tuning: the marching kernel's events
 
-    // packed device rows on their way to or from the host (pitched copies)
-    void *stage = nullptr;
+    // packed device rows on their way to or from the host (pitched copies);
+    // stage_min is part of the arena, for when there is no room for the other
+    void *stage = nullptr, *stage_min = nullptr;
     size_t stage_cap = 0;
 
     // the allocations that hold the arrays above, and the second buffer set
@@ -361,6 +362,8 @@ extern "C" size_t fd23_desc_device_bytes(const fd23_desc *d) {
 }
 
 extern "C" size_t fd23_ctx_device_bytes(const fd23_ctx *c) { return c ? fd23_desc_device_bytes(&c->d) : 0; }
+
+static const size_t kMinStage = (size_t)64 << 10;
 
 // parts of one device allocation, each from a multiple of 4 KiB on
 struct Parts {
@@ -453,6 +456,7 @@ extern "C" int fd23_ctx_create(const fd23_desc *desc, fd23_ctx **out) {
         off += 3L * c->prof_n[p];
     }
     parts.add(c->prof, (size_t)off * c->csize);
+    parts.add(c->stage_min, kMinStage);
     parts.add(c->d_fieldtab, sizeof(void *) * 5);
     parts.add(c->d_comptab, sizeof(void *) * 2);
     parts.add(c->d_compfield, sizeof(int) * 2);
@@ -531,29 +535,37 @@ static hipError_t launch(void (*kernel)(P...), dim3 grid, dim3 block, hipStream_
 template <class S> static int rows_xfer_t(fd23_ctx *c, void *dev, long pitch, long w, long h, void *host, float scale,
                                           bool to_host) {
     using C = typename Store<S>::C;
-    const size_t row = (size_t)w * sizeof(C);
-    const long per = std::max<long>(1, (long)std::min<size_t>(kStageBytes / row, (size_t)h)); // rows of one copy
-    if ((size_t)per * row > c->stage_cap) {
+    const size_t all = (size_t)w * h * sizeof(C), want = std::min(kStageBytes, all);
+    if (want > c->stage_cap) {
         if (c->stage) HIPCHK(hipFree(c->stage));
-        c->stage = nullptr;
         c->stage_cap = 0;
-        HIPCHK(hipMalloc(&c->stage, (size_t)per * row));
-        c->stage_cap = (size_t)per * row;
-    }
-    const dim3 block(256);
-    for (long r = 0; r < h; r += per) {
-        const long n = std::min(per, h - r);
-        const dim3 grid((unsigned)std::min<long>((w + 255) / 256, 1024), (unsigned)std::min<long>(n, 4096));
-        S *d = (S *)dev + r * pitch;
-        char *p = (char *)host + (size_t)r * row;
-        if (to_host) {
-            HIPCHK(launch(k_pack_rows<S>, grid, block, c->stream, (C *)c->stage, d, pitch, w, n, scale));
-            HIPCHK(hipMemcpyAsync(p, c->stage, (size_t)n * row, hipMemcpyDeviceToHost, c->stream));
-        } else {
-            HIPCHK(hipMemcpyAsync(c->stage, p, (size_t)n * row, hipMemcpyHostToDevice, c->stream));
-            HIPCHK(launch(k_unpack_rows<S>, grid, block, c->stream, d, (const C *)c->stage, pitch, w, n, scale));
+        if (hipMalloc(&c->stage, want) == hipSuccess) {
+            c->stage_cap = want;
+        } else { // the context's own piece carries it, in smaller copies
+            c->stage = nullptr;
+            (void)hipGetLastError();
         }
     }
+    C *stage = c->stage ? (C *)c->stage : (C *)c->stage_min;
+    const long cap = (long)((c->stage ? c->stage_cap : kMinStage) / sizeof(C));
+    // whole rows, or parts of one
+    const long cols = std::min(w, cap), per = cols < w ? 1 : std::min(cap / w, h);
+    const dim3 block(256);
+    for (long r = 0; r < h; r += per)
+        for (long x = 0; x < w; x += cols) {
+            const long n = std::min(per, h - r), m = std::min(cols, w - x);
+            const size_t bytes = (size_t)n * m * sizeof(C);
+            const dim3 grid((unsigned)std::min<long>((m + 255) / 256, 1024), (unsigned)std::min<long>(n, 4096));
+            S *d = (S *)dev + r * pitch + x;
+            C *p = (C *)host + r * w + x;
+            if (to_host) {
+                HIPCHK(launch(k_pack_rows<S>, grid, block, c->stream, stage, d, pitch, m, n, scale));
+                HIPCHK(hipMemcpyAsync(p, stage, bytes, hipMemcpyDeviceToHost, c->stream));
+            } else {
+                HIPCHK(hipMemcpyAsync(stage, p, bytes, hipMemcpyHostToDevice, c->stream));
+                HIPCHK(launch(k_unpack_rows<S>, grid, block, c->stream, d, stage, pitch, m, n, scale));
+            }
+        }
     HIPCHK(hipStreamSynchronize(c->stream));
     return FD23_OK;
 }

@@ -5,7 +5,7 @@ import pytest
 from hosthip import run
 
 CALLS = """
-c = context(%s, 130, 70, 2, %s)
+c = context(%s, 130, 70, 2, %s, nt=300)
 c.run(0, 6, 1)
 def calls(c):
     for s in range(2):
@@ -14,7 +14,7 @@ def calls(c):
         for f in (("U", "Txz") if c.wave == PSV else ("V", "Tz")):
             c.set_field(f, c.field(f, s), s)
         for k in range(c.ncomp):
-            c.seismograms(s, k, 6)
+            c.seismograms(s, k, 300)
         c.reset_shot(s)
     c.set_material([c.material(i) for i in range(5 if c.wave == PSV else 3)])
 """
@@ -29,4 +29,13 @@ def test_errors_of_others_stay_theirs(kind):
 hh.hh_error = 2
 calls(c)
 assert hh.hh_error == 2
+""")
+
+
+@pytest.mark.parametrize("kind", KINDS)
+def test_transfers_need_no_free_memory(kind):
+    """A context whose run has filled the device still gives its results."""
+    run(CALLS % kind + """
+hh.hh_room = 0
+calls(c)
 """)

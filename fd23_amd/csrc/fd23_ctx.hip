@@ -2197,7 +2197,7 @@ static int run_prologue(fd23_ctx *c, int it0, int nt, int itrecord) {
 extern "C" int fd23_run(fd23_ctx *c, int it0, int nt, int itrecord) {
     int r = run_prologue(c, it0, nt, itrecord);
     if (r) return r;
-    hipLaunchKernelGGL(k_set_clock, dim3(1), dim3(64), 0, c->stream, c->clock, it0);
+    hipLaunchKernelGGL(k_set_clock, dim3(1), dim3(64), 0, c->stream, c->clock, it0, c->scl);
     const int full = nt / kGraphSteps, rest = nt % kGraphSteps;
     for (int i = 0; i < full; i++)
         if ((r = launch_chunk(c, itrecord, kGraphSteps))) return r;

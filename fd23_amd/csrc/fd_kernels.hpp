@@ -1612,9 +1612,11 @@ static __global__ void k_set_ptrs(void **tab, PtrTable5 v, int n) {
     if (threadIdx.x < n) tab[threadIdx.x] = v.p[threadIdx.x];
 }
 
-// set the step clock in stream order (no host round trip)
-static __global__ void k_set_clock(int *clock, int it0) {
+// set the step clock in stream order (no host round trip); a run begins with
+// every array in its current scale, whatever half of a step came before it
+static __global__ void k_set_clock(int *clock, int it0, float *scl) {
     if (threadIdx.x == 0) clock[0] = it0;
+    if (threadIdx.x < kNextScale) scl[kPrevScale + threadIdx.x] = scl[threadIdx.x];
 }
 
 } // namespace fd23

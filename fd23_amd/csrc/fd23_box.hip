@@ -752,6 +752,7 @@ extern "C" int fd23_box_get_residual(fd23_ctx *c, int shot, void *out) {
 void fd23_box_free(fd23_ctx *c) {
     Box *b = get(c);
     if (!b) return;
+    fd23_ctx_invalidate_graphs(c); // they name its arrays
     if (b->resid) (void)hipFree(b->resid);
     if (b->gtab) (void)hipFree(b->gtab);
     if (b->frames) (void)hipFree(b->frames);

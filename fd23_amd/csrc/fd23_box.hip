@@ -405,7 +405,13 @@ struct Box {
     int nframes = 0;
     double *sdrive = nullptr; // [5][bw*bw]
     int nforced = 0;          // box cells whose material was forced
+    size_t bytes = 0;         // of resid, plane-wave drive
 };
+void drop(Box *b) {
+    for (void *p : {b->resid, (void *)b->gtab, (void *)b->frames, (void *)b->sdrive})
+        if (p) (void)hipFree(p);
+    delete b;
+}
 
 Box *get(fd23_ctx *c) { return (Box *)fd23_ctx_box(c); }
 
@@ -527,8 +533,16 @@ extern "C" int fd23_box_configure(fd23_ctx *c, int shot, int x0, int z0, int bx,
         fd23_set_error_(msg);
         return FD23_EINVAL;
     }
-    fd23_box_free(c);
+    // the arrays of a box of the same size are taken over: freed and allocated
+    // again they cost up to 3 ms of a first call (640 x 401 FP64, 60 steps 5.4
+    // ms instead of 2.3)
+    const size_t bytes = (size_t)d.nshots * 5 * bx * bz * (d.storage == FD23_STORE_F64 ? 8 : 4);
     Box *b = new Box();
+    if (Box *old = get(c); old && old->bytes == bytes) {
+        std::swap(b->resid, old->resid);
+        std::swap(b->gtab, old->gtab);
+    }
+    fd23_box_free(c);
     BoxPar &p = b->p;
     p.x0 = x0;
     p.z0 = z0;
@@ -552,7 +566,7 @@ extern "C" int fd23_box_configure(fd23_ctx *c, int shot, int x0, int z0, int bx,
         p.sxz = -(2.0 * mu * p.nx_ * p.nz_) / vp;
     } else {
         if (!(vs > 0)) {
-            delete b;
+            drop(b);
             fd23_set_error_("SV incidence needs vs > 0");
             return FD23_EINVAL;
         }
@@ -578,12 +592,11 @@ extern "C" int fd23_box_configure(fd23_ctx *c, int shot, int x0, int z0, int bx,
     b->lam = lam * fac;
     b->mu = mu * fac;
     b->b = fac / rho;
-    const size_t cs = b->f64 ? 8 : 4;
-    const size_t bytes = (size_t)d.nshots * 5 * bx * bz * cs;
-    if (hipMalloc(&b->resid, bytes) != hipSuccess || hipMalloc((void **)&b->gtab, 5 * sizeof(void *)) != hipSuccess) {
+    b->bytes = bytes;
+    if (!b->resid &&
+        (hipMalloc(&b->resid, bytes) != hipSuccess || hipMalloc((void **)&b->gtab, 5 * sizeof(void *)) != hipSuccess)) {
         fd23_set_error_("box allocation failed");
-        if (b->resid) (void)hipFree(b->resid);
-        delete b;
+        drop(b);
         return FD23_ENOMEM;
     }
     hipStream_t st = fd23_ctx_stream(c);
@@ -605,9 +618,7 @@ extern "C" int fd23_box_configure(fd23_ctx *c, int shot, int x0, int z0, int bx,
                            (float *)fd23_ctx_material(c, 4), (float)b->b, (float)b->mu, (float)b->lam);
     if (hipStreamSynchronize(st) != hipSuccess) {
         fd23_set_error_("box set-up failed");
-        (void)hipFree(b->resid);
-        (void)hipFree(b->gtab);
-        delete b;
+        drop(b);
         return FD23_EHIP;
     }
     fd23_ctx_box(c) = b;
@@ -677,12 +688,8 @@ extern "C" int fd23_box_configure_frames(fd23_ctx *c, int xs, int zs, int bw, co
         hipMalloc((void **)&b->sdrive, sbytes) != hipSuccess ||
         hipMalloc((void **)&d_nforced, sizeof(int)) != hipSuccess) {
         fd23_set_error_("box allocation failed");
-        if (b->resid) (void)hipFree(b->resid);
-        if (b->gtab) (void)hipFree(b->gtab);
-        if (b->frames) (void)hipFree(b->frames);
-        if (b->sdrive) (void)hipFree(b->sdrive);
         if (d_nforced) (void)hipFree(d_nforced);
-        delete b;
+        drop(b);
         return FD23_ENOMEM;
     }
     hipStream_t st = fd23_ctx_stream(c);
@@ -712,11 +719,7 @@ extern "C" int fd23_box_configure_frames(fd23_ctx *c, int xs, int zs, int bw, co
     if (e != hipSuccess) {
         snprintf(msg, sizeof msg, "box set-up failed: %s", hipGetErrorString(e));
         fd23_set_error_(msg);
-        (void)hipFree(b->resid);
-        (void)hipFree(b->gtab);
-        (void)hipFree(b->frames);
-        (void)hipFree(b->sdrive);
-        delete b;
+        drop(b);
         return FD23_EHIP;
     }
     fd23_ctx_box(c) = b;
@@ -753,10 +756,6 @@ void fd23_box_free(fd23_ctx *c) {
     Box *b = get(c);
     if (!b) return;
     fd23_ctx_invalidate_graphs(c); // they name its arrays
-    if (b->resid) (void)hipFree(b->resid);
-    if (b->gtab) (void)hipFree(b->gtab);
-    if (b->frames) (void)hipFree(b->frames);
-    if (b->sdrive) (void)hipFree(b->sdrive);
-    delete b;
+    drop(b);
     fd23_ctx_box(c) = nullptr;
 }

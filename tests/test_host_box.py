@@ -20,3 +20,18 @@ before = hh.hh_graphs
 c.run(0, 6, 1)
 assert hh.hh_graphs == before + 1
 """)
+
+
+def test_same_box_again_allocates_nothing():
+    """The next plane wave on a box of the same size takes over its arrays."""
+    run(BOX + """
+before = hh.hh_mallocs, hh.hh_room
+for incident in (1, 0):
+    box(c, incident=incident, x0=30)
+    c.run(0, 6, 1)
+    c.box_residual()
+assert (hh.hh_mallocs, hh.hh_room) == before
+box(c, 50)
+assert hh.hh_mallocs == before[0] + 2 and hh.hh_room < before[1]
+c.close()
+""")

@@ -186,7 +186,7 @@ def kernel_names(ctx, wl, march=False):
     if kind == _lib.TILE_FUSED and blk != -1:
         rz, spb = ctx.tile_shape(0)[:2]
     regions = (1, 2) if ctx.tile_split() and not window else (0,)
-    return tuple(tuple("fd23::k_psv_%s<%s, %d, %d, %d>" % (p, t, rz, spb, region) for region in regions)
+    return tuple(tuple("fd23::k_psv_%s<%s, %d, %d, %d, false>" % (p, t, rz, spb, region) for region in regions)
                  for p in ("stress", "velocity"))
 
 
@@ -194,20 +194,20 @@ def measured_traffic(workload, kernels):
     """HBM bytes per pass (summed over its kernels) on a workload, from the
     rocprofv3 FETCH_SIZE / WRITE_SIZE summaries kept beside this file
     (scaled by the copy calibration stated there); None when a kernel of
-    the pass was not profiled."""
+    the pass was not profiled.  A marching launch: the width that runs, and
+    the frame's two passes twice."""
     path = os.path.join(os.path.dirname(os.path.abspath(__file__)), "profiles", "traffic.json")
     try:
         with open(path) as f:
             table = json.load(f)
     except (OSError, ValueError):
         return None
-    total = 0
-    for k in kernels:
-        e = table.get("%s|%s" % (workload, k))
-        if e is None:
-            return None
-        total += int(e["hbm_bytes"])
-    return total
+    entries = {k: table.get("%s|%s" % (workload, k)) for k in kernels}
+    wide = [k for k in kernels if "_march<" in k]
+    counted = [k for k in wide if entries[k]][:1] + 2 * [k for k in kernels if k not in wide] if wide else kernels
+    if len(counted) < (5 if wide else 1) or any(entries[k] is None for k in counted):
+        return None
+    return sum(int(entries[k]["hbm_bytes"]) for k in counted)
 
 
 def cpu_baseline(wl, budget_s=12.0, budget_1t=4.0):

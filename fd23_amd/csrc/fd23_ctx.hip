@@ -842,7 +842,7 @@ extern "C" int fd23_set_shot_slot(fd23_ctx *c, int shot, int active, int t0) {
         return fail(FD23_EINVAL, "the box and the first-arrival window run every shot from step 0");
     if (c->src[shot].t0 != t0) {
         c->src[shot].t0 = t0;
-        c->src_dirty = true; // rebuilds the lists, and with them the graphs
+        c->src_dirty = true; // rebuilds the lists
     }
     if (shot < 64) {
         const unsigned long long bit = 1ull << shot, was = c->idle;
@@ -922,8 +922,10 @@ static bool march_rect(const fd23_ctx *c, MarchWork &w) {
     if (w.x1 <= w.x0 || w.z1 <= w.z0) return false;
     // Sources and receivers near the surface are left to the frame when that
     // costs the rectangle at most an eighth of its rows: items with events run
-    // checked rows, and a launch lasts as long as its slowest item (8 shots of
-    // 4096 x 2048 with the source at row 8: 972 against 712 us).
+    // checked rows, and a launch lasts as long as its slowest item (source at
+    // row 8, receivers at row 4, us a step with the rectangle above them and
+    // below: 8 shots of 4096 x 2048 FP16 440 / 378, FP32 463 / 462, SH 4 shots
+    // 135 / 131, 2 shots of 3000 x 1800 110 / 106, 64 of 1024 x 512 318 / 322).
     int deep = w.z0 - 1;
     for (const HostSrc &h : c->src)
         if (h.kind >= 0 && !h.stf.empty()) deep = std::max(deep, h.zs + 1 + kMarchReach);

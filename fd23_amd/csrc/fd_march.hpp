@@ -25,15 +25,19 @@
 // (121 against 163 Gcell/s on 4096 x 2048 x 8 in FP32).  Lanes that own
 // nothing, and rows outside the segment, store beyond the buffer's range,
 // which drops them.  Items with a source tap or a recorded receiver run the
-// same rows with the checks.
+// same rows with the checks (a source, or a line of receivers, at mid-depth:
+// 0 to 9% more a step in FP32, 11 to 23% in 16 bits; a receiver in every row of
+// one column 2 to 20% and 24 to 43%).
 //
-// Measured, 8 shots of 4096 x 2048, FP32: 701 us for the two steps of the
-// 4000 x 1984 interior (181 Gcell/s, 4.4 TB/s through the L2; without any
-// load or store 388 us) where the two passes take 1680; FP16 617 us.  One
-// column per thread and three workgroups per CU: 781 us.  Non-temporal field
-// loads and stores keep the material in the L2: 757 -> 701 us in FP32; FP16,
-// half the bytes, is not faster with them (617 / 629).  The register files
-// are full: 256 VGPRs, two wavefronts per SIMD.
+// Measured, 8 shots of 4096 x 2048, FP32: 701-725 us for the two steps of the
+// 4000 x 1984 interior (176-181 Gcell/s; 3.08 GB from and to the HBM, 4.2 TB/s;
+// 206 M wavefront instructions of the vector units, 46% of their issue slots)
+// where the two passes take 1680; FP16 591-617 us (1.91 GB, 3.2 TB/s, 254 M,
+// 68%).  One column per thread and three workgroups per CU: 781 us.
+// Non-temporal field loads and stores keep the material in the L2: 757 -> 701
+// us in FP32; FP16, half the bytes, is not faster with them (617 / 629).  The
+// register files are full: 256 VGPRs, two wavefronts per SIMD; nothing spills
+// to memory but, in 16 bits, the checked body that gathers maxima (40).
 //
 // The arithmetic of a cell is that of the two-pass kernels' interior path
 // (psv_stress_interior, psv_velocity_interior), and values that the passes

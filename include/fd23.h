@@ -155,8 +155,8 @@ int fd23_set_receivers(fd23_ctx *ctx, int shot, int comp, const int *rx,
  * records its frame f at step t0 + f*itrecord, so its seismograms read
  * back from frame 0 as if it had run alone from step 0.  An idle shot
  * (active 0; shots 0..63) is not stepped by fd23_run.  Defaults: active,
- * t0 = 0.  A change takes effect on the next fd23_run (its graphs are
- * captured again).  Contexts with a box or a first-arrival window run
+ * t0 = 0.  A change takes effect on the next fd23_run (after one of active
+ * its graphs are captured again).  Contexts with a box or a first-arrival window run
  * every shot from step 0: fd23_run refuses other slots there.           */
 int fd23_set_shot_slot(fd23_ctx *ctx, int shot, int active, int t0);
 /* Zero one shot's fields, C-PML memory (both buffer sets) and seismogram
@@ -267,8 +267,12 @@ int fd23_box_forced_cells(fd23_ctx *ctx);
 int fd23_box_get_residual(fd23_ctx *ctx, int shot, void *out);
 
 /* ---- tuning and introspection ---------------------------------------- */
-/* tile shape index (0 = default); fd23_autotune times the candidates on
- * this context's own arrays and keeps the fastest.  State is preserved. */
+/* tile shape index.  A context starts on a shape picked from its size and
+ * storage; where that shape needs a second buffer set and the device has no
+ * room for it, the first run goes on with a two-pass shape in place (a shape
+ * set here, or tuned, is refused with FD23_ENOMEM then).  fd23_autotune times
+ * the candidates on this context's own arrays, the marching step with its
+ * sources and receivers, and keeps the fastest.  State is preserved.       */
 int fd23_set_tile(fd23_ctx *ctx, int tile);
 int fd23_get_tile(const fd23_ctx *ctx);
 int fd23_num_tiles(void);
@@ -289,8 +293,9 @@ int fd23_num_tiles(void);
  * marching step's of SH ones too) without a box, the block step to fd23_run of SH contexts with FP32/FP64
  * storage, both without a first-arrival window; the staged entry points,
  * the box and the window run the tiled kernels (tile 0's shape, or for the
- * marching step its frame's; so do contexts with idle slots or with
- * other storage set to the marching step, and grids with no interior).  No
+ * marching step its frame's; so do contexts with idle slots, for as long as
+ * any slot is idle, or with other storage set to the marching step, and grids
+ * with no interior).  No
  * reference counterpart: the reference launches two kernels per step
  * (SH/main.cpp:93-141).                                                 */
 enum { FD23_TILE_TILED = 0, FD23_TILE_FUSED = 1, FD23_TILE_BLOCK = 2 };

@@ -13,7 +13,7 @@
 //
 // Measured, us a step with the frame's passes (two passes on the whole grid):
 // 6 shots of 2048 x 1024 68 (82), 4 shots of 4096 x 2048 133 (265).  The
-// registers (197) leave two wavefronts per SIMD; three, with segments a third
+// registers (204) leave two wavefronts per SIMD; three, with segments a third
 // shorter, take 81 and 149: the 24 rows that a segment recomputes weigh more.
 // Of the 68 us the frame's four launches take 25.
 #pragma once

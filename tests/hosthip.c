@@ -9,7 +9,7 @@ typedef struct {
 } dim3_;
 
 long hh_room = 1L << 40;   /* bytes hipMalloc may still give */
-long hh_graphs, hh_held, hh_launches, hh_mallocs, hh_copied;
+long hh_graphs, hh_held, hh_launches, hh_mallocs, hh_copied, hh_async;
 int hh_error;              /* the error hipGetLastError returns next */
 
 static int failed(int e) {
@@ -44,10 +44,17 @@ int hipMemcpy(void *d, const void *s, size_t n, int kind) {
     hh_copied += (long)n;
     return 0;
 }
-int hipMemcpyAsync(void *d, const void *s, size_t n, int kind, void *st) { return (void)st, hipMemcpy(d, s, n, kind); }
-int hipMemcpy2DAsync(void *d, size_t dp, const void *s, size_t sp, size_t w, size_t h, int kind, void *st) {
-    for (size_t i = 0; i < h; i++) hipMemcpyAsync((char *)d + i * dp, (const char *)s + i * sp, w, kind, st);
+int hipMemcpyAsync(void *d, const void *s, size_t n, int kind, void *st) {
+    (void)st;
+    hh_async++;
+    return hipMemcpy(d, s, n, kind);
+}
+int hipMemcpy2D(void *d, size_t dp, const void *s, size_t sp, size_t w, size_t h, int kind) {
+    for (size_t i = 0; i < h; i++) hipMemcpy((char *)d + i * dp, (const char *)s + i * sp, w, kind);
     return 0;
+}
+int hipMemcpy2DAsync(void *d, size_t dp, const void *s, size_t sp, size_t w, size_t h, int kind, void *st) {
+    return (void)st, hipMemcpy2D(d, dp, s, sp, w, h, kind);
 }
 int hipMemset(void *d, int v, size_t n) { return memset(d, v, n), 0; }
 int hipMemsetAsync(void *d, int v, size_t n, void *st) { return (void)st, hipMemset(d, v, n); }

@@ -39,3 +39,18 @@ def test_transfers_need_no_free_memory(kind):
 hh.hh_room = 0
 calls(c)
 """)
+
+
+@pytest.mark.parametrize("kind", KINDS)
+def test_one_or_two_frames_come_in_one_call(kind):
+    """Neither packed nor queued: that takes about twice as long as the runtime's
+    own copy of one or two rows."""
+    run(CALLS % kind + """
+for n in (1, 2):
+    before = hh.hh_launches, hh.hh_async
+    c.seismograms(1, 0, n)
+    assert (hh.hh_launches, hh.hh_async) == before, n
+before = hh.hh_launches
+c.seismograms(1, 0, 3)
+assert hh.hh_launches == before + 1
+""")
